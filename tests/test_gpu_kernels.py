@@ -444,6 +444,44 @@ def test_aggregate_finalize_non_finite_matches_oracle(hip_device, layer_mode) ->
     torch.testing.assert_close(got[finite], want[finite], rtol=1e-3, atol=1e-3)
 
 
+@pytest.mark.parametrize("layer_mode", ["mean", "max"])
+@pytest.mark.parametrize("layers,heads", [(1, 17), (3, 7), (6, 40), (2, 1), (8, 64), (64, 33)])
+def test_aggregate_few_tokens_bit_identical(hip_device, layers, heads, layer_mode) -> None:
+    # Batches of few tokens share 32 tokens between a workgroup's waves; a
+    # max_seq_len bound past that form's limit takes one wave per 32 tokens.
+    # Both combine the same values in the same layer order: the same bits, and
+    # the same per-layer maxima from kvc_layer_head_max.
+    from kvcompress_mi355x import _native
+    from kvcompress_mi355x.methods.triattention import _device as dev
+
+    g = torch.Generator().manual_seed(layers * 100 + heads)
+    lens = [31, 1, 33, 640, 32]
+    total = sum(lens)
+    offs = [sum(lens[:i]) for i in range(len(lens))]
+    raw = torch.randn(layers, heads, total + 3, generator=g) * 2
+    raw[0, heads - 1, 3] = float("nan")
+    raw[layers - 1, 0, 40] = float("inf")
+    d = hip_device
+    raw_d = raw.to(d)
+    mean = torch.randn(layers, len(lens), heads, generator=g).to(d)
+    var = (torch.rand(layers, len(lens), heads, generator=g) + 0.1).to(d)
+    seq_lens = torch.tensor(lens, dtype=torch.int32, device=d)
+    tok_off = torch.tensor(offs, dtype=torch.int64, device=d)
+    mode = _native.LAYER_MEAN if layer_mode == "mean" else _native.LAYER_MAX
+    outs = []
+    for bound in (max(lens), 1 << 17):
+        agg = torch.full((total,), 123.0, device=d)
+        per_layer = torch.full((layers, total), 123.0, device=d)
+        head = (dev.stream_handle(d), layers, heads, len(lens), bound, dev.ptr(seq_lens), dev.ptr(tok_off), dev.ptr(raw_d),
+                heads * (total + 3), 1, total + 3, dev.ptr(mean), dev.ptr(var), len(lens) * heads, heads)
+        _native.call("kvc_aggregate", *head, mode, _native.AGG_FINALIZE, dev.ptr(agg))
+        _native.call("kvc_layer_head_max", *head, 0, dev.ptr(per_layer), total)
+        outs.append((agg.cpu(), per_layer.cpu()))
+    assert outs[0][0].view(torch.int32).equal(outs[1][0].view(torch.int32))
+    assert torch.equal(torch.nan_to_num(outs[0][1], nan=5e5), torch.nan_to_num(outs[1][1], nan=5e5))
+    assert bool((outs[0][0] != 123.0).all()) and bool((outs[0][1] != 123.0).all())
+
+
 # ----------------------------------------------------------------- select --
 
 

@@ -471,10 +471,10 @@ __device__ __forceinline__ float finalize(float total, const AggArgs& a) {
   return finalize_total(total, a.flags, a.layer_mode, a.n_layers);
 }
 
-__device__ void load_layer_stats(const AggArgs& a, int b, float* s_mean, float* s_scale) {
+__device__ void load_layer_stats(const AggArgs& a, int b, float* s_mean, float* s_scale, int threads = kAggThreads) {
   const int n_stats = a.n_layers * a.n_heads;
   const bool rsqrt_form = (a.flags & KVC_AGG_RSQRT) != 0;
-  for (int i = threadIdx.x; i < n_stats; i += kAggThreads) {
+  for (int i = threadIdx.x; i < n_stats; i += threads) {
     const int l = i / a.n_heads, h = i - l * a.n_heads;
     const int64_t si = l * a.stats_layer_stride + b * a.stats_seq_stride + h;
     const float v = fmaxf(a.var[si], 1e-6f);
@@ -584,6 +584,75 @@ __global__ __launch_bounds__(kAggThreads) void aggregate_tokens_kernel(AggArgs a
     total = combine_layers(total, best, l, a, tok);
   }
   if (valid && part == 0 && !a.layer_out_stride) a.agg[tok] = finalize(total, a);
+}
+
+// The same for few tokens, where 32 tokens a wave leave most of the chip idle
+// and a wave's layers x heads loads are a serial chain of load groups (latency
+// bound: 22 us for one 4600-token sequence x 6 layers x 40 heads, 4.4 MB from
+// the L2): the eight waves of a workgroup share 32 tokens, wave w taking
+// (layer, head slice) items w, w + 8, ... of at most kAggSliceHeads heads (one
+// group of loads), and the items' maxima meet in LDS, where the layers are
+// combined in layer order as above, so the aggregates are bit-identical.
+// Microseconds per launch at 6 layers x 40 heads, this form (4 / 8 / 16 waves)
+// against the one above: 1 x 4600 tokens 10.4 / 7.7 / 7.2 against 22.1,
+// 2 x 16384 14.5 / 12.6 / 13.9 against 22.9, 4 x 16384 22.1 / 21.1 / 25.9
+// against 28.2, 8 x 16384 35.7 / 36.8 / 48.2 against 33.0 (per-workgroup
+// statistics loads outweigh the latency once the chip is full).  So eight waves
+// for at most kAggSplitMaxGroups groups of 32 tokens (4 x 16384).
+constexpr int kAggSplitWaves = 8;
+constexpr int kAggSliceHeads = kAggTokLanes * kAggHeadUnroll;
+constexpr int kAggMaxItems = 128;  // 16 KB of LDS
+constexpr int64_t kAggSplitMaxGroups = 2048;
+
+__global__ __launch_bounds__(64 * kAggSplitWaves) void aggregate_split_kernel(AggArgs a, int slices) {
+  extern __shared__ float dyn[];
+  float* s_mean = dyn;
+  float* s_scale = dyn + a.n_layers * a.n_heads;
+  float* s_item = dyn + 2 * a.n_layers * a.n_heads;  // [layers * slices][32]
+  const int b = blockIdx.y;
+  const int n = a.seq_lens[b];
+  if (static_cast<int64_t>(blockIdx.x) * 32 >= n) return;
+  load_layer_stats(a, b, s_mean, s_scale, 64 * kAggSplitWaves);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int part = lane >> 5;
+  const int t = blockIdx.x * 32 + (lane & 31);
+  const bool valid = t < n;
+  const bool rsqrt_form = (a.flags & KVC_AGG_RSQRT) != 0;
+  const int64_t tok = a.token_offsets[b] + (valid ? t : 0);
+  const int per = (a.n_heads + slices - 1) / slices;
+  for (int it = threadIdx.x >> 6; it < a.n_layers * slices; it += kAggSplitWaves) {
+    const int l = it / slices;
+    const int h0 = (it - l * slices) * per + part, last = min((it - l * slices + 1) * per, a.n_heads) - 1;
+    const float* col = a.raw + l * a.raw_layer_stride + tok;
+    const float* lm = s_mean + l * a.n_heads;
+    const float* ls = s_scale + l * a.n_heads;
+    // One group of loads: heads past the slice repeat its last one.
+    float v[kAggHeadUnroll];
+#pragma unroll
+    for (int u = 0; u < kAggHeadUnroll; ++u) v[u] = col[min(h0 + kAggTokLanes * u, last) * a.raw_head_stride];
+    float best = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < kAggHeadUnroll; ++u) {
+      const int h = min(h0 + kAggTokLanes * u, last);
+      best = max_nan(best, normalise(v[u], lm[h], ls[h], rsqrt_form));
+    }
+    best = max_nan(best, __shfl_xor(best, 32));
+    if (part == 0) s_item[it * 32 + lane] = best;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 32 || !valid) return;
+  float total = 0.0f;
+  for (int l = 0; l < a.n_layers; ++l) {
+    float best = s_item[l * slices * 32 + lane];
+    for (int s = 1; s < slices; ++s) best = max_nan(best, s_item[(l * slices + s) * 32 + lane]);
+    if (a.layer_out_stride) {
+      a.agg[l * a.layer_out_stride + tok] = best;
+      continue;
+    }
+    total = combine_layers(total, best, l, a, tok);
+  }
+  if (!a.layer_out_stride) a.agg[tok] = finalize(total, a);
 }
 
 // Layer scores [n_layers][stride] -> aggregate: layers combined in layer order
@@ -927,6 +996,14 @@ int launch_aggregate(const char* who, kvc_stream_t stream, int n_layers, int n_h
   aa.layer_out_stride = layer_out_stride;
   const size_t lds = static_cast<size_t>(2) * n_layers * n_heads * sizeof(float);
   if (raw_token_stride == 1) {
+    const int slices = static_cast<int>(ceil_div(n_heads, kAggSliceHeads));
+    const int64_t groups = ceil_div(max_seq_len, 32) * n_seq;
+    if (groups <= kAggSplitMaxGroups && slices * n_layers > 1 && slices * n_layers <= kAggMaxItems) {
+      dim3 grid(static_cast<unsigned>(ceil_div(max_seq_len, 32)), static_cast<unsigned>(n_seq));
+      aggregate_split_kernel<<<grid, 64 * kAggSplitWaves, lds + slices * n_layers * 32 * sizeof(float), as_stream(stream)>>>(
+          aa, slices);
+      return launch_status(who);
+    }
     dim3 grid(static_cast<unsigned>(ceil_div(max_seq_len, kAggTokPerBlock)), static_cast<unsigned>(n_seq));
     aggregate_tokens_kernel<<<grid, kAggThreads, lds, as_stream(stream)>>>(aa);
     return launch_status(who);
