@@ -619,6 +619,56 @@ def test_select_split_matches_single_and_brute_force(hip_device, case, ties) -> 
         np.testing.assert_array_equal(split[b, :budget].cpu().numpy(), want)
 
 
+def _score_distribution(kind: str, n: int, g: torch.Generator) -> torch.Tensor:
+    x = torch.randn(n, generator=g)
+    if kind == "outlier":  # +inf aggregates become 1e30: every other score falls into one value bin
+        x[n // 2] = 1e30
+    elif kind == "past-float32":  # a range that overflows
+        x[0], x[-1] = 3.3e38, -3.3e38
+    elif kind == "few-ulps":
+        x = 1.0 + torch.randint(0, 5, (n,), generator=g) * 2.0**-23
+    elif kind == "two-values":
+        x = torch.where(x > 0.3, 2.0, -1.0)
+    elif kind == "constant":
+        x = torch.full((n,), -0.25)
+    elif kind == "full-bin":  # more scores in the threshold's bin than are ranked against each other
+        x = x * 1e-5
+        x[:: max(n // 7, 1)] = 5.0
+    elif kind == "unresolved":  # NaN layers finalise to -inf
+        x[torch.rand(n, generator=g) < 0.7] = float("-inf")
+        x[n // 3] = float("nan")
+    elif kind == "signed-zeros":
+        x = torch.where(x > 0, 0.0, -0.0)
+        x[n // 4] = 1.0
+    return x
+
+
+@pytest.mark.parametrize(
+    "kind", ["normal", "outlier", "past-float32", "few-ulps", "two-values", "constant", "full-bin", "unresolved", "signed-zeros"]
+)
+def test_select_score_distributions(hip_device, kind) -> None:
+    # The threshold comes from value bins or, where those do not separate the
+    # scores, from radix passes; lengths around the single read of a segment
+    # (16384 scores) and its second walk, misaligned starts, keep counts from
+    # one score to all but one.
+    _, selection, _ = _kvc()
+    g = torch.Generator().manual_seed(len(kind))
+    lens = [2, 7, 1027, 2050, 16384, 16389, 20011]
+    parts = [_score_distribution(kind, n, g) for n in lens]
+    offsets = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    d_scores = torch.cat(parts).to(hip_device)
+    for i, (n, part) in enumerate(zip(lens, parts)):
+        for keep_count in sorted({1, 2, n // 3 + 1, n - 1}):
+            seq_lens = torch.tensor([n], dtype=torch.int32, device=hip_device)
+            token_offsets = torch.tensor(offsets[i : i + 2], dtype=torch.int64, device=hip_device)
+            keep = torch.full((1, keep_count), -7, dtype=torch.int64, device=hip_device)
+            selection.select_keep_indices_batched(
+                d_scores, seq_lens, token_offsets, [n], keep, budget=keep_count, protected_prefix=0, protected_recent=0,
+                segments=1, policy="global", shape="single",
+            )
+            np.testing.assert_array_equal(keep[0].cpu().numpy(), _stable_keep_np(part.numpy(), keep_count, 0, 0, 1, "global"))
+
+
 def test_select_split_rejects_a_small_workspace(hip_device) -> None:
     _, selection, _ = _kvc()
     scores = torch.randn(50000, device=hip_device)

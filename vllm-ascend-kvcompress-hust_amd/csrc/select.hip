@@ -1,18 +1,19 @@
-// Per-sequence keep-set selection on CDNA4: segmented radix select.
+// Per-sequence keep-set selection on CDNA4: segmented threshold select.
 //
 // A job is one (sequence, segment).  The segment's scores are mapped to
-// order-preserving 32-bit keys; four 8-bit radix passes build LDS histograms
-// of the keys that still match the selected high digits and walk them from
-// the top, which pins the exact key T of the K-th largest score and how many
-// scores equal to T are still needed.  Emission keeps every key > T plus the
-// first `need` keys == T (ties go to the lowest index), walking the segment in
-// coalesced tiles: one workgroup prefix sum of packed (greater, equal) counts
-// per tile gives every key its output slot, so the output is sorted without a
-// sort.
+// order-preserving 32-bit keys; the exact key T of the K-th largest score and
+// how many scores equal to T are still needed come from a histogram over value
+// bins and an exact ranking inside one bin, or from four 8-bit radix passes
+// (LDS histograms of the keys that still match the selected high digits).
+// Emission keeps every key > T plus the first `need` keys == T (ties go to the
+// lowest index), walking the segment in coalesced tiles: prefix sums of packed
+// (greater, equal) counts give every key its output slot, so the output is
+// sorted without a sort.
 //
 // Two launch shapes:
-//  * kvc_select_keep: one 1024-thread workgroup per job; every pass stays in
-//    the workgroup.  Right for batches of many sequences.
+//  * kvc_select_keep: one 1024-thread workgroup per job (value bins, radix
+//    passes where they do not separate the scores).  Right for batches of many
+//    sequences.
 //  * kvc_select_keep_split: a job's segment is cut into chunks of >= 4096 keys,
 //    one 256-thread workgroup each.  Every radix pass is a launch: workgroups
 //    add their chunk histograms into the pass's histogram in the workspace;
@@ -41,7 +42,6 @@ constexpr int kSplitMaxChunks = 64;
 constexpr int kSelUnroll = 4;  // float4 words per thread in flight in a histogram pass
 constexpr int kEmitWords = 2;  // float4 words per thread per emission tile
 constexpr int kSelPeel = 1;    // dominant digits counted with one atomic per wave
-static_assert(kSelThreads * kEmitWords * 4 < 65536, "packed emission counts need 16 bits per half");
 
 struct SelectArgs {
   int n_seq, budget, prefix, recent, segments, policy;
@@ -57,10 +57,22 @@ struct Segment {
   int64_t start, stop, keep;
 };
 
-__device__ Segment v3_segment(int64_t ms, int64_t mc, int64_t evict, int k, int nseg) {
+// floor(p / c) for p >= 0, c > 0 and a quotient below 2^31 (scores of one
+// sequence): the double quotient is off by one at most, which the remainder
+// shows.  The compiler's 64-bit division is some 150 instructions, five of
+// them a job.
+__device__ __forceinline__ int64_t div_floor(int64_t p, int64_t c) {
+  int64_t q = static_cast<int64_t>(static_cast<double>(p) / static_cast<double>(c));
+  const int64_t r = p - q * c;
+  if (r < 0) --q;
+  if (r >= c) ++q;
+  return q;
+}
+
+__device__ __forceinline__ Segment v3_segment(int64_t ms, int64_t mc, int64_t evict, int k, int nseg) {
   Segment s;
-  s.start = ms + mc * k / nseg;
-  s.stop = ms + mc * (k + 1) / nseg;
+  s.start = ms + div_floor(mc * k, nseg);
+  s.stop = ms + div_floor(mc * (k + 1), nseg);
   const int64_t len = s.stop - s.start;
   if (len <= 0) {
     s.keep = 0;
@@ -95,8 +107,16 @@ __device__ Job make_job(const SelectArgs& a, int b, int seg) {
   if (a.policy == KVC_POLICY_V3) {
     if (mc <= 0) return j;
     const int64_t evict = j.n - a.budget;
-    for (int k = 0; k < seg; ++k) j.out_base += v3_segment(ms, mc, evict, k, nseg).keep;
     j.s = v3_segment(ms, mc, evict, seg, nseg);
+    if (evict >= 0 && evict <= mc) {
+      // Every quota is len - (after - before) >= 0 then, so the quotas before
+      // this segment telescope (a chain of 64-bit divisions per segment cost
+      // the eighth segment's workgroup 2 us before its first load).
+      const int64_t before = j.s.start - ms;
+      j.out_base += before - div_floor(evict * before, mc);
+    } else {
+      for (int k = 0; k < seg; ++k) j.out_base += v3_segment(ms, mc, evict, k, nseg).keep;
+    }
   } else {
     j.s = Segment{ms, ms + mc, a.budget - j.prefix - j.recent};
   }
@@ -123,16 +143,16 @@ __device__ bool fill_fixed(const SelectArgs& a, const Job& j, int seg, int64_t* 
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// Calls f(i, key) for every i in [start, stop), spread over a workgroup of T
-// threads: scalar head up to 16-byte alignment, float4 words kSelUnroll at a
+// Calls f(score) for every score in [start, stop), spread over a workgroup of
+// T threads: scalar head up to 16-byte alignment, float4 words kSelUnroll at a
 // time (loads issued together), scalar tail.
 template <int T, typename F>
-__device__ __forceinline__ void for_each_key(const float* sc, int64_t start, int64_t stop, F&& f) {
+__device__ __forceinline__ void for_each_score(const float* sc, int64_t start, int64_t stop, F&& f) {
   const int tid = threadIdx.x;
   const int64_t misalign = (reinterpret_cast<uintptr_t>(sc + start) >> 2) & 3;
   int64_t head = (4 - misalign) & 3;
   if (head > stop - start) head = stop - start;
-  for (int64_t i = start + tid; i < start + head; i += T) f(i, float_key(sc[i]));
+  for (int64_t i = start + tid; i < start + head; i += T) f(sc[i]);
   const int64_t body = start + head;
   const int64_t n4 = (stop - body) >> 2;
   const f32x4* v = reinterpret_cast<const f32x4*>(sc + body);
@@ -148,11 +168,11 @@ __device__ __forceinline__ void for_each_key(const float* sc, int64_t start, int
       const int64_t w = w0 + static_cast<int64_t>(u) * T;
       if (w < n4) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f(body + 4 * w + e, float_key(x[u][e]));
+        for (int e = 0; e < 4; ++e) f(x[u][e]);
       }
     }
   }
-  for (int64_t i = body + 4 * n4 + tid; i < stop; i += T) f(i, float_key(sc[i]));
+  for (int64_t i = body + 4 * n4 + tid; i < stop; i += T) f(sc[i]);
 }
 
 // Exclusive prefix sum over a workgroup of T threads (thread order); *total
@@ -210,7 +230,8 @@ __device__ void range_histogram(const float* sc, int64_t start, int64_t stop, ui
   for (int i = tid; i < (T / 64) * 256; i += T) (&whist[0][0])[i] = 0;
   __syncthreads();
   uint32_t* mine = whist[tid >> 6];
-  for_each_key<T>(sc, start, stop, [&](int64_t, uint32_t k) {
+  for_each_score<T>(sc, start, stop, [&](float x) {
+    const uint32_t k = float_key(x);
     if ((k & mask) == want) count_digit(mine, (k >> shift) & 255u);
   });
   __syncthreads();
@@ -248,218 +269,377 @@ __device__ __forceinline__ void pick_digit(const uint32_t* hist, uint32_t need, 
   }
 }
 
+// What the emission keeps: key k iff k > thresh, or k == thresh and fewer than
+// need_eq ties precede it in the segment.  `all_ties`: every tie is kept (the
+// usual case, one key at the threshold), so one comparison k >= thresh decides.
+struct Keep {
+  uint32_t thresh, need_eq;
+  bool all_ties;
+  int64_t* out;  // the row of kept indices; slots past `budget` are not written
+  int out_base, budget;
+};
+
+__device__ __forceinline__ void emit_one(const Keep& kp, int64_t i, uint32_t k, uint32_t g, uint32_t e) {
+  if (k > kp.thresh || (k == kp.thresh && e < kp.need_eq)) {
+    const uint32_t slot = kp.out_base + g + min(e, kp.need_eq);
+    if (slot < static_cast<uint32_t>(kp.budget)) kp.out[slot] = i;
+  }
+}
+
+// Inclusive prefix sum over a wave's lanes: row shifts inside the rows of 16,
+// then each row's last lane into the next row and row 1's into rows 2 and 3
+// (VALU only; the same scan by lane exchanges is six LDS round trips).
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
+  int x = static_cast<int>(v);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
+  return static_cast<uint32_t>(x);
+}
+
+// One tile of the ordered emission by a workgroup of T threads: wave w holds
+// words [64 words w, 64 words (w + 1)) of the tile, lane l of it words l,
+// 64 + l, ... (coalesced, and wave, word, lane order is index order); words
+// from n_words on are not part of the segment.  A word's count is packed
+// (kept, ties apart unless all_ties); per word one scan over the lanes, and one
+// total per wave through LDS.  first: index of the tile's first score.  g_run,
+// e_run: keys > thresh and == thresh before the tile; with all_ties both kinds
+// count in g_run.
+template <int T, int K>
+__device__ __forceinline__ void emit_tile(const Keep& kp, const f32x4 (&x)[K], int words, int n_words, int64_t first,
+                                          uint32_t* s_wave, uint32_t* g_run, uint32_t* e_run) {
+  static_assert(T * K * 4 < 65536, "a tile's counts fit 16 bits each");
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int w0 = wave * 64 * words + lane;
+  const uint32_t tie = kp.all_ties ? 1u : 65536u;
+  uint32_t before[K];  // packed counts of the wave's earlier words, this one's earlier lanes
+  uint32_t mine = 0;
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    if (u < words) {
+      uint32_t c = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t k = float_key(x[u][q]);
+        c += k > kp.thresh ? 1u : (k == kp.thresh ? tie : 0u);
+      }
+      c = w0 + 64 * u < n_words ? c : 0u;
+      const uint32_t incl = wave_inclusive_scan(c);
+      before[u] = mine + incl - c;
+      mine += __builtin_amdgcn_readlane(incl, 63);
+    }
+  }
+  if (lane == 0) s_wave[wave] = mine;
+  __syncthreads();
+  uint32_t base = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) {
+    const uint32_t c = s_wave[w];
+    if (w < wave) base += c;
+    all += c;
+  }
+  if (kp.all_ties) {
+    const uint32_t slot0 = kp.out_base + *g_run + base;
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      if (u < words && w0 + 64 * u < n_words) {
+        uint32_t slot = slot0 + before[u];
+        const int64_t i0 = first + 4 * static_cast<int64_t>(w0 + 64 * u);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const bool take = float_key(x[u][q]) >= kp.thresh;
+          if (take && slot < static_cast<uint32_t>(kp.budget)) kp.out[slot] = i0 + q;
+          slot += take;
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      if (u < words && w0 + 64 * u < n_words) {
+        uint32_t g = *g_run + ((base + before[u]) & 0xFFFFu), e = *e_run + ((base + before[u]) >> 16);
+        const int64_t i0 = first + 4 * static_cast<int64_t>(w0 + 64 * u);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t k = float_key(x[u][q]);
+          emit_one(kp, i0 + q, k, g, e);
+          g += k > kp.thresh;
+          e += k == kp.thresh;
+        }
+      }
+    }
+  }
+  *g_run += all & 0xFFFFu;
+  *e_run += all >> 16;
+}
+
+// Counts `n` of three scores before or after the words and, in thread 0, emits them.
+__device__ __forceinline__ void emit_ends(const Keep& kp, float x0, float x1, float x2, int n, int64_t first,
+                                          uint32_t* g_run, uint32_t* e_run) {
+  const float x[3] = {x0, x1, x2};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    if (i < n) {
+      const uint32_t k = float_key(x[i]);
+      if (threadIdx.x == 0) emit_one(kp, first + i, k, *g_run, kp.all_ties ? 0u : *e_run);
+      const bool eq = k == kp.thresh;
+      *g_run += k > kp.thresh || (kp.all_ties && eq);
+      if (!kp.all_ties) *e_run += eq;
+    }
+  }
+}
+
 // Ordered emission of [start, stop) by a workgroup of T threads, given the
 // numbers g_run, e_run of keys > thresh and == thresh before `start` in the
-// segment.  Key i is kept iff k > thresh, or k == thresh and fewer than
-// need_eq ties precede it; its slot is out_base + G(i) + min(E(i), need_eq).
-// Tiles of T*kEmitWords float4 words: thread t takes the tile's words
-// [t*kEmitWords, (t+1)*kEmitWords), so loads are coalesced and thread order is
-// index order; one scan of packed (G, E) counts per tile.  The up to three
-// keys before the first 16-byte boundary and after the last are counted by
-// every thread and written by thread 0.
+// segment (all_ties: their sum in g_run), in tiles of T * kEmitWords float4
+// words; the up to three scores before the first 16-byte boundary and after
+// the last are counted by every thread and written by thread 0.
 template <int T>
-__device__ void emit_range(const float* sc, int64_t start, int64_t stop, uint32_t thresh, uint32_t need_eq,
-                           uint32_t g_run, uint32_t e_run, int64_t* out, int64_t out_base, int budget,
+__device__ __forceinline__ void emit_range(const Keep& kp, const float* sc, int64_t start, int64_t stop, uint32_t g_run, uint32_t e_run,
                            uint32_t* s_wave) {
-  const int tid = threadIdx.x;
-  auto emit = [&](int64_t i, uint32_t k, uint32_t g, uint32_t e) {
-    if (k > thresh || (k == thresh && e < need_eq)) {
-      const int64_t slot = out_base + g + min(e, need_eq);
-      if (slot < budget) out[slot] = i;
-    }
-  };
-  auto serial = [&](int64_t i0, int64_t i1) {
-    for (int64_t i = i0; i < i1; ++i) {
-      const uint32_t k = float_key(sc[i]);
-      if (tid == 0) emit(i, k, g_run, e_run);
-      g_run += k > thresh;
-      e_run += k == thresh;
-    }
-  };
   const int64_t misalign = (reinterpret_cast<uintptr_t>(sc + start) >> 2) & 3;
   const int64_t head = min((4 - misalign) & 3, stop - start);
-  serial(start, start + head);
   const int64_t body = start + head;
   const int64_t n4 = (stop - body) >> 2;
-  const f32x4* v = reinterpret_cast<const f32x4*>(sc + body);
-  for (int64_t w0 = 0; w0 < n4; w0 += static_cast<int64_t>(T) * kEmitWords) {
-    uint32_t k[kEmitWords][4];
-    bool valid[kEmitWords];
-    uint32_t g = 0, e = 0;
+  const int64_t tail0 = body + 4 * n4;
+  float ends[6];
 #pragma unroll
-    for (int u = 0; u < kEmitWords; ++u) {
-      const int64_t w = w0 + static_cast<int64_t>(tid) * kEmitWords + u;
-      valid[u] = w < n4;
-      const f32x4 x = v[valid[u] ? w : n4 - 1];  // in range; surplus words are masked
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        k[u][q] = float_key(x[q]);
-        g += valid[u] && k[u][q] > thresh;
-        e += valid[u] && k[u][q] == thresh;
-      }
-    }
-    uint32_t tile_total;
-    // Per-tile counts stay below 2^16 (T * kEmitWords * 4 keys), so the two
-    // halves of the packed sum never carry into each other.
-    const uint32_t before = block_exclusive_scan<T>(g | (e << 16), s_wave, &tile_total);
-    uint32_t gb = g_run + (before & 0xFFFFu), eb = e_run + (before >> 16);
-#pragma unroll
-    for (int u = 0; u < kEmitWords; ++u) {
-      const int64_t i0 = body + 4 * (w0 + static_cast<int64_t>(tid) * kEmitWords + u);
-      if (!valid[u]) continue;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        emit(i0 + q, k[u][q], gb, eb);
-        gb += k[u][q] > thresh;
-        eb += k[u][q] == thresh;
-      }
-    }
-    g_run += tile_total & 0xFFFFu;
-    e_run += tile_total >> 16;
+  for (int i = 0; i < 3; ++i) {
+    ends[i] = sc[min(start + i, stop - 1)];
+    ends[3 + i] = sc[min(tail0 + i, stop - 1)];
   }
-  serial(body + 4 * n4, stop);
+  emit_ends(kp, ends[0], ends[1], ends[2], static_cast<int>(head), start, &g_run, &e_run);
+  const f32x4* v = reinterpret_cast<const f32x4*>(sc + body);
+  constexpr int64_t kTile = static_cast<int64_t>(T) * kEmitWords;
+  const int w0 = (threadIdx.x >> 6) * 64 * kEmitWords + (threadIdx.x & 63);
+  for (int64_t t0 = 0; t0 < n4; t0 += kTile) {
+    f32x4 x[kEmitWords];
+    const int left = static_cast<int>(min(n4 - t0, kTile));
+#pragma unroll
+    for (int u = 0; u < kEmitWords; ++u) x[u] = v[t0 + min(w0 + 64 * u, left - 1)];  // in range; surplus words are masked
+    emit_tile<T, kEmitWords>(kp, x, kEmitWords, left, body + 4 * t0, s_wave, &g_run, &e_run);
+    __syncthreads();  // s_wave is reused by the next tile
+  }
+  emit_ends(kp, ends[3], ends[4], ends[5], static_cast<int>(stop - tail0), tail0, &g_run, &e_run);
 }
 
 // ------------------------------------------------- one workgroup per job --
 
-// Segments whose aligned body has at most kCacheTiles emission tiles (16 384
-// scores at 1024 threads) are read once: each thread keeps its words of every
-// tile in registers, in the emission's layout, and the four radix passes and
-// the emission walk those (the up to three scores before the first and after
-// the last 16-byte boundary are read again each time, as in the uncached
-// walk).
-constexpr int kCacheTiles = 2;
+// Segments whose aligned body has at most kCacheWords float4 words a thread
+// (16 384 scores at 1024 threads) are read once, into registers, in the
+// emission's layout with as few words a thread as hold the segment.
+constexpr int kCacheWords = 4;
 
-__global__ __launch_bounds__(kSelThreads) void select_kernel(SelectArgs a) {
+// The threshold by value bins: the scores' range is cut into kBins equal bins,
+// one histogram of which names the bin that holds the K-th largest score; that
+// bin's keys (a few dozen of 16 K aggregated scores) are gathered and ranked
+// exactly against each other.  bin(x) = trunc((x - lo) * scale) is a
+// composition of roundings that never decrease, so bins keep the order of the
+// keys.  One walk over scores that spread over many bins, where a radix pass
+// on the sign and exponent sends most lanes of a wave to the same two
+// counters, four times over.  Scores that defeat it (an infinity or NaN, a
+// range of zero or past float32, or more than kMaxCand keys in the bin: heavy
+// ties, an outlier of 1e30) take the four radix passes instead.  One
+// workgroup's instructions per score bound this kernel (1024 threads on one
+// CU), not its loads.  Microseconds per launch against the radix passes: one
+// 4096-score sequence 7.4 / 11.2, 16 x 16384 11.3 / 18.1, 8 x 65536 in eight v3
+// segments 9.7 / 17.6, one of 65000 31 / 53.
+constexpr int kBins = 2048;
+constexpr int kMaxCand = 1024;
+static_assert(kBins == 2 * kSelThreads, "a thread owns two bins of the scan");
+static_assert(kMaxCand <= kSelThreads, "a thread ranks one candidate");
+
+struct Picked {
+  uint32_t thresh, need_eq, ties;  // key of the K-th largest score, its ties to keep, all its ties
+};
+
+// The threshold by four radix passes over the scores.  Out of line, as
+// select_long below: what most calls run stays small in the instruction cache.
+__device__ __noinline__ Picked radix_threshold(const float* sc, int64_t start, int64_t stop, uint32_t need) {
   __shared__ uint32_t whist[kSelThreads / 64][256];
   __shared__ uint32_t hist[256];
   __shared__ uint32_t s_digit, s_need;
+  Picked p{0u, need, 0u};
+  uint32_t mask = 0;
+  for (int pass = 0; pass < 4; ++pass) {
+    const int shift = 24 - 8 * pass;
+    range_histogram<kSelThreads>(sc, start, stop, p.thresh, mask, shift, whist, hist);
+    if (threadIdx.x < 64) pick_digit(hist, p.need_eq, &s_digit, &s_need);
+    __syncthreads();
+    p.thresh |= s_digit << shift;
+    mask |= 0xFFu << shift;
+    p.need_eq = s_need;
+    p.ties = hist[s_digit];
+    __syncthreads();
+  }
+  return p;
+}
+
+// Keeps the `keep` largest scores of [start, stop), their indices written from
+// slot out_base on.  CACHED: at most kCacheWords words a thread.
+template <bool CACHED>
+__device__ __forceinline__ void select_segment(const float* sc, int64_t start, int64_t stop, uint32_t keep, int64_t* out,
+                                               int out_base, int budget) {
+  __shared__ uint32_t bins[kBins];
+  __shared__ uint32_t cand[kMaxCand];
+  __shared__ uint32_t s_bin, s_need, s_count, s_filled;
   __shared__ uint32_t s_wave[kSelThreads / 64];
-
-  const int b = blockIdx.y;
-  const int seg = blockIdx.x;
+  __shared__ float s_range[3][kSelThreads / 64];
   const int tid = threadIdx.x;
-  const Job j = make_job(a, b, seg);
-  int64_t* out = a.keep + static_cast<int64_t>(b) * a.keep_stride;
-  if (!fill_fixed(a, j, seg, out, tid, kSelThreads)) return;
-  const float* sc = a.scores + a.token_offsets[b];
-
-  constexpr int64_t kTileWords = static_cast<int64_t>(kSelThreads) * kEmitWords;
-  const int64_t start = j.s.start, stop = j.s.stop;
+  const int lane = tid & 63, wave = tid >> 6;
   const int64_t misalign = (reinterpret_cast<uintptr_t>(sc + start) >> 2) & 3;
   const int64_t head = min((4 - misalign) & 3, stop - start);
   const int64_t body = start + head;
   const int64_t n4 = (stop - body) >> 2;
   const int64_t tail0 = body + 4 * n4;
   const f32x4* v = reinterpret_cast<const f32x4*>(sc + body);
-  const bool cached = n4 <= kCacheTiles * kTileWords;
-  uint32_t ck[kCacheTiles][kEmitWords][4];
-  bool cv[kCacheTiles][kEmitWords];
-  if (cached) {
+  const int words = CACHED ? static_cast<int>((n4 + kSelThreads - 1) / kSelThreads) : 0;
+  const int n_words = static_cast<int>(CACHED ? n4 : 0);
+  const int w0 = wave * 64 * words + lane;
+  f32x4 cx[kCacheWords];
+  float ends[6];  // the up to three scores before the first and after the last 16-byte boundary
+  if constexpr (CACHED) {
 #pragma unroll
-    for (int t = 0; t < kCacheTiles; ++t) {
+    for (int u = 0; u < kCacheWords; ++u)
+      if (u < words) cx[u] = v[min(w0 + 64 * u, n_words - 1)];  // surplus words are masked
 #pragma unroll
-      for (int u = 0; u < kEmitWords; ++u) {
-        const int64_t w = t * kTileWords + static_cast<int64_t>(tid) * kEmitWords + u;
-        cv[t][u] = w < n4;
-        const f32x4 x = cv[t][u] ? v[w] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) ck[t][u][q] = float_key(x[q]);
-      }
+    for (int e = 0; e < 3; ++e) {
+      ends[e] = sc[min(start + e, stop - 1)];
+      ends[3 + e] = sc[min(tail0 + e, stop - 1)];
     }
   }
-
-  uint32_t want = 0, mask = 0;
-  uint32_t need = static_cast<uint32_t>(j.s.keep);
-  for (int pass = 0; pass < 4; ++pass) {
-    const int shift = 24 - 8 * pass;
-    if (cached) {
-      for (int i = tid; i < (kSelThreads / 64) * 256; i += kSelThreads) (&whist[0][0])[i] = 0;
-      __syncthreads();
-      uint32_t* mine = whist[tid >> 6];
-      auto count = [&](uint32_t k) {
-        if ((k & mask) == want) count_digit(mine, (k >> shift) & 255u);
-      };
-      for (int64_t i = start + tid; i < body; i += kSelThreads) count(float_key(sc[i]));
+  const int n_head = static_cast<int>(head), n_tail = static_cast<int>(stop - tail0);
+  float my_end = 0.0f;  // lane e < 3 counts the head's score e, lane 3 + e the tail's
+  if constexpr (CACHED) {
 #pragma unroll
-      for (int t = 0; t < kCacheTiles; ++t)
-#pragma unroll
-        for (int u = 0; u < kEmitWords; ++u)
-          if (cv[t][u]) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) count(ck[t][u][q]);
-          }
-      for (int64_t i = tail0 + tid; i < stop; i += kSelThreads) count(float_key(sc[i]));
-      __syncthreads();
-      for (int i = tid; i < 256; i += kSelThreads) {
-        uint32_t c = 0;
-#pragma unroll
-        for (int w = 0; w < kSelThreads / 64; ++w) c += whist[w][i];
-        hist[i] = c;
-      }
-      __syncthreads();
+    for (int e = 0; e < 6; ++e) my_end = tid == e ? ends[e] : my_end;
+  }
+  // f(score) for every score of the segment, each by one thread.
+  auto walk = [&](auto&& f) {
+    if constexpr (!CACHED) {
+      for_each_score<kSelThreads>(sc, start, stop, f);
     } else {
-      range_histogram<kSelThreads>(sc, start, stop, want, mask, shift, whist, hist);
-    }
-    if (tid < 64) pick_digit(hist, need, &s_digit, &s_need);
-    __syncthreads();
-    want |= s_digit << shift;
-    mask |= 0xFFu << shift;
-    need = s_need;
-    __syncthreads();
-  }
-  // want: the exact key of the K-th largest score; need: its ties to keep.
-  if (!cached) {
-    emit_range<kSelThreads>(sc, start, stop, want, need, 0u, 0u, out, j.out_base, a.budget, s_wave);
-    return;
-  }
-  // The cached emission: emit_range's walk with the tiles' words from registers.
-  const uint32_t thresh = want, need_eq = need;
-  uint32_t g_run = 0, e_run = 0;
-  auto emit = [&](int64_t i, uint32_t k, uint32_t g, uint32_t e) {
-    if (k > thresh || (k == thresh && e < need_eq)) {
-      const int64_t slot = j.out_base + g + min(e, need_eq);
-      if (slot < a.budget) out[slot] = i;
+#pragma unroll
+      for (int u = 0; u < kCacheWords; ++u)
+        if (u < words && w0 + 64 * u < n_words) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) f(cx[u][q]);
+        }
+      if (tid < 6 && (tid < 3 ? tid < n_head : tid - 3 < n_tail)) f(my_end);
     }
   };
-  auto serial = [&](int64_t i0, int64_t i1) {
-    for (int64_t i = i0; i < i1; ++i) {
-      const uint32_t k = float_key(sc[i]);
-      if (tid == 0) emit(i, k, g_run, e_run);
-      g_run += k > thresh;
-      e_run += k == thresh;
-    }
-  };
-  serial(start, body);
+
+  // Range of the scores; `odd` ends as NaN if one of them is not finite.
+  for (int i = tid; i < kBins; i += kSelThreads) bins[i] = 0;
+  if (tid == 0) s_filled = 0;
+  float lo = INFINITY, hi = -INFINITY, odd = 0.0f;
+  walk([&](float x) {
+    lo = fminf(lo, x);
+    hi = fmaxf(hi, x);
+    odd = fmaf(x, 0.0f, odd);
+  });
 #pragma unroll
-  for (int t = 0; t < kCacheTiles; ++t) {
-    if (t * kTileWords >= n4) break;  // the same for every thread
-    uint32_t g = 0, e = 0;
-#pragma unroll
-    for (int u = 0; u < kEmitWords; ++u)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        g += cv[t][u] && ck[t][u][q] > thresh;
-        e += cv[t][u] && ck[t][u][q] == thresh;
-      }
-    uint32_t tile_total;
-    const uint32_t before = block_exclusive_scan<kSelThreads>(g | (e << 16), s_wave, &tile_total);
-    uint32_t gb = g_run + (before & 0xFFFFu), eb = e_run + (before >> 16);
-#pragma unroll
-    for (int u = 0; u < kEmitWords; ++u) {
-      if (!cv[t][u]) continue;
-      const int64_t i0 = body + 4 * (t * kTileWords + static_cast<int64_t>(tid) * kEmitWords + u);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        emit(i0 + q, ck[t][u][q], gb, eb);
-        gb += ck[t][u][q] > thresh;
-        eb += ck[t][u][q] == thresh;
-      }
-    }
-    g_run += tile_total & 0xFFFFu;
-    e_run += tile_total >> 16;
+  for (int off = 32; off >= 1; off >>= 1) {
+    lo = fminf(lo, __shfl_xor(lo, off));
+    hi = fmaxf(hi, __shfl_xor(hi, off));
+    odd += __shfl_xor(odd, off);
   }
-  serial(tail0, stop);
+  if (lane == 0) {
+    s_range[0][wave] = lo;
+    s_range[1][wave] = hi;
+    s_range[2][wave] = odd;
+  }
+  __syncthreads();
+  lo = s_range[0][0], hi = s_range[1][0], odd = s_range[2][0];
+#pragma unroll
+  for (int w = 1; w < kSelThreads / 64; ++w) {
+    lo = fminf(lo, s_range[0][w]);
+    hi = fmaxf(hi, s_range[1][w]);
+    odd += s_range[2][w];
+  }
+  // A little below kBins / (hi - lo), so that hi itself rounds to at most the last bin.
+  const float scale = (kBins - 1.0f / 512.0f) / (hi - lo);
+  auto bin_of = [&](float x) { return static_cast<int>((x - lo) * scale); };
+  Picked picked{0u, 0u, 0u};
+  // The same for every thread.  A range past float32 gives a scale of zero.
+  bool found = odd == 0.0f && hi > lo && scale > 0.0f && scale < INFINITY;
+  if (found) {
+    walk([&](float x) { atomicAdd(&bins[bin_of(x)], 1u); });
+    __syncthreads();
+    // Thread t owns bins kBins - 1 - 2t and the one below it: thread order is
+    // falling order of the scores.
+    const uint32_t c0 = bins[kBins - 1 - 2 * tid], c1 = bins[kBins - 2 - 2 * tid];
+    uint32_t total;
+    uint32_t above = block_exclusive_scan<kSelThreads>(c0 + c1, s_wave, &total);
+    if (above < keep && keep <= above + c0 + c1) {
+      const bool first = keep <= above + c0;
+      if (!first) above += c0;
+      s_bin = static_cast<uint32_t>(kBins - 1 - 2 * tid - (first ? 0 : 1));
+      s_need = keep - above;
+      s_count = first ? c0 : c1;
+    }
+    __syncthreads();
+    const int bin = static_cast<int>(s_bin);
+    const uint32_t count = s_count, rank = s_need;
+    found = count <= kMaxCand;
+    if (found) {
+      walk([&](float x) {
+        if (bin_of(x) == bin) cand[atomicAdd(&s_filled, 1u)] = float_key(x);
+      });
+      __syncthreads();
+      if (tid < count) {
+        const uint32_t mine = cand[tid];
+        uint32_t g = 0, e = 0;
+        for (uint32_t i = 0; i < count; ++i) {
+          g += cand[i] > mine;
+          e += cand[i] == mine;
+        }
+        if (g < rank && rank <= g + e) {  // every candidate equal to the threshold writes the same
+          s_bin = mine;
+          s_need = rank - g;
+          s_count = e;
+        }
+      }
+      __syncthreads();
+      picked = Picked{s_bin, s_need, s_count};
+    }
+  }
+  if (!found) picked = radix_threshold(sc, start, stop, keep);
+  const Keep kp{picked.thresh, picked.need_eq, picked.ties == picked.need_eq, out, out_base, budget};
+  if constexpr (CACHED) {
+    uint32_t g_run = 0, e_run = 0;
+    emit_ends(kp, ends[0], ends[1], ends[2], n_head, start, &g_run, &e_run);
+    emit_tile<kSelThreads, kCacheWords>(kp, cx, words, n_words, body, s_wave, &g_run, &e_run);
+    emit_ends(kp, ends[3], ends[4], ends[5], n_tail, tail0, &g_run, &e_run);
+  } else {
+    emit_range<kSelThreads>(kp, sc, start, stop, 0u, 0u, s_wave);
+  }
+}
+
+// Longer segments re-read the scores in every walk.  Out of line: the short
+// form's code then stays small in the instruction cache.
+__device__ __noinline__ void select_long(const float* sc, int64_t start, int64_t stop, uint32_t keep, int64_t* out,
+                                         int out_base, int budget) {
+  select_segment<false>(sc, start, stop, keep, out, out_base, budget);
+}
+
+__global__ __launch_bounds__(kSelThreads) void select_kernel(SelectArgs a) {
+  const int b = blockIdx.y;
+  const int seg = blockIdx.x;
+  const Job j = make_job(a, b, seg);
+  int64_t* out = a.keep + static_cast<int64_t>(b) * a.keep_stride;
+  if (!fill_fixed(a, j, seg, out, threadIdx.x, kSelThreads)) return;
+  const float* sc = a.scores + a.token_offsets[b];
+  const uint32_t keep = static_cast<uint32_t>(j.s.keep);
+  const int out_base = static_cast<int>(j.out_base);
+  if (j.s.stop - j.s.start <= 4 * kCacheWords * kSelThreads)
+    select_segment<true>(sc, j.s.start, j.s.stop, keep, out, out_base, a.budget);
+  else
+    select_long(sc, j.s.start, j.s.stop, keep, out, out_base, a.budget);
 }
 
 // ------------------------------------------------------ split over chunks --
@@ -577,7 +757,8 @@ __global__ __launch_bounds__(kSplitThreads) void select_split_count_kernel(Selec
   const uint32_t thresh = s_th.want;
   const float* sc = a.scores + a.token_offsets[b];
   uint32_t g = 0, e = 0;
-  for_each_key<kSplitThreads>(sc, c0, c1, [&](int64_t, uint32_t k) {
+  for_each_score<kSplitThreads>(sc, c0, c1, [&](float x) {
+    const uint32_t k = float_key(x);
     g += k > thresh;
     e += k == thresh;
   });
@@ -610,8 +791,9 @@ __global__ __launch_bounds__(kSplitThreads) void select_split_emit_kernel(Select
   }
   derive_threshold(st, 4, s_prev, &s_th);
   int64_t* out = a.keep + static_cast<int64_t>(b) * a.keep_stride;
-  emit_range<kSplitThreads>(a.scores + a.token_offsets[b], c0, c1, s_th.want, s_th.need, g0, e0, out, j.out_base,
-                            a.budget, s_wave);
+  // Whether a later chunk holds ties is not known here: ties count apart.
+  const Keep kp{s_th.want, s_th.need, false, out, static_cast<int>(j.out_base), a.budget};
+  emit_range<kSplitThreads>(kp, a.scores + a.token_offsets[b], c0, c1, g0, e0, s_wave);
 }
 
 int check_select_args(const char* who, int n_seq, int max_seq_len, const int32_t* seq_lens,
