@@ -233,6 +233,96 @@ def test_score_paged_max_matches_oracle(hip_device, case) -> None:
     assert float((want - mean).abs().max()) > 1e-2
 
 
+# Head shapes whose K steps of 32 are partly filled, or that keep three words a
+# weight: remainders of the frequencies and of the pass dims, 1 to 10 steps.
+PART_SHAPES = [
+    # (kv, qpk, head_dim, rotary, style, dtype, tokens)
+    (2, 4, 96, 96, "half", torch.bfloat16, 700),
+    (8, 1, 96, 96, "interleaved", torch.float16, 129),
+    (4, 3, 80, 80, "half", torch.float16, 257),
+    (2, 8, 80, 80, "interleaved", torch.bfloat16, 300),
+    (1, 5, 16, 16, "half", torch.bfloat16, 128),
+    (4, 4, 128, 32, "half", torch.bfloat16, 513),
+    (2, 7, 128, 32, "interleaved", torch.float16, 33),
+    (4, 2, 192, 192, "half", torch.bfloat16, 400),
+    (1, 8, 192, 64, "interleaved", torch.bfloat16, 270),
+    (2, 2, 256, 16, "half", torch.float16, 300),
+    (2, 3, 256, 224, "half", torch.bfloat16, 290),
+    (1, 6, 256, 208, "interleaved", torch.bfloat16, 1),
+    (8, 2, 112, 48, "half", torch.float16, 1000),
+]
+
+
+def _layer_scores(kernels, device, cache, blocks, stats, cos, sin, tokens):
+    d = lambda t: None if t is None else t.to(device)  # noqa: E731
+    kv, qpk = stats.q_mean_real.shape[:2]
+    out = torch.full((kv, qpk, tokens), 7.0, device=device)
+    extra = stats.q_abs_mean - torch.sqrt(stats.q_mean_real.square() + stats.q_mean_imag.square() + 1e-8)
+    kernels.score_paged_keys_mean_precomputed(
+        cache.to(device), blocks.to(device), d(stats.q_mean_real), d(stats.q_mean_imag), d(torch.sqrt(stats.freq_scale_sq)),
+        d(extra), d(cos), d(sin), tokens, out, 128, stats.rope_style, q_pass_mean=d(stats.q_pass_mean), rotary_dim=stats.rotary_dim)
+    return out.cpu(), extra
+
+
+@pytest.mark.parametrize("case", PART_SHAPES, ids=[f"kv{c[0]}q{c[1]}d{c[2]}r{c[3]}{c[4][0]}{str(c[5]).split('.')[-1]}t{c[6]}" for c in PART_SHAPES])
+def test_score_paged_part_steps_keep_float32(hip_device, case) -> None:
+    """Within float32's rounding of a float64 evaluation of the same inputs.
+    With S the sum of the terms' magnitudes, the fold rounds each weight about
+    4 times, its words and those of |k| drop 2^-24 each and the accumulators
+    add at most S per step: 16 x 2^-24 x S covers them (two 16-bit bf16 words
+    a weight would be off by up to 2^-17 x S)."""
+    kernels, _, _ = _kvc()
+    kv, qpk, head_dim, rotary, style, dtype, tokens = case
+    g = torch.Generator().manual_seed(sum(case[:4]) + tokens)
+    freq = rotary // 2
+    stats = _random_stats(g, kv, qpk, freq, head_dim - rotary, rotary, style=style)
+    n_blocks = -(-tokens // 128)
+    cache = torch.randn(n_blocks + 3, 128, kv, head_dim, generator=g).to(dtype)
+    blocks = torch.randperm(n_blocks + 3, generator=g)[:n_blocks]
+    phase = torch.rand(freq, generator=g) * 6.0
+    cos, sin = 0.7 * torch.cos(phase), 0.7 * torch.sin(phase)
+    got, extra = _layer_scores(kernels, hip_device, cache, blocks, stats, cos, sin, tokens)
+    keys = cache[blocks].reshape(-1, kv, head_dim)[:tokens].double().permute(1, 2, 0).unsqueeze(1)  # [kv, 1, D, tokens]
+    re, im = (keys[:, :, 0:rotary:2], keys[:, :, 1:rotary:2]) if style == "interleaved" else (keys[:, :, :freq], keys[:, :, freq:rotary])
+    a, qr, qi, e = (t.double().unsqueeze(-1) for t in (torch.sqrt(stats.freq_scale_sq), stats.q_mean_real, stats.q_mean_imag, extra))
+    c, s = cos.double().view(-1, 1), sin.double().view(-1, 1)
+    terms = [a * qr * c * re, -a * qi * s * re, a * qi * c * im, a * qr * s * im, a * e * torch.sqrt(re * re + im * im)]
+    if head_dim > rotary:
+        terms.append(stats.q_pass_mean.double().unsqueeze(-1) * keys[:, :, rotary:])
+    want = sum(t.sum(2) for t in terms)
+    size = sum(t.abs().sum(2) for t in terms)
+    err = (got.double() - want).abs() / size
+    assert float(err.max()) <= 16 * 2.0**-24, float(err.max() * 2**24)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_score_paged_part_steps_non_finite_keys(hip_device, dtype) -> None:
+    """Infinite, NaN and overflowing keys reach their own token's scores as in
+    float32 (an infinity stays one), and no other token's."""
+    kernels, _, _ = _kvc()
+    kv, qpk, dim, tokens = 2, 3, 96, 200
+    g = torch.Generator().manual_seed(5)
+    stats = _random_stats(g, kv, qpk, dim // 2, 0, dim)
+    cache = torch.randn(3, 128, kv, dim, generator=g).to(dtype)
+    blocks = torch.tensor([2, 0])
+    phase = torch.rand(dim // 2, generator=g) * 6.0
+    clean, _ = _layer_scores(kernels, hip_device, cache, blocks, stats, torch.cos(phase), torch.sin(phase), tokens)
+    big = 1e30 if dtype == torch.bfloat16 else 60000.0
+    for t, value in ((3, float("inf")), (77, float("nan")), (140, -float("inf")), (199, big)):
+        cache[blocks[t // 128], t % 128, 1, 17] = value
+    got, extra = _layer_scores(kernels, hip_device, cache, blocks, stats, torch.cos(phase), torch.sin(phase), tokens)
+    keys = cache[blocks].reshape(-1, kv, dim)[:tokens].float()
+    a, qr, qi = torch.sqrt(stats.freq_scale_sq), stats.q_mean_real, stats.q_mean_imag
+    c, s = torch.cos(phase), torch.sin(phase)
+    hit = [3, 77, 140, 199]
+    for t in hit:
+        re, im = keys[t, 1, : dim // 2], keys[t, 1, dim // 2 :]
+        want = (a * (qr * c - qi * s) * re + a * (qi * c + qr * s) * im + a * extra * torch.sqrt(re * re + im * im))[1].sum(-1)
+        torch.testing.assert_close(got[1, :, t], want, rtol=1e-5, atol=1e-4 if abs(want).max() < 1e4 else 0.0, equal_nan=True)
+    rest = [t for t in range(tokens) if t not in hit]
+    assert torch.equal(got[:, :, rest], clean[:, :, rest]) and torch.equal(got[0], clean[0])
+
+
 @pytest.mark.parametrize("case", FP16_RANGE_CASES, ids=[f"k{c[0]:g}w{min(c[1]):g}-{max(c[1]):g}" for c in FP16_RANGE_CASES])
 def test_score_paged_max_fp16_ranges(hip_device, case) -> None:
     # fp16 keys up to +-65000 (|k| past fp16's range) and query heads whose

@@ -34,6 +34,8 @@ template <>
 struct MfmaElem<false> {
   typedef bf16x8 vec;
   static constexpr float kMagScale = 1.0f;
+  static constexpr float kLowScale = 1.0f;
+  static constexpr uint32_t kLeadMask = 0xffffu;
   __device__ __forceinline__ static f32x4 mfma(vec a, vec b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
@@ -45,6 +47,12 @@ template <>
 struct MfmaElem<true> {
   typedef f16x8 vec;
   static constexpr float kMagScale = 0.25f;  // |k| of fp16 keys reaches 2^16.5
+  // Of three words the first keeps eight significant bits, as bf16 does: its
+  // products then leave the matrix core's sum the bits that full fp16 products
+  // would use up.  The lower two words of |k| are held times 2^8 (at most
+  // 2^15), clear of fp16's subnormals; their products are scaled back.
+  static constexpr float kLowScale = 1.0f / 256.0f;
+  static constexpr uint32_t kLeadMask = 0xfff8u;
   __device__ __forceinline__ static f32x4 mfma(vec a, vec b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -68,16 +76,17 @@ __device__ __forceinline__ uint32_t bf16_bits(float x) {
 __device__ __forceinline__ float bf16_value(uint32_t bits) { return __uint_as_float(bits << 16); }
 
 // |k| of the eight frequencies of magnitude K step q held by this lane, as
-// hi/lo 16-bit A operands (hi + lo = |k| * kMagScale to ~2^-16).  Two
+// TERMS 16-bit A operands, each the rounding of what the ones before it leave
+// (two: |k| * kMagScale to ~2^-16; three: to float32, the lower two divided by
+// kLowScale).  Two
 // frequencies per output word: half style pairs word w of linear steps q
 // (real parts) and q + NF (imaginary parts); interleaved takes words 2w, 2w+1
 // of step 2q (w < 2) or 2q + 1, each word one (real, imaginary) pair.
-template <bool F16, bool IL, int NK, int NF>
-__device__ __forceinline__ void magnitude_operands(const u32x4 (&ka)[NK], int q, typename MfmaElem<F16>::vec* khi,
-                                                   typename MfmaElem<F16>::vec* klo) {
+template <bool F16, bool IL, int NK, int NF, int TERMS>
+__device__ __forceinline__ void magnitude_words(const u32x4 (&ka)[NK], int q, typename MfmaElem<F16>::vec (&out)[TERMS]) {
   typedef MfmaElem<F16> E;
   typedef typename E::vec vec_t;
-  u32x4 hi, lo;
+  u32x4 words[TERMS];
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
     uint32_t re_w, im_w;
@@ -92,14 +101,23 @@ __device__ __forceinline__ void magnitude_operands(const u32x4 (&ka)[NK], int q,
     }
     const float re0 = E::lo(re_w), re1 = E::hi(re_w);
     const float im0 = E::lo(im_w), im1 = E::hi(im_w);
-    const float m0 = __builtin_amdgcn_sqrtf(fmaf(im0, im0, re0 * re0)) * E::kMagScale;
-    const float m1 = __builtin_amdgcn_sqrtf(fmaf(im1, im1, re1 * re1)) * E::kMagScale;
-    const uint32_t hw = E::pack(m0, m1);
-    hi[w] = hw;
-    lo[w] = E::pack(m0 - E::lo(hw), m1 - E::hi(hw));
+    float m0 = __builtin_amdgcn_sqrtf(fmaf(im0, im0, re0 * re0)) * E::kMagScale;
+    float m1 = __builtin_amdgcn_sqrtf(fmaf(im1, im1, re1 * re1)) * E::kMagScale;
+#pragma unroll
+    for (int k = 0; k < TERMS; ++k) {
+      uint32_t word = E::pack(m0, m1);
+      if (F16 && TERMS == 3 && k == 0) word &= E::kLeadMask * 0x10001u;
+      words[k][w] = word;
+      m0 -= E::lo(word);
+      m1 -= E::hi(word);
+      if (TERMS == 3 && k == 0) {
+        m0 *= 1.0f / E::kLowScale;
+        m1 *= 1.0f / E::kLowScale;
+      }
+    }
   }
-  *khi = __builtin_bit_cast(vec_t, hi);
-  *klo = __builtin_bit_cast(vec_t, lo);
+#pragma unroll
+  for (int k = 0; k < TERMS; ++k) out[k] = __builtin_bit_cast(vec_t, words[k]);
 }
 
 }  // namespace kvc

@@ -765,7 +765,7 @@ extern "C" int kvc_score_raw_layout(int dtype, int rope_style, int kv_heads, int
     return fail(KVC_EINVAL, "kvc_score_raw_layout: dtype must be bf16 or fp16");
   if (rope_style != KVC_ROPE_HALF && rope_style != KVC_ROPE_INTERLEAVED)
     return fail(KVC_EINVAL, "kvc_score_raw_layout: unknown rope style %d", rope_style);
-  return mfma_scorer_supported(s, dtype, rope_style) ? KVC_RAW_HEAD_MAJOR : KVC_RAW_TOKEN_MAJOR;
+  return mfma_full_steps(s) && mfma_scorer_supported(s, dtype, rope_style) ? KVC_RAW_HEAD_MAJOR : KVC_RAW_TOKEN_MAJOR;
 }
 
 namespace kvc {

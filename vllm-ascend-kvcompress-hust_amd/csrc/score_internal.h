@@ -88,13 +88,43 @@ inline bool make_shape(ScoreShape* s, int n_layers, int kv_heads, int head_dim, 
 inline size_t weights_floats(const ScoreShape& s) {
   return static_cast<size_t>(s.n_seq) * s.n_layers * s.kv_heads * s.units * 3 * s.qpk * 8;
 }
-// MFMA fragments: per (sequence, layer, KV head), 2*(head_dim/32) linear and
-// 2*(F/32) |k| fragments (16-bit hi/lo), each holding the 16-byte words of the
-// 4*qpk lanes of live query heads; then one float per (sequence, layer, KV
-// head, query head): the column scale the fp16 fragments are divided by.
+// K steps of 32 of the matrix-core scorer: nf pairs (real, imaginary) for the
+// rotary frequencies and one step per 32 pass dims, each rounded up (the last
+// step of a kind may hold dead lanes, see score_mfma.hip).
+struct MfmaSteps {
+  int nk, nf;  // linear / magnitude K steps
+  int terms;   // 16-bit words a float32 weight is split into
+};
+// Every K step full: head_dim and F multiples of 32.
+inline bool mfma_full_steps(const ScoreShape& s) { return s.freq % 32 == 0 && s.pass % 32 == 0; }
+// Head dims 64, 128 and 256 with full steps take two words a weight; the other
+// shapes of up to 128 rotary and 256 dims take three, which keep the whole
+// float32 (score_mfma.hip).  With more rotary dims the vector scorer stays: the
+// matrix cores' sums were further from float64 there (relative error over
+// 20000 tokens 5.4e-8 against 4.8e-8 at 192 rotary dims; at 96 dims 5.1e-8
+// against 5.3e-8, at 128 with 32 rotary 5.6e-8 against 7.9e-8).
+inline bool mfma_two_words(const ScoreShape& s) {
+  return mfma_full_steps(s) && (s.head_dim == 64 || s.head_dim == 128 || s.head_dim == 256) &&
+         (s.freq == 32 || s.freq == 64 || s.freq == 128);
+}
+inline bool mfma_shape(const ScoreShape& s) {
+  return mfma_two_words(s) || (s.head_dim <= 256 && s.rotary_dim <= 128);
+}
+inline MfmaSteps mfma_steps(const ScoreShape& s) {
+  MfmaSteps m;
+  m.nf = (s.freq + 31) / 32;
+  m.nk = 2 * m.nf + (s.pass + 31) / 32;
+  m.terms = mfma_two_words(s) ? 2 : 3;
+  return m;
+}
+// MFMA fragments: per (sequence, layer, KV head), terms*nk linear and terms*nf
+// |k| fragments, each holding the 16-byte words of the 4*qpk lanes of live
+// query heads; then one float per (sequence, layer, KV head, query head): the
+// column scale the fp16 fragments are divided by.
 inline size_t mfma_fragment_only_bytes(const ScoreShape& s) {
-  if (s.head_dim % 32 != 0 || s.freq % 32 != 0) return 0;
-  const size_t frags = 2 * static_cast<size_t>(s.head_dim / 32) + 2 * static_cast<size_t>(s.freq / 32);
+  if (!mfma_shape(s)) return 0;
+  const MfmaSteps m = mfma_steps(s);
+  const size_t frags = static_cast<size_t>(m.terms) * (m.nk + m.nf);
   return static_cast<size_t>(s.n_seq) * s.n_layers * s.kv_heads * frags * 4 * s.qpk * 16;
 }
 inline size_t mfma_fragment_bytes(const ScoreShape& s) {

@@ -379,11 +379,11 @@ __attribute__((amdgpu_waves_per_eu(MaxTiling<NK, ONE_TILE>::kWavesPerSimd))) voi
     }
 #pragma unroll
     for (int q = 0; q < NF; ++q) {
-      vec_t khi, klo;
-      magnitude_operands<F16, IL, NK, NF>(ka, q, &khi, &klo);
-      acc0 = E::mfma(m_hi[q], khi, acc0);
-      acc1 = E::mfma(m_lo[q], khi, acc1);
-      acc0 = E::mfma(m_hi[q], klo, acc0);
+      vec_t km[2];
+      magnitude_words<F16, IL, NK, NF, 2>(ka, q, km);
+      acc0 = E::mfma(m_hi[q], km[0], acc0);
+      acc1 = E::mfma(m_lo[q], km[0], acc1);
+      acc0 = E::mfma(m_hi[q], km[1], acc0);
     }
     return acc0 + acc1;
   };
@@ -812,6 +812,8 @@ MaxKernel pick_max_typed(int nk, int nf, int nch, bool one_tile) {
   return nullptr;
 }
 
+bool max_matrix_shape(const ScoreShape& s) { return mfma_two_words(s); }
+
 }  // namespace
 
 int launch_max_scorer(hipStream_t stream, const ScoreShape& s, int dtype, int n_offsets, const FoldArgs& fa,
@@ -825,7 +827,7 @@ int launch_max_scorer(hipStream_t stream, const ScoreShape& s, int dtype, int n_
   int nch = geo.nch;
   geo.tail_r = geo.tail_qpc = geo.tail_n = 0;
   geo.tail_base = 0;
-  if (!mfma_scorer_supported(s, dtype, fa.interleaved ? KVC_ROPE_INTERLEAVED : KVC_ROPE_HALF)) {
+  if (!max_matrix_shape(s)) {
     const size_t lds = sizeof(float) * (2 * static_cast<size_t>(16 * nch) * s.freq + s.freq + s.pass);
     if (lds > static_cast<size_t>(kValuMaxLds))
       return fail(KVC_EINVAL, "kvc_score_paged_max: %d offsets x %d frequencies exceed the LDS of one workgroup",

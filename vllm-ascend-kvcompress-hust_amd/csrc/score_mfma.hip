@@ -33,6 +33,15 @@
 // scaled by 1/4 before its fp16 split (|k| of fp16 keys can exceed 65504) and
 // the magnitude weights by 4.
 //
+// Two words a weight drop 2^-17 of it.  The shapes that the vector scorer used
+// to take, in float32, keep that: three words a weight and three of |k|, the
+// six products that reach 2^-24.  Their K steps may be partly filled (F not a
+// multiple of 32: 96 or 80 dims, 32 rotary of 128): the real parts, the
+// imaginary parts and the pass dims each start a step of their own, and lanes
+// past a kind's dims hold zero weights.  Scoring 8 sequences of 2048-16384
+// tokens x 4 layers, 8 KV heads of 96 dims, took 150 us on the vector ALUs and
+// 131 here (with its weight fold, which reads along the frequencies, 12 to 6).
+//
 // Work split: a wave owns one KV head and walks 16-token tiles of its
 // workgroup's 256-token span; a workgroup covers hpw KV heads (hpw in {1,2,4}
 // dividing kv_heads) and 4/hpw interleaved tile streams per head.  The next
@@ -49,15 +58,17 @@ namespace {
 constexpr int kMfmaMaxHeadsPerWg = 4;            // hpw
 
 struct MfmaGeometry {
-  int nk, nf;         // linear / magnitude K steps of 32
+  int nk, nf, terms;  // linear / magnitude K steps of 32, words per weight
   int hpw, nsub;      // KV heads per workgroup, tile streams per head
   int head_groups;    // kv_heads / hpw
 };
 
 inline MfmaGeometry geometry(const ScoreShape& s) {
   MfmaGeometry g;
-  g.nk = s.head_dim / 32;
-  g.nf = s.freq / 32;
+  const MfmaSteps m = mfma_steps(s);
+  g.nk = m.nk;
+  g.nf = m.nf;
+  g.terms = m.terms;
   g.hpw = (s.kv_heads % 4 == 0) ? 4 : (s.kv_heads % 2 == 0) ? 2 : 1;
   g.nsub = 4 / g.hpw;
   g.head_groups = s.kv_heads / g.hpw;
@@ -71,43 +82,46 @@ inline MfmaGeometry geometry(const ScoreShape& s) {
 // (g < qpk) are stored, packed as [fragment][kb][g]; the scorer zeroes the
 // B columns of the other lanes, so a wave reads qpk/16 of a full fragment.  Linear weight of head dim d for query head g
 // (tri/scoring.py:70-81, 117-119 folded with the phase means):
-//   d <  F      : sqrt(fss) (qr c - qi s)     (real part, frequency d)
-//   F <= d < 2F : sqrt(fss) (qi c + qr s)     (imaginary part, frequency d-F)
-//   d >= R      : q_pass[d - R]
-// Magnitude weight of frequency f: sqrt(fss) * extra.  Fragments 2j / 2j+1
-// hold the hi / lo bf16 parts of linear step j, 2nk+2q / 2nk+2q+1 those of
-// magnitude step q.
+//   real part of frequency f      : sqrt(fss) (qr c - qi s)
+//   imaginary part of frequency f : sqrt(fss) (qi c + qr s)
+//   pass dim p                    : q_pass[p]
+// Magnitude weight of frequency f: sqrt(fss) * extra.  Fragment terms*j + k
+// holds word k of K step j (linear steps, then magnitude steps): the bf16 of
+// what the words before it leave of the weight.
 // Folded weight of K-step element (step, kb, e) for query head g of
-// (sequence b, layer, KV head): see fold_mfma_kernel.
-__device__ __forceinline__ float folded_weight(const FoldArgs& a, int nk, int b, int layer, int64_t row, int step,
-                                              int kb, int e) {
-  const int head_dim = a.rotary_dim + a.pass;
+// (sequence b, layer, KV head): see fold_mfma_kernel.  Elements past the
+// frequencies or the pass dims (dead lanes of a kind's last step) are zero.
+__device__ __forceinline__ float folded_weight(const FoldArgs& a, int nk, int nf, int b, int layer, int64_t row,
+                                              int step, int kb, int e) {
+  if (step < 2 * nf) {
+    if (a.zero_rotary) return 0.0f;
+    // Half style: steps 0 .. nf-1 real, nf .. 2nf-1 imaginary parts of 32
+    // frequencies each; interleaved: 32 dims of (real, imaginary) pairs.
+    const int i = 32 * step + 8 * kb + e;
+    const bool real = a.interleaved ? (i & 1) == 0 : step < nf;
+    const int f = a.interleaved ? i >> 1 : (step < nf ? i : i - 32 * nf);
+    if (f >= a.freq) return 0.0f;
+    const float* pc = a.phase_cos + b * a.phase_seq_stride + static_cast<int64_t>(layer) * a.freq;
+    const float* ps = a.phase_sin + b * a.phase_seq_stride + static_cast<int64_t>(layer) * a.freq;
+    const int64_t o = row * a.freq + f;
+    const float qr = a.q_real[o], qi = a.q_imag[o], sc = a.scale[o];
+    const float c = pc[f], sn = ps[f];
+    return real ? sc * (qr * c - qi * sn) : sc * (qi * c + qr * sn);
+  }
   if (step < nk) {
-    const int d = 32 * step + 8 * kb + e;
-    if (d >= head_dim) return 0.0f;
-    if (d < 2 * a.freq) {
-      if (a.zero_rotary) return 0.0f;
-      const float* pc = a.phase_cos + b * a.phase_seq_stride + static_cast<int64_t>(layer) * a.freq;
-      const float* ps = a.phase_sin + b * a.phase_seq_stride + static_cast<int64_t>(layer) * a.freq;
-      // Half style: real parts in dims [0, F), imaginary in [F, 2F); interleaved: (2f, 2f+1).
-      const bool real = a.interleaved ? (d & 1) == 0 : d < a.freq;
-      const int f = a.interleaved ? d >> 1 : (d < a.freq ? d : d - a.freq);
-      const int64_t o = row * a.freq + f;
-      const float qr = a.q_real[o], qi = a.q_imag[o], sc = a.scale[o];
-      const float c = pc[f], sn = ps[f];
-      return real ? sc * (qr * c - qi * sn) : sc * (qi * c + qr * sn);
-    }
-    return a.q_pass[row * a.pass + (d - a.rotary_dim)];
+    const int p = 32 * (step - 2 * nf) + 8 * kb + e;
+    return p < a.pass ? a.q_pass[row * a.pass + p] : 0.0f;
   }
   const int q = step - nk;
   const int f = a.interleaved ? 16 * (2 * q + (e >> 2)) + 4 * kb + (e & 3) : 32 * q + 8 * kb + e;
+  if (f >= a.freq) return 0.0f;
   const int64_t o = row * a.freq + f;
   return a.scale[o] * a.extra[o];
 }
 
-__global__ void fold_mfma_kernel(FoldArgs a, int nk, int nf, uint16_t* __restrict__ frags) {
+__global__ void fold_mfma_kernel(FoldArgs a, int nk, int nf, int terms, uint16_t* __restrict__ frags) {
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int n_frag = 2 * nk + 2 * nf;
+  const int n_frag = terms * (nk + nf);
   const int packed = 4 * a.qpk;  // live lanes per fragment
   const int64_t total = static_cast<int64_t>(a.n_seq) * a.n_layers * a.kv_heads * n_frag * packed;
   if (idx >= total) return;
@@ -122,14 +136,18 @@ __global__ void fold_mfma_kernel(FoldArgs a, int nk, int nf, uint16_t* __restric
   const int g = pl % a.qpk;
   const int kb = pl / a.qpk;
   const int64_t row = ((static_cast<int64_t>(layer) * a.kv_heads + head) * a.qpk + g);
-  const bool low = (frag & 1) != 0;
-  const int step = frag >> 1;
+  const int step = frag / terms;
+  const int term = frag - step * terms;
   uint16_t out[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float w = folded_weight(a, nk, b, layer, row, step, kb, e);
-    const uint32_t hi = bf16_bits(w);
-    out[e] = static_cast<uint16_t>(low ? bf16_bits(w - bf16_value(hi)) : hi);
+    float w = folded_weight(a, nk, nf, b, layer, row, step, kb, e);
+    uint32_t word = bf16_bits(w);
+    for (int k = 0; k < term; ++k) {
+      w -= bf16_value(word);
+      word = bf16_bits(w);
+    }
+    out[e] = static_cast<uint16_t>(word);
   }
   uint16_t* dst = frags + (((((static_cast<int64_t>(b) * a.n_layers + layer) * a.kv_heads + head) * n_frag + frag) * packed) + pl) * 8;
 #pragma unroll
@@ -141,9 +159,10 @@ __global__ void fold_mfma_kernel(FoldArgs a, int nk, int nf, uint16_t* __restric
 // its eight weights (magnitude weights times 1/kMagScale), then the column's
 // largest magnitude over the wave picks the power-of-two scale 2^s that brings
 // it to [2^13, 2^14) (s in [-126, 126]; none when it is 0, inf or NaN).  The
-// lane writes fp16(2^s w) and fp16(2^s w - hi) to fragments 2 step and
-// 2 step + 1 in the packed layout of fold_mfma_kernel; lane 0 writes 2^-s.
-__global__ __launch_bounds__(256) void fold_mfma_f16_kernel(FoldArgs a, int nk, int nf, uint16_t* __restrict__ frags,
+// lane writes the fp16 words of 2^s w, each of what the ones before it leave,
+// in the packed layout of fold_mfma_kernel; lane 0 writes 2^-s.
+__global__ __launch_bounds__(256) void fold_mfma_f16_kernel(FoldArgs a, int nk, int nf, int terms,
+                                                            uint16_t* __restrict__ frags,
                                                             float* __restrict__ inv_scale) {
   const int64_t col = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int64_t cols = static_cast<int64_t>(a.n_seq) * a.n_layers * a.kv_heads * a.qpk;
@@ -162,7 +181,7 @@ __global__ __launch_bounds__(256) void fold_mfma_f16_kernel(FoldArgs a, int nk, 
   float big = 0.0f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    w[e] = active ? folded_weight(a, nk, b, layer, row, step, kb, e) : 0.0f;
+    w[e] = active ? folded_weight(a, nk, nf, b, layer, row, step, kb, e) : 0.0f;
     if (step >= nk) w[e] *= 1.0f / MfmaElem<true>::kMagScale;
     big = fmaxf(big, fabsf(w[e]));
   }
@@ -176,24 +195,22 @@ __global__ __launch_bounds__(256) void fold_mfma_f16_kernel(FoldArgs a, int nk, 
     sh = sh < -126 ? -126 : (sh > 126 ? 126 : sh);
   }
   if (active) {
-    const int n_frag = 2 * nk + 2 * nf;
+    const int n_frag = terms * (nk + nf);
     const int packed = 4 * a.qpk;
-    const int64_t base = (((static_cast<int64_t>(b) * a.n_layers + layer) * a.kv_heads + head) * n_frag + 2 * step) * packed +
-                         kb * a.qpk + g;
-    uint16_t hi[8], lo[8];
+    const int64_t base =
+        (((static_cast<int64_t>(b) * a.n_layers + layer) * a.kv_heads + head) * n_frag + terms * step) * packed +
+        kb * a.qpk + g;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float v = ldexpf(w[e], sh);
-      const _Float16 h = static_cast<_Float16>(v);
-      hi[e] = __builtin_bit_cast(uint16_t, h);
-      lo[e] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v - static_cast<float>(h)));
-    }
-    uint16_t* dhi = frags + base * 8;
-    uint16_t* dlo = frags + (base + packed) * 8;
+    for (int e = 0; e < 8; ++e) w[e] = ldexpf(w[e], sh);
+    for (int k = 0; k < terms; ++k) {
+      uint16_t* dst = frags + (base + k * packed) * 8;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      dhi[e] = hi[e];
-      dlo[e] = lo[e];
+      for (int e = 0; e < 8; ++e) {
+        uint16_t bits = __builtin_bit_cast(uint16_t, static_cast<_Float16>(w[e]));
+        if (terms == 3 && k == 0) bits &= MfmaElem<true>::kLeadMask;
+        dst[e] = bits;
+        w[e] -= static_cast<float>(__builtin_bit_cast(_Float16, bits));
+      }
     }
   }
   if (lane == 0) inv_scale[col] = ldexpf(1.0f, -sh);
@@ -201,9 +218,43 @@ __global__ __launch_bounds__(256) void fold_mfma_f16_kernel(FoldArgs a, int nk, 
 
 // --------------------------------------------------------------- score ------
 
-template <int NK, int NF, bool F16, bool IL>
-__global__ __launch_bounds__(kScoreThreads) void score_mfma_kernel(ScoreArgs a, MfmaGeometry geo, int qpk,
-                                                                   const u32x4* __restrict__ frags,
+// The score of one key row for one query head in plain float32, weights folded
+// in place.  Split words turn an infinity into a NaN (inf - inf, inf * 0), so
+// the tokens whose products are not finite are scored again here.
+template <bool F16>
+__device__ __forceinline__ float plain_score(const FoldArgs& a, int b, int layer, int64_t row,
+                                             KVC_GLOBAL const uint16_t* key) {
+  auto at = [&](int d) { return F16 ? fp16_lo(key[d]) : bf16_lo(key[d]); };
+  const float* pc = a.phase_cos + b * a.phase_seq_stride + static_cast<int64_t>(layer) * a.freq;
+  const float* ps = a.phase_sin + b * a.phase_seq_stride + static_cast<int64_t>(layer) * a.freq;
+  float v = 0.0f;
+#pragma unroll 1
+  for (int f = 0; f < a.freq; ++f) {
+    const int64_t o = row * a.freq + f;
+    const float qr = a.q_real[o], qi = a.q_imag[o], sc = a.scale[o], c = pc[f], sn = ps[f];
+    const float re = at(a.interleaved ? 2 * f : f), im = at(a.interleaved ? 2 * f + 1 : a.freq + f);
+    v = fmaf(sc * (qr * c - qi * sn), re, v);
+    v = fmaf(sc * (qi * c + qr * sn), im, v);
+    v = fmaf(sc * a.extra[o], __builtin_amdgcn_sqrtf(fmaf(im, im, re * re)), v);
+  }
+#pragma unroll 1
+  for (int p = 0; p < a.pass; ++p) v = fmaf(a.q_pass[row * a.pass + p], at(a.rotary_dim + p), v);
+  return v;
+}
+
+// 16-token tiles per prefetch group, and the waves per SIMD asked of the
+// compiler: three words a weight in registers leave room for two waves up to
+// nine K steps when a group is one tile from six steps on.
+template <int NK, int NF, bool PART>
+struct MfmaTiling {
+  static constexpr int G = PART && NK >= 6 ? 1 : 2;
+  static constexpr int kWavesPerSimd = PART && 12 * (NK + NF) + 8 * G * NK <= 232 ? 2 : 1;  // 1: no request
+};
+
+template <int NK, int NF, bool F16, bool IL, bool PART>
+__global__ __launch_bounds__(kScoreThreads)
+__attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) void score_mfma_kernel(ScoreArgs a, FoldArgs fold, MfmaGeometry geo,
+                                                                   int qpk, const u32x4* __restrict__ frags,
                                                                    const float* __restrict__ inv_scale) {
   typedef MfmaElem<F16> E;
   typedef typename E::vec vec_t;
@@ -224,7 +275,8 @@ __global__ __launch_bounds__(kScoreThreads) void score_mfma_kernel(ScoreArgs a, 
   const int sub = wave / geo.hpw;
 
   // Folded weight fragments of (sequence, layer, head).
-  constexpr int kFrags = 2 * NK + 2 * NF;
+  constexpr int TERMS = PART ? 3 : 2;
+  constexpr int kFrags = TERMS * (NK + NF);
   // Packed fragments [frag][kb][g < qpk]; lanes of query heads g >= qpk read
   // the kb group's first word (a line the live lanes read anyway) and zero it.
   const int packed = 4 * qpk;
@@ -235,28 +287,54 @@ __global__ __launch_bounds__(kScoreThreads) void score_mfma_kernel(ScoreArgs a, 
     const u32x4 v = fp[f * packed];
     return __builtin_bit_cast(vec_t, live_col ? v : u32x4{0, 0, 0, 0});
   };
-  vec_t w_hi[NK], w_lo[NK], m_hi[NF], m_lo[NF];
+  vec_t w[NK][TERMS], m[NF][TERMS];
   // fp16: the scale that takes this lane's output column back from the
   // scaled weights.
   const float col_scale =
       F16 ? inv_scale[((static_cast<int64_t>(b) * a.n_layers + layer) * a.kv_heads + head) * qpk + (live_col ? r : 0)]
           : 1.0f;
 #pragma unroll
-  for (int j = 0; j < NK; ++j) {
-    w_hi[j] = frag_word(2 * j);
-    w_lo[j] = frag_word(2 * j + 1);
-  }
+  for (int k = 0; k < TERMS; ++k) {
 #pragma unroll
-  for (int q = 0; q < NF; ++q) {
-    m_hi[q] = frag_word(2 * NK + 2 * q);
-    m_lo[q] = frag_word(2 * NK + 2 * q + 1);
+    for (int j = 0; j < NK; ++j) w[j][k] = frag_word(TERMS * j + k);
+#pragma unroll
+    for (int q = 0; q < NF; ++q) m[q][k] = frag_word(TERMS * (NK + q) + k);
   }
 
   KVC_GLOBAL const uint16_t* kbase = gptr_from_int<const uint16_t>(a.k_layer_ptrs[layer]);
   const int64_t* bt = a.block_ids + a.block_offsets[b];
   const int64_t n_blocks = a.block_offsets[b + 1] - a.block_offsets[b];
   const int64_t row_elems = static_cast<int64_t>(a.kv_heads) * a.head_dim;
-  const int64_t lane_off = static_cast<int64_t>(head) * a.head_dim + 8 * kb;
+  const int64_t lane_off = static_cast<int64_t>(head) * a.head_dim;
+  // Element of the head row that this lane's chunk of K step j starts at.
+  // With every step full it is 32*j + 8*kb.  PART: the steps of a kind start
+  // at their own base, and a chunk of the kind's last step that lies past its
+  // dims re-reads the row's first chunk and counts as zeros (bit j of dead).
+  int chunk[NK];
+  unsigned dead = 0;
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    chunk[j] = 32 * j + 8 * kb;
+    if (PART) {
+      int at, end;  // place inside the kind, its dims
+      if (j >= 2 * NF) {
+        at = 32 * (j - 2 * NF) + 8 * kb;
+        end = a.head_dim - a.rotary_dim;
+        chunk[j] = a.rotary_dim + at;
+      } else if (IL) {
+        at = chunk[j];
+        end = a.rotary_dim;
+      } else {
+        at = 32 * (j % NF) + 8 * kb;
+        end = a.freq;
+        chunk[j] = (j < NF ? 0 : a.freq) + at;
+      }
+      if (at >= end) {
+        chunk[j] = 0;
+        dead |= 1u << j;
+      }
+    }
+  }
   const int64_t tok_base = a.token_offsets[b];
   float* raw_out = a.raw + layer * a.raw_layer_stride;
   const int n_mt = (t1 - t0 + 15) / 16;  // 16-token tiles in the span
@@ -286,37 +364,91 @@ __global__ __launch_bounds__(kScoreThreads) void score_mfma_kernel(ScoreArgs a, 
     KVC_GLOBAL const uint16_t* row = pbase + static_cast<int64_t>(t & (kBlockSize - 1)) * row_elems + lane_off;
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
-      const u32x4 v = load_k(reinterpret_cast<KVC_GLOBAL const u32x4*>(row + 32 * j));
-      ka[j] = ok ? v : u32x4{0, 0, 0, 0};
+      const u32x4 v = load_k(reinterpret_cast<KVC_GLOBAL const u32x4*>(row + chunk[j]));
+      ka[j] = ok && !(PART && (dead >> j & 1)) ? v : u32x4{0, 0, 0, 0};
     }
   };
 
   double sum = 0.0, sumsq = 0.0;
   auto score_tile = [&](int mt, const u32x4 (&ka)[NK]) {
-    // Two independent accumulation chains keep consecutive MFMAs apart.
+    // Independent accumulation chains keep consecutive MFMAs apart.
     f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f};
     f32x4 acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (PART) {
+      // Three words a weight and three of |k|: the products that reach 2^-24.
+      // Each step's leading products are a sum of their own and the sums meet
+      // pairwise, so that they round at their own size.
+      constexpr int kChains = NK + NF;
+      f32x4 lead[kChains];
 #pragma unroll
-    for (int j = 0; j < NK; ++j) {
-      const vec_t kv = __builtin_bit_cast(vec_t, ka[j]);
-      if (j & 1) {
-        acc1 = E::mfma(kv, w_hi[j], acc1);
-        acc1 = E::mfma(kv, w_lo[j], acc1);
-      } else {
-        acc0 = E::mfma(kv, w_hi[j], acc0);
-        acc0 = E::mfma(kv, w_lo[j], acc0);
+      for (int c = 0; c < kChains; ++c) lead[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      f32x4 low = {0.0f, 0.0f, 0.0f, 0.0f};  // products with the lower words of |k|
+#pragma unroll
+      for (int j = 0; j < NK; ++j) {
+        const vec_t kv = __builtin_bit_cast(vec_t, ka[j]);
+        lead[j] = E::mfma(kv, w[j][0], lead[j]);
+        acc0 = E::mfma(kv, w[j][1], acc0);
+        acc1 = E::mfma(kv, w[j][2], acc1);
       }
-    }
 #pragma unroll
-    for (int q = 0; q < NF; ++q) {
-      vec_t khi, klo;
-      magnitude_operands<F16, IL, NK, NF>(ka, q, &khi, &klo);
-      acc0 = E::mfma(khi, m_hi[q], acc0);
-      acc1 = E::mfma(khi, m_lo[q], acc1);
-      acc0 = E::mfma(klo, m_hi[q], acc0);
+      for (int q = 0; q < NF; ++q) {
+        vec_t k3[3];
+        magnitude_words<F16, IL, NK, NF, 3>(ka, q, k3);
+        lead[NK + q] = E::mfma(k3[0], m[q][0], lead[NK + q]);
+        acc0 = E::mfma(k3[0], m[q][1], acc0);
+        acc1 = E::mfma(k3[0], m[q][2], acc1);
+        low = E::mfma(k3[1], m[q][0], low);
+        low = E::mfma(k3[1], m[q][1], low);
+        low = E::mfma(k3[2], m[q][0], low);
+      }
+#pragma unroll
+      for (int width = 1; width < kChains; width *= 2)
+#pragma unroll
+        for (int c = 0; c + width < kChains; c += 2 * width) lead[c] += lead[c + width];
+      acc1 += F16 ? low * E::kLowScale : low;
+      acc1 += acc0;
+      acc0 = lead[0];
+    } else {
+#pragma unroll
+      for (int j = 0; j < NK; ++j) {
+        const vec_t kv = __builtin_bit_cast(vec_t, ka[j]);
+        if (j & 1) {
+          acc1 = E::mfma(kv, w[j][0], acc1);
+          acc1 = E::mfma(kv, w[j][1], acc1);
+        } else {
+          acc0 = E::mfma(kv, w[j][0], acc0);
+          acc0 = E::mfma(kv, w[j][1], acc0);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < NF; ++q) {
+        vec_t k2[2];
+        magnitude_words<F16, IL, NK, NF, 2>(ka, q, k2);
+        acc0 = E::mfma(k2[0], m[q][0], acc0);
+        acc1 = E::mfma(k2[0], m[q][1], acc1);
+        acc0 = E::mfma(k2[1], m[q][0], acc0);
+      }
     }
     f32x4 acc = acc0 + acc1;
     if (F16) acc *= col_scale;
+    if constexpr (PART) {
+      unsigned plain = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (writer && t0 + mt * 16 + 4 * kb + i < t1 && !(fabsf(acc[i]) <= 3.402823466e38f)) plain |= 1u << i;
+      if (__any(plain != 0)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int rel = mt * 16 + 4 * kb + i;
+          bool page_ok = false;
+          KVC_GLOBAL const uint16_t* pbase = pages.page(rel < kScoreTile ? rel : 0, &page_ok);
+          if (plain >> i & 1)
+            acc[i] = !page_ok ? 0.0f
+                              : plain_score<F16>(fold, b, layer, (static_cast<int64_t>(layer) * a.kv_heads + head) * qpk + r,
+                                                 pbase + ((t0 + rel) & (kBlockSize - 1)) * row_elems + lane_off);
+        }
+      }
+    }
     // D[4*kb + i][r]: token t0 + 16*mt + 4*kb + i, query head r of this KV head.
     // Scores go to the workgroup's LDS stage (four adjacent tokens per lane,
     // one 16-byte write); global stores wait until the span is done, so the
@@ -338,7 +470,7 @@ __global__ __launch_bounds__(kScoreThreads) void score_mfma_kernel(ScoreArgs a, 
 
   // Tiles sub, sub + nsub, ... in groups of G; the next group's
   // keys are in flight while the current group is scored.
-  constexpr int G = 2;  // 16-token tiles per prefetch group
+  constexpr int G = MfmaTiling<NK, NF, PART>::G;
   u32x4 ka[G][NK], kb2[G][NK];
   const int step = geo.nsub;
   int mt = sub;
@@ -410,24 +542,45 @@ __global__ __launch_bounds__(kScoreThreads) void score_mfma_kernel(ScoreArgs a, 
   }
 }
 
-using MfmaKernel = void (*)(ScoreArgs, MfmaGeometry, int, const u32x4*, const float*);
+using MfmaKernel = void (*)(ScoreArgs, FoldArgs, MfmaGeometry, int, const u32x4*, const float*);
 
 template <bool F16, bool IL>
-MfmaKernel pick_typed(int nk, int nf) {
+MfmaKernel pick_full(int nk, int nf) {
   switch (nk * 16 + nf) {
-    case 2 * 16 + 1: return score_mfma_kernel<2, 1, F16, IL>;
-    case 4 * 16 + 1: return score_mfma_kernel<4, 1, F16, IL>;
-    case 4 * 16 + 2: return score_mfma_kernel<4, 2, F16, IL>;
-    case 8 * 16 + 1: return score_mfma_kernel<8, 1, F16, IL>;
-    case 8 * 16 + 2: return score_mfma_kernel<8, 2, F16, IL>;
-    case 8 * 16 + 4: return score_mfma_kernel<8, 4, F16, IL>;
+    case 2 * 16 + 1: return score_mfma_kernel<2, 1, F16, IL, false>;
+    case 4 * 16 + 1: return score_mfma_kernel<4, 1, F16, IL, false>;
+    case 4 * 16 + 2: return score_mfma_kernel<4, 2, F16, IL, false>;
+    case 8 * 16 + 1: return score_mfma_kernel<8, 1, F16, IL, false>;
+    case 8 * 16 + 2: return score_mfma_kernel<8, 2, F16, IL, false>;
+    case 8 * 16 + 4: return score_mfma_kernel<8, 4, F16, IL, false>;
     default: return nullptr;
   }
 }
-MfmaKernel pick(int nk, int nf, int dtype, int rope_style) {
+// The other shapes: every (nf, pass steps) that up to 128 rotary of up to 256
+// dims give.
+template <bool F16, bool IL, int NF, int NP_MAX>
+MfmaKernel pick_part_pass(int np) {
+  if (np == NP_MAX) return score_mfma_kernel<2 * NF + NP_MAX, NF, F16, IL, true>;
+  if constexpr (NP_MAX > 0) return pick_part_pass<F16, IL, NF, NP_MAX - 1>(np);
+  return nullptr;
+}
+template <bool F16, bool IL>
+MfmaKernel pick_part(int nk, int nf) {
+  switch (nf) {
+    case 1: return pick_part_pass<F16, IL, 1, 8>(nk - 2);
+    case 2: return pick_part_pass<F16, IL, 2, 6>(nk - 4);
+    default: return nullptr;
+  }
+}
+template <bool F16, bool IL>
+MfmaKernel pick_typed(const ScoreShape& s) {
+  const MfmaSteps m = mfma_steps(s);
+  return mfma_two_words(s) ? pick_full<F16, IL>(m.nk, m.nf) : pick_part<F16, IL>(m.nk, m.nf);
+}
+MfmaKernel pick(const ScoreShape& s, int dtype, int rope_style) {
   const bool il = rope_style == KVC_ROPE_INTERLEAVED;
-  if (dtype == KVC_DTYPE_FP16) return il ? pick_typed<true, true>(nk, nf) : pick_typed<true, false>(nk, nf);
-  return il ? pick_typed<false, true>(nk, nf) : pick_typed<false, false>(nk, nf);
+  if (dtype == KVC_DTYPE_FP16) return il ? pick_typed<true, true>(s) : pick_typed<true, false>(s);
+  return il ? pick_typed<false, true>(s) : pick_typed<false, false>(s);
 }
 
 }  // namespace
@@ -435,8 +588,8 @@ MfmaKernel pick(int nk, int nf, int dtype, int rope_style) {
 bool mfma_scorer_supported(const ScoreShape& s, int dtype, int rope_style) {
   if (dtype != KVC_DTYPE_BF16 && dtype != KVC_DTYPE_FP16) return false;
   if (rope_style != KVC_ROPE_HALF && rope_style != KVC_ROPE_INTERLEAVED) return false;
-  if (s.head_dim % 32 != 0 || s.freq % 32 != 0 || s.qpk > kMfmaMaxQpk) return false;
-  return pick(s.head_dim / 32, s.freq / 32, dtype, rope_style) != nullptr;
+  if (!mfma_shape(s) || s.qpk > kMfmaMaxQpk) return false;
+  return pick(s, dtype, rope_style) != nullptr;
 }
 
 int64_t mfma_fold_items(const ScoreShape& s, int dtype) {
@@ -445,7 +598,7 @@ int64_t mfma_fold_items(const ScoreShape& s, int dtype) {
   // fp16: one wave per weight column, four per workgroup; bf16: one thread per
   // live lane of every fragment.
   if (dtype == KVC_DTYPE_FP16) return ceil_div(cols, 4) * 256;
-  return ceil_div(cols * (2 * geo.nk + 2 * geo.nf) * 4, 256) * 256;
+  return ceil_div(cols * geo.terms * (geo.nk + geo.nf) * 4, 256) * 256;
 }
 
 int launch_mfma_fold(hipStream_t stream, const ScoreShape& s, int dtype, const FoldArgs& fa, void* weights) {
@@ -458,9 +611,9 @@ int launch_mfma_fold(hipStream_t stream, const ScoreShape& s, int dtype, const F
   float* inv_scale = reinterpret_cast<float*>(static_cast<char*>(weights) + mfma_fragment_only_bytes(s));
   const unsigned blocks = static_cast<unsigned>(items / 256);
   if (dtype == KVC_DTYPE_FP16) {
-    fold_mfma_f16_kernel<<<blocks, 256, 0, stream>>>(fa, geo.nk, geo.nf, frags, inv_scale);
+    fold_mfma_f16_kernel<<<blocks, 256, 0, stream>>>(fa, geo.nk, geo.nf, geo.terms, frags, inv_scale);
   } else {
-    fold_mfma_kernel<<<blocks, 256, 0, stream>>>(fa, geo.nk, geo.nf, frags);
+    fold_mfma_kernel<<<blocks, 256, 0, stream>>>(fa, geo.nk, geo.nf, geo.terms, frags);
   }
   return launch_status("kvc_score_paged(fold)");
 }
@@ -468,15 +621,17 @@ int launch_mfma_fold(hipStream_t stream, const ScoreShape& s, int dtype, const F
 int launch_mfma_scorer(hipStream_t stream, const ScoreShape& s, int dtype, const FoldArgs& fa, const ScoreArgs& sa,
                        void* weights) {
   const MfmaGeometry geo = geometry(s);
-  MfmaKernel kern = pick(geo.nk, geo.nf, dtype, fa.interleaved ? KVC_ROPE_INTERLEAVED : KVC_ROPE_HALF);
+  MfmaKernel kern = pick(s, dtype, fa.interleaved ? KVC_ROPE_INTERLEAVED : KVC_ROPE_HALF);
   if (!kern) return fail(KVC_EINVAL, "kvc_score_paged: no MFMA scorer for head_dim %d rotary_dim %d", s.head_dim, s.rotary_dim);
   if (int rc = launch_mfma_fold(stream, s, dtype, fa, weights)) return rc;
   const uint16_t* frags = static_cast<const uint16_t*>(weights);
   const float* inv_scale = reinterpret_cast<const float*>(static_cast<const char*>(weights) + mfma_fragment_only_bytes(s));
+  if (s.n_seq > 65535 || s.n_layers > 65535)
+    return fail(KVC_EINVAL, "kvc_score_paged: too many sequences or layers for one launch");
   const int64_t gx = static_cast<int64_t>(s.max_tiles) * geo.head_groups;
   if (gx > 0x7fffffff) return fail(KVC_EINVAL, "kvc_score_paged: grid too large");
   dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(s.n_seq), static_cast<unsigned>(s.n_layers));
-  kern<<<grid, kScoreThreads, 0, stream>>>(sa, geo, s.qpk, reinterpret_cast<const u32x4*>(frags), inv_scale);
+  kern<<<grid, kScoreThreads, 0, stream>>>(sa, fa, geo, s.qpk, reinterpret_cast<const u32x4*>(frags), inv_scale);
   return launch_status("kvc_score_paged");
 }
 
