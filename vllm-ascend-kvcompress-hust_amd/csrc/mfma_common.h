@@ -42,6 +42,10 @@ struct MfmaElem<false> {
   __device__ __forceinline__ static float lo(uint32_t w) { return bf16_lo(w); }
   __device__ __forceinline__ static float hi(uint32_t w) { return bf16_hi(w); }
   __device__ __forceinline__ static uint32_t pack(float a, float b) { return pack_bf16(a, b); }
+  __device__ __forceinline__ static float square_sum(uint32_t w) {
+    const bf16x2 v = __builtin_bit_cast(bf16x2, w);
+    return __builtin_amdgcn_fdot2_f32_bf16(v, v, 0.0f, false);
+  }
 };
 template <>
 struct MfmaElem<true> {
@@ -59,6 +63,10 @@ struct MfmaElem<true> {
   __device__ __forceinline__ static float lo(uint32_t w) { return fp16_lo(w); }
   __device__ __forceinline__ static float hi(uint32_t w) { return fp16_hi(w); }
   __device__ __forceinline__ static uint32_t pack(float a, float b) { return pack_f16(a, b); }
+  __device__ __forceinline__ static float square_sum(uint32_t w) {
+    const f16x2 v = __builtin_bit_cast(f16x2, w);
+    return __builtin_amdgcn_fdot2(v, v, 0.0f, false);
+  }
 };
 
 // K is read once per scoring layer, with plain loads: non-temporal ones
@@ -99,10 +107,19 @@ __device__ __forceinline__ void magnitude_words(const u32x4 (&ka)[NK], int q, ty
       re_w = ka[q][w];
       im_w = ka[q + NF][w];
     }
-    const float re0 = E::lo(re_w), re1 = E::hi(re_w);
-    const float im0 = E::lo(im_w), im1 = E::hi(im_w);
-    float m0 = __builtin_amdgcn_sqrtf(fmaf(im0, im0, re0 * re0)) * E::kMagScale;
-    float m1 = __builtin_amdgcn_sqrtf(fmaf(im1, im1, re1 * re1)) * E::kMagScale;
+    float m0, m1;
+    if constexpr (TERMS == 2) {
+      // Both squares and their sum in one instruction on (real, imaginary) words.
+      const uint32_t p0 = IL ? ka[2 * q + (w >> 1)][(2 * w) & 3] : __builtin_amdgcn_perm(im_w, re_w, 0x05040100);
+      const uint32_t p1 = IL ? ka[2 * q + (w >> 1)][(2 * w + 1) & 3] : __builtin_amdgcn_perm(im_w, re_w, 0x07060302);
+      m0 = __builtin_amdgcn_sqrtf(E::square_sum(p0)) * E::kMagScale;
+      m1 = __builtin_amdgcn_sqrtf(E::square_sum(p1)) * E::kMagScale;
+    } else {
+      const float re0 = E::lo(re_w), re1 = E::hi(re_w);
+      const float im0 = E::lo(im_w), im1 = E::hi(im_w);
+      m0 = __builtin_amdgcn_sqrtf(fmaf(im0, im0, re0 * re0)) * E::kMagScale;
+      m1 = __builtin_amdgcn_sqrtf(fmaf(im1, im1, re1 * re1)) * E::kMagScale;
+    }
 #pragma unroll
     for (int k = 0; k < TERMS; ++k) {
       uint32_t word = E::pack(m0, m1);

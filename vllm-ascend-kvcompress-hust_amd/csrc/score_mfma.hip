@@ -40,7 +40,8 @@
 // imaginary parts and the pass dims each start a step of their own, and lanes
 // past a kind's dims hold zero weights.  Scoring 8 sequences of 2048-16384
 // tokens x 4 layers, 8 KV heads of 96 dims, took 150 us on the vector ALUs and
-// 131 here (with its weight fold, which reads along the frequencies, 12 to 6).
+// 120 here (with its weight fold, which reads along the frequencies, 12 to 6);
+// the vector instructions that split |k| bound it.
 //
 // Work split: a wave owns one KV head and walks 16-token tiles of its
 // workgroup's 256-token span; a workgroup covers hpw KV heads (hpw in {1,2,4}
@@ -48,6 +49,13 @@
 // tile's keys are loaded before the current tile's MFMAs.  Raw scores and the
 // float64 per-tile partial sums have the same layout as the VALU scorer's, so
 // kvc_head_stats and kvc_aggregate are shared.
+//
+// A tile costs 136 vector instructions at 128 dims (208 with masked keys,
+// per-lane addresses, separate squares and sums of the scores in the loop), so
+// the shapes of two words a weight are bound by memory: 16 x 16384 tokens x 6
+// layers of 8 heads x 128 dims read 3.2 GB of keys, 523 us for a bare read in
+// this access pattern, and write 0.25 GB of scores, which stretch the bare
+// read and write to 655 us (the kernel: 668).
 
 #include "mfma_common.h"
 
@@ -268,7 +276,9 @@ __attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) vo
   const int t1 = min(n, t0 + kScoreTile);
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  // The wave's number, and what follows from it (its head, its tiles and their
+  // addresses), is kept in scalar registers.
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15;   // A row (token in tile) / D column (query head)
   const int kb = lane >> 4;  // K block of A/B, row block of D
   const int head = hg * geo.hpw + wave % geo.hpw;
@@ -305,35 +315,33 @@ __attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) vo
   const int64_t* bt = a.block_ids + a.block_offsets[b];
   const int64_t n_blocks = a.block_offsets[b + 1] - a.block_offsets[b];
   const int64_t row_elems = static_cast<int64_t>(a.kv_heads) * a.head_dim;
-  const int64_t lane_off = static_cast<int64_t>(head) * a.head_dim;
-  // Element of the head row that this lane's chunk of K step j starts at.
-  // With every step full it is 32*j + 8*kb.  PART: the steps of a kind start
-  // at their own base, and a chunk of the kind's last step that lies past its
-  // dims re-reads the row's first chunk and counts as zeros (bit j of dead).
-  int chunk[NK];
-  unsigned dead = 0;
+  const int64_t head_off = static_cast<int64_t>(head) * a.head_dim;
+  // Byte offset from a tile's first token to this lane's chunk of K step j.
+  // With every step full it is 64*j past the lane's own.  PART: the steps of a
+  // kind start at their own base, and a chunk of the kind's last step that lies
+  // past its dims re-reads the row's first chunk (its weights are zero).
+  const uint32_t row_off = static_cast<uint32_t>(r) * static_cast<uint32_t>(row_elems) * 2;
+  uint32_t chunk[NK];
 #pragma unroll
   for (int j = 0; j < NK; ++j) {
-    chunk[j] = 32 * j + 8 * kb;
+    int d = 32 * j + 8 * kb;
     if (PART) {
       int at, end;  // place inside the kind, its dims
       if (j >= 2 * NF) {
         at = 32 * (j - 2 * NF) + 8 * kb;
         end = a.head_dim - a.rotary_dim;
-        chunk[j] = a.rotary_dim + at;
+        d = a.rotary_dim + at;
       } else if (IL) {
-        at = chunk[j];
+        at = d;
         end = a.rotary_dim;
       } else {
         at = 32 * (j % NF) + 8 * kb;
         end = a.freq;
-        chunk[j] = (j < NF ? 0 : a.freq) + at;
+        d = (j < NF ? 0 : a.freq) + at;
       }
-      if (at >= end) {
-        chunk[j] = 0;
-        dead |= 1u << j;
-      }
+      if (at >= end) d = 0;
     }
+    chunk[j] = row_off + 2 * static_cast<uint32_t>(d);
   }
   const int64_t tok_base = a.token_offsets[b];
   float* raw_out = a.raw + layer * a.raw_layer_stride;
@@ -354,22 +362,18 @@ __attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) vo
     // compiler wait for every load in flight at the join) and always hit a row
     // inside the pool: tiles the prefetch reaches past the span re-read the
     // span's last tile, which this wave has just read (a cache hit, not HBM
-    // traffic), and unresolved pages read page 0.  Out-of-range rows are zeroed.
-    const int mt_read = mt < n_mt ? mt : n_mt - 1;
-    const int rel = mt_read * 16 + r;
-    const int t = t0 + rel;
+    // traffic), unresolved pages read page 0 and rows past the sequence
+    // whatever their page holds.  A token is a row of every product, so those
+    // rows reach only scores that are set to zero or never stored, and the keys
+    // need no masking; the tile's address is scalar.
+    const int rel = min(mt, n_mt - 1) * 16;
     bool page_ok = false;
-    KVC_GLOBAL const uint16_t* pbase = pages.page(rel, &page_ok);
-    const bool ok = mt < n_mt && t < t1 && page_ok;
-    KVC_GLOBAL const uint16_t* row = pbase + static_cast<int64_t>(t & (kBlockSize - 1)) * row_elems + lane_off;
+    KVC_GLOBAL const char* at = reinterpret_cast<KVC_GLOBAL const char*>(
+        pages.page(rel, &page_ok) + static_cast<int64_t>(rel & (kBlockSize - 1)) * row_elems + head_off);
 #pragma unroll
-    for (int j = 0; j < NK; ++j) {
-      const u32x4 v = load_k(reinterpret_cast<KVC_GLOBAL const u32x4*>(row + chunk[j]));
-      ka[j] = ok && !(PART && (dead >> j & 1)) ? v : u32x4{0, 0, 0, 0};
-    }
+    for (int j = 0; j < NK; ++j) ka[j] = load_k(reinterpret_cast<KVC_GLOBAL const u32x4*>(at + chunk[j]));
   };
 
-  double sum = 0.0, sumsq = 0.0;
   auto score_tile = [&](int mt, const u32x4 (&ka)[NK]) {
     // Independent accumulation chains keep consecutive MFMAs apart.
     f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -431,6 +435,9 @@ __attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) vo
     }
     f32x4 acc = acc0 + acc1;
     if (F16) acc *= col_scale;
+    bool page_ok = false;
+    KVC_GLOBAL const uint16_t* tile_base = pages.page(mt * 16, &page_ok);
+    if (!page_ok) acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (PART) {
       unsigned plain = 0;
 #pragma unroll
@@ -439,33 +446,20 @@ __attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) vo
       if (__any(plain != 0)) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int rel = mt * 16 + 4 * kb + i;
-          bool page_ok = false;
-          KVC_GLOBAL const uint16_t* pbase = pages.page(rel < kScoreTile ? rel : 0, &page_ok);
+          const int in_page = (mt * 16 + 4 * kb + i) & (kBlockSize - 1);
           if (plain >> i & 1)
-            acc[i] = !page_ok ? 0.0f
-                              : plain_score<F16>(fold, b, layer, (static_cast<int64_t>(layer) * a.kv_heads + head) * qpk + r,
-                                                 pbase + ((t0 + rel) & (kBlockSize - 1)) * row_elems + lane_off);
+            acc[i] = plain_score<F16>(fold, b, layer, (static_cast<int64_t>(layer) * a.kv_heads + head) * qpk + r,
+                                      tile_base + in_page * row_elems + head_off);
         }
       }
     }
     // D[4*kb + i][r]: token t0 + 16*mt + 4*kb + i, query head r of this KV head.
     // Scores go to the workgroup's LDS stage (four adjacent tokens per lane,
-    // one 16-byte write); global stores wait until the span is done, so the
-    // loop's waits cover only K loads (vector memory operations retire in
-    // issue order, and a store in the loop would hold up the next tile).
-    const int rel = mt * 16 + 4 * kb;
-    if (writer && mt < n_mt) {
-      *reinterpret_cast<f32x4*>(stage_row + rel) = acc;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (t0 + rel + i < t1) {
-          const double dv = static_cast<double>(acc[i]);
-          sum += dv;
-          sumsq = fma(dv, dv, sumsq);
-        }
-      }
-    }
+    // one 16-byte write); global stores and the head sums wait until the span
+    // is done: the loop's waits then cover only K loads (vector memory
+    // operations retire in issue order, and a store in the loop would hold up
+    // the next tile), and the sums use every lane instead of qpk of 16.
+    if (writer) *reinterpret_cast<f32x4*>(stage_row + mt * 16 + 4 * kb) = acc;
   };
 
   // Tiles sub, sub + nsub, ... in groups of G; the next group's
@@ -480,33 +474,30 @@ __attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) vo
 #pragma unroll
     for (int g = 0; g < G; ++g) load_tile(mt + (G + g) * step, kb2[g]);
 #pragma unroll
-    for (int g = 0; g < G; ++g) score_tile(mt + g * step, ka[g]);
+    for (int g = 0; g < G; ++g)
+      if (mt + g * step < n_mt) score_tile(mt + g * step, ka[g]);
     if (mt + G * step >= n_mt) break;
 #pragma unroll
     for (int g = 0; g < G; ++g) load_tile(mt + (2 * G + g) * step, ka[g]);
 #pragma unroll
-    for (int g = 0; g < G; ++g) score_tile(mt + (G + g) * step, kb2[g]);
+    for (int g = 0; g < G; ++g)
+      if (mt + (G + g) * step < n_mt) score_tile(mt + (G + g) * step, kb2[g]);
   }
 
-  // Per query head: sum the lanes of the four row blocks and the tile streams.
-  __shared__ double red[2][kScoreThreads];
-  red[0][threadIdx.x] = sum;
-  red[1][threadIdx.x] = sumsq;
   __syncthreads();
 
   // Stage -> raw scores: row (hl, g) holds query head (hg*hpw + hl)*qpk + g
-  // for the span's tokens.  Head-major scores are contiguous per row (16-byte
-  // stores where aligned); token-major ones are contiguous across the rows.
-  // Non-temporal 16-byte stores measured 1-2% faster scoring than plain ones
-  // (the scores are read once more, by the aggregation pass).
+  // for the span's tokens.  Head-major scores are contiguous per row (a wave a
+  // row, 16-byte stores where aligned); token-major ones are contiguous across
+  // the rows.  Non-temporal 16-byte stores measured 1-2% faster scoring than
+  // plain ones (the scores are read once more, by the aggregation pass).
   const int span = t1 - t0;
   const int rows = geo.hpw * qpk;
   const int q_first = hg * geo.hpw * qpk;
   if (a.raw_token_stride == 1) {
-    const int span4 = (span + 3) >> 2;
-    for (int idx = threadIdx.x; idx < rows * span4; idx += kScoreThreads) {
-      const int row = idx / span4;
-      const int c = (idx - row * span4) << 2;
+    static_assert(kScoreTile == 4 * 64, "a lane stores four tokens of a row");
+    const int c = lane << 2;
+    for (int row = wave; row < rows; row += kScoreThreads / 64) {
       const float* src = stage + row * kStageStride + c;
       float* dst = raw_out + (tok_base + t0 + c) + static_cast<int64_t>(q_first + row) * a.raw_head_stride;
       if (c + 3 < span && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
@@ -516,27 +507,52 @@ __attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) vo
       }
     }
   } else {
-    for (int idx = threadIdx.x; idx < rows * span; idx += kScoreThreads) {
-      const int t = idx / rows;
-      const int row = idx - t * rows;
+    int t = threadIdx.x / rows, row = threadIdx.x - t * rows;
+    const int dt = kScoreThreads / rows, drow = kScoreThreads - dt * rows;
+    while (t < span) {
       raw_out[(tok_base + t0 + t) * a.raw_token_stride + static_cast<int64_t>(q_first + row) * a.raw_head_stride] =
           stage[row * kStageStride + t];
-    }
-  }
-  const int heads_here = geo.hpw * qpk;
-  for (int i = threadIdx.x; i < heads_here; i += kScoreThreads) {
-    const int hl = i / qpk, g = i - hl * qpk;
-    double s0 = 0.0, s1 = 0.0;
-    for (int sb = 0; sb < geo.nsub; ++sb) {
-      const int w = sb * geo.hpw + hl;
-      for (int k = 0; k < 4; ++k) {
-        s0 += red[0][w * 64 + k * 16 + g];
-        s1 += red[1][w * 64 + k * 16 + g];
+      t += dt;
+      row += drow;
+      if (row >= rows) {
+        row -= rows;
+        ++t;
       }
     }
-    const int q = (hg * geo.hpw + hl) * qpk + g;
+  }
+
+  // Per query head, the float64 sums of the span's scores and their squares:
+  // `per` threads a row take every per-th four tokens, then one adds them up.
+  constexpr int kSumThreads = 16;
+  __shared__ double red[2][kScoreThreads];
+  const int per = min(kSumThreads, kScoreThreads / rows);
+  {
+    const int row = threadIdx.x / per, part = threadIdx.x - row * per;
+    double sum = 0.0, sumsq = 0.0;
+    if (row < rows) {
+      for (int c = part * 4; c < span; c += per * 4) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(stage + row * kStageStride + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const double dv = static_cast<double>(c + i < span ? v[i] : 0.0f);
+          sum += dv;
+          sumsq = fma(dv, dv, sumsq);
+        }
+      }
+    }
+    red[0][threadIdx.x] = sum;
+    red[1][threadIdx.x] = sumsq;
+  }
+  __syncthreads();
+  if (static_cast<int>(threadIdx.x) < rows) {
+    double s0 = 0.0, s1 = 0.0;
+    for (int k = 0; k < per; ++k) {
+      s0 += red[0][threadIdx.x * per + k];
+      s1 += red[1][threadIdx.x * per + k];
+    }
     const int n_heads = a.kv_heads * qpk;
-    double* dst = a.partials + (((static_cast<int64_t>(layer) * a.n_seq + b) * a.max_tiles + tile) * n_heads + q) * 2;
+    double* dst = a.partials +
+                  (((static_cast<int64_t>(layer) * a.n_seq + b) * a.max_tiles + tile) * n_heads + q_first + threadIdx.x) * 2;
     dst[0] = s0;
     dst[1] = s1;
   }
