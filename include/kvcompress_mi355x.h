@@ -383,7 +383,8 @@ int kvc_shift_lengths(kvc_stream_t stream, void* seq_lens, int elem_bytes, const
  * token_stride >= heads*head_dim, e.g. 2*heads*head_dim for a q_proj whose
  * output carries a gate after Q).  kvc_qstats_accumulate adds the tokens'
  * partial sums into `state` (kvc_qstats_state_bytes bytes, zeroed by the
- * caller before the first call); kvc_qstats_finish writes the totals over
+ * caller before the first call, or begun by kvc_qstats_start, which replaces
+ * what the state holds by these tokens' sums); kvc_qstats_finish writes the totals over
  * every call so far.  With F = rotary_dim/2 and P = head_dim - rotary_dim, for
  * h < heads, f < F, p < P:
  *   real_sum[h*F + f] = sum_t q(t, h, f)
@@ -397,6 +398,9 @@ size_t kvc_qstats_state_bytes(int heads, int head_dim, int rotary_dim);
 int kvc_qstats_accumulate(kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens,
                           int64_t token_stride, int heads, int head_dim, int rotary_dim, void* state,
                           size_t state_bytes);
+int kvc_qstats_start(kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens,
+                     int64_t token_stride, int heads, int head_dim, int rotary_dim, void* state,
+                     size_t state_bytes);
 int kvc_qstats_finish(kvc_stream_t stream, int heads, int head_dim, int rotary_dim, const void* state,
                       double* real_sum, double* imag_sum, double* abs_sum, double* pass_sum);
 

@@ -317,3 +317,27 @@ def test_generator_end_to_end_on_a_local_qwen2_checkpoint(hip_device, tmp_path: 
             torch.testing.assert_close(getattr(got, key), want[key], rtol=1e-4, atol=1e-5)
         torch.testing.assert_close(got.inv_freq, inv_freq)
         assert torch.equal(got.freq_scale_sq, torch.ones(1, 16))
+
+
+@pytest.mark.parametrize("heads, head_dim, rotary, tokens", [(1, 16, 6, 33), (40, 128, 128, 2049), (90, 128, 64, 31), (2, 64, 64, 5000)])
+def test_qstats_first_tokens_replace_the_state(hip_device, heads, head_dim, rotary, tokens) -> None:
+    """The first call stores every row of an uncleared state (32 to 128 rows by
+    the shape's units), later calls add to it."""
+    calibration = _calib()
+    from kvcompress_mi355x import _native
+
+    g = torch.Generator().manual_seed(tokens)
+    q = torch.randn(tokens + 5, heads * head_dim, generator=g).to(torch.bfloat16)
+    state_bytes = int(_native.load().kvc_qstats_state_bytes(heads, head_dim, rotary))
+    acc = calibration.LayerAccumulator()
+    dev = q.to(hip_device)
+    dirty = torch.full((state_bytes,), 255, dtype=torch.uint8, device=hip_device)  # NaN sums, freed for the state
+    del dirty
+    acc.add(dev[:tokens], heads, head_dim, rotary)
+    acc.add(dev[tokens:], heads, head_dim, rotary)
+    acc.add(dev[:0], heads, head_dim, rotary)
+    torch.cuda.synchronize()
+    _check_sums(acc, q.float().reshape(-1, heads, head_dim).numpy(), rotary)
+    empty = calibration.LayerAccumulator()
+    empty.add(dev[:0], heads, head_dim, rotary)
+    assert float(empty.abs_sum.abs().max()) == 0.0

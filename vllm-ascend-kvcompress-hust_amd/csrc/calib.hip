@@ -18,12 +18,22 @@
 // addresses allow vector loads, else 1).  The accumulation grid is (blocks of
 // 64 lanes) x (token splits): a workgroup of 4 waves covers 64*V units over
 // one split's tokens, wave w summing the split's tokens t = w (mod 4) with 8
-// tokens' loads in flight; the four wave partials are combined in wave order
-// in LDS and added into the caller's state at [split][unit][3].  Every state
+// tokens' loads in flight; the wave partials are combined in wave order in LDS
+// and added into the caller's state at [split][unit][3] (the first call of a
+// state stores instead, all rows, so nothing has to be cleared).  Every state
 // entry has one owner per launch, so calls add up in call order, and the
-// finish kernel sums a unit's splits in split order: repeated runs give
-// identical sums.  Accumulation reads the projections once (bound: HBM, 2-4
-// bytes per element); the state is 128 splits x units x 24 bytes.
+// finish kernel sums a unit's splits in a fixed order: repeated runs give
+// identical sums.
+//
+// Accumulation reads the projections once (HBM, 2-4 bytes per element), but
+// the state is written (and after the first call read) by every call and read
+// by the finish, so its rows are as few as fill the chip: about 760
+// workgroups, three a CU (77 rows for 40 heads of 128 dims: 4.7 MB against
+// 42 MB of 4096 projections).  Of that shape a layer's clear, accumulation and
+// finish took 6.9 + 12.8 + 7.4 us with 128 rows and a cleared state; now
+// 13.1 + 5.0.  640 and 1020 workgroups measured 13.9 and 14.3 us, eight waves
+// a workgroup 14.6; without any store it is 12.0, the latency of one round of
+// loads over a chip that starts and drains.
 
 #include "kvc_common.h"
 
@@ -33,14 +43,15 @@ namespace {
 constexpr int kQsWaves = 4;
 constexpr int kQsThreads = kQsWaves * 64;
 constexpr int kQsUnroll = 8;
-constexpr int kQsSplits = 128;         // state rows
+constexpr int kQsMinRows = 32, kQsMaxRows = 128;  // state rows
 constexpr int kQsMinSplitTokens = 32;  // tokens per split, at least
 
 struct QStatsArgs {
   const void* q;
   int64_t n_tokens, token_stride, split_tokens;
   int heads, head_dim, freq, pass;
-  double* state;  // [kQsSplits][units][3]
+  int store;      // 1: replace the state's rows instead of adding to them
+  double* state;  // [rows][units][3]
 };
 
 inline int64_t qstats_units(int heads, int head_dim, int rotary_dim) {
@@ -60,6 +71,12 @@ __device__ __forceinline__ float widen<_Float16>(_Float16 v) {
 template <>
 __device__ __forceinline__ float widen<float>(float v) {
   return v;
+}
+
+// State rows, the most splits a call makes: 64*4 units x 760 rows' worth.
+inline int qstats_rows(int64_t units) {
+  const int64_t rows = ceil_div(760 * 256, units);
+  return static_cast<int>(rows < kQsMinRows ? kQsMinRows : (rows > kQsMaxRows ? kQsMaxRows : rows));
 }
 
 // V consecutive elements widened to float32, read with one load of
@@ -82,11 +99,11 @@ __global__ __launch_bounds__(kQsThreads) void qstats_accumulate_kernel(QStatsArg
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int fg = a.freq / V, pg = a.pass / V;  // unit groups per head
-  const int64_t groups = static_cast<int64_t>(a.heads) * (fg + pg);
-  const int64_t group = static_cast<int64_t>(blockIdx.x) * 64 + lane;
+  const int groups = a.heads * (fg + pg);  // fits (launch_accumulate)
+  const int group = static_cast<int>(blockIdx.x) * 64 + lane;
   const bool live = group < groups;
-  const int h = live ? static_cast<int>(group / (fg + pg)) : 0;
-  const int c = live ? static_cast<int>(group - static_cast<int64_t>(h) * (fg + pg)) : 0;
+  const int h = live ? group / (fg + pg) : 0;
+  const int c = live ? group - h * (fg + pg) : 0;
   const bool pair = c < fg;
   // Row offsets: real dims f0.., imaginary F+f0.. for frequencies; R+p0.. for pass dims.
   const int64_t d0 = static_cast<int64_t>(h) * a.head_dim + (pair ? c * V : 2 * a.freq + (c - fg) * V);
@@ -129,34 +146,49 @@ __global__ __launch_bounds__(kQsThreads) void qstats_accumulate_kernel(QStatsArg
     red[wave][3 * e + 2][lane] = s_abs[e];
   }
   __syncthreads();
-  if (wave != 0 || !live) return;
+  // Entry k of lane l: statistic k%3 of unit unit0(l) + k/3, contiguous in the state.
   const int64_t units = static_cast<int64_t>(a.heads) * (a.freq + a.pass);
-  // Unit index of element e: frequencies h*(F+P) + f, pass dims h*(F+P) + F + p.
-  const int64_t unit0 = static_cast<int64_t>(h) * (a.freq + a.pass) + (pair ? c * V : a.freq + (c - fg) * V);
-  double* st = a.state + (static_cast<int64_t>(blockIdx.y) * units + unit0) * 3;
+  for (int i = threadIdx.x; i < 64 * 3 * V; i += kQsThreads) {
+    const int l = i / (3 * V), k = i - l * (3 * V);
+    const int grp = static_cast<int>(blockIdx.x) * 64 + l;
+    if (grp >= groups) continue;
+    const int hh = grp / (fg + pg), cc = grp - hh * (fg + pg);
+    // Frequencies are units h*(F+P) + f, pass dims h*(F+P) + F + p.
+    const int64_t unit0 = static_cast<int64_t>(hh) * (a.freq + a.pass) + (cc < fg ? cc * V : a.freq + (cc - fg) * V);
+    double sum = 0.0;
 #pragma unroll
-  for (int k = 0; k < 3 * V; ++k) {
-    double r = 0.0;
-#pragma unroll
-    for (int w = 0; w < kQsWaves; ++w) r += red[w][k][lane];
-    st[k] += r;  // element e, statistic k%3 at unit0 + e: [e][3] is contiguous
+    for (int w = 0; w < kQsWaves; ++w) sum += red[w][k][l];
+    double* st = a.state + (static_cast<int64_t>(blockIdx.y) * units + unit0) * 3 + k;
+    *st = a.store ? sum : *st + sum;
   }
 }
 
-__global__ void qstats_finish_kernel(const double* __restrict__ state, int64_t units, int heads, int freq, int pass,
-                                     double* __restrict__ real_sum, double* __restrict__ imag_sum,
-                                     double* __restrict__ abs_sum, double* __restrict__ pass_sum) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;  // unit*3 + statistic
-  if (idx >= units * 3) return;
-  // Splits in order, 16 loads in flight at a time.
+// kQsFinishParts threads an entry, each summing a quarter of the rows (in
+// order, 32 loads in flight), the quarters added in order.
+constexpr int kQsFinishParts = 4;
+__global__ __launch_bounds__(256) void qstats_finish_kernel(const double* __restrict__ state, int rows, int64_t units,
+                                                            int heads, int freq, int pass, double* __restrict__ real_sum,
+                                                            double* __restrict__ imag_sum, double* __restrict__ abs_sum,
+                                                            double* __restrict__ pass_sum) {
+  __shared__ double quarter[kQsFinishParts][64];
+  const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 64 + lane;  // unit*3 + statistic
+  const bool live = idx < units * 3;
+  const int per = (rows + kQsFinishParts - 1) / kQsFinishParts;
+  const int end = min(rows, (part + 1) * per);
   double sum = 0.0;
-  for (int s0 = 0; s0 < kQsSplits; s0 += 16) {
-    double r[16];
+  for (int s0 = part * per; live && s0 < end; s0 += 32) {
+    double r[32];
 #pragma unroll
-    for (int s = 0; s < 16; ++s) r[s] = state[static_cast<int64_t>(s0 + s) * units * 3 + idx];
+    for (int s = 0; s < 32; ++s) r[s] = state[static_cast<int64_t>(min(s0 + s, end - 1)) * units * 3 + idx];
 #pragma unroll
-    for (int s = 0; s < 16; ++s) sum += r[s];
+    for (int s = 0; s < 32; ++s)
+      if (s0 + s < end) sum += r[s];
   }
+  quarter[part][lane] = sum;
+  __syncthreads();
+  if (part != 0 || !live) return;
+  for (int p = 1; p < kQsFinishParts; ++p) sum += quarter[p][lane];
   const int64_t unit = idx / 3;
   const int k = static_cast<int>(idx - unit * 3);
   const int h = static_cast<int>(unit / (freq + pass));
@@ -180,12 +212,15 @@ using namespace kvc;
 
 extern "C" size_t kvc_qstats_state_bytes(int heads, int head_dim, int rotary_dim) {
   if (!shape_ok(heads, head_dim, rotary_dim)) return 0;
-  return static_cast<size_t>(kQsSplits) * qstats_units(heads, head_dim, rotary_dim) * 3 * sizeof(double);
+  const int64_t units = qstats_units(heads, head_dim, rotary_dim);
+  return static_cast<size_t>(qstats_rows(units)) * units * 3 * sizeof(double);
 }
 
-extern "C" int kvc_qstats_accumulate(kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens,
-                                     int64_t token_stride, int heads, int head_dim, int rotary_dim, void* state,
-                                     size_t state_bytes) {
+namespace kvc {
+namespace {
+
+int launch_accumulate(kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens, int64_t token_stride, int heads,
+                      int head_dim, int rotary_dim, void* state, size_t state_bytes, bool store) {
   if (dtype != KVC_DTYPE_BF16 && dtype != KVC_DTYPE_FP16 && dtype != KVC_DTYPE_FP32)
     return fail(KVC_EINVAL, "kvc_qstats_accumulate: unknown dtype %d", dtype);
   if (heads <= 0 || head_dim <= 0 || n_tokens < 0) return fail(KVC_EINVAL, "kvc_qstats_accumulate: bad sizes");
@@ -196,8 +231,8 @@ extern "C" int kvc_qstats_accumulate(kvc_stream_t stream, int dtype, const void*
   const size_t need = kvc_qstats_state_bytes(heads, head_dim, rotary_dim);
   if (!state || state_bytes < need)
     return fail(KVC_EINVAL, "kvc_qstats_accumulate: state of %zu bytes needed", need);
-  if (n_tokens == 0) return 0;
-  if (!q) return fail(KVC_EINVAL, "kvc_qstats_accumulate: null input");
+  if (n_tokens == 0 && !store) return 0;
+  if (!q && n_tokens > 0) return fail(KVC_EINVAL, "kvc_qstats_accumulate: null input");
   QStatsArgs a;
   a.q = q;
   a.n_tokens = n_tokens;
@@ -207,10 +242,14 @@ extern "C" int kvc_qstats_accumulate(kvc_stream_t stream, int dtype, const void*
   a.freq = rotary_dim / 2;
   a.pass = head_dim - rotary_dim;
   a.state = static_cast<double*>(state);
+  a.store = store ? 1 : 0;
+  const int rows = qstats_rows(qstats_units(heads, head_dim, rotary_dim));
   int64_t splits = ceil_div(n_tokens, kQsMinSplitTokens);
-  if (splits > kQsSplits) splits = kQsSplits;
+  if (splits > rows) splits = rows;
+  if (splits < 1) splits = 1;
   a.split_tokens = ceil_div(n_tokens, splits);
-  splits = ceil_div(n_tokens, a.split_tokens);
+  // A storing call covers every row; those past the tokens store zeros.
+  splits = store ? rows : ceil_div(n_tokens, a.split_tokens);
 
   const int esize = dtype == KVC_DTYPE_FP32 ? 4 : 2;
   // Four-wide loads need every vector start aligned: frequency and pass
@@ -220,7 +259,7 @@ extern "C" int kvc_qstats_accumulate(kvc_stream_t stream, int dtype, const void*
   const int v = wide ? 4 : 1;
   const int64_t groups = static_cast<int64_t>(heads) * (a.freq / v + a.pass / v);
   const int64_t blocks = ceil_div(groups, 64);
-  if (blocks > 0x7fffffff) return fail(KVC_EINVAL, "kvc_qstats_accumulate: too many heads");
+  if (groups > 0x7fffffff - 64) return fail(KVC_EINVAL, "kvc_qstats_accumulate: too many heads");
   const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(splits));
   hipStream_t st = as_stream(stream);
   switch (dtype * 2 + (wide ? 1 : 0)) {
@@ -234,6 +273,22 @@ extern "C" int kvc_qstats_accumulate(kvc_stream_t stream, int dtype, const void*
   return launch_status("kvc_qstats_accumulate");
 }
 
+}  // namespace
+}  // namespace kvc
+
+extern "C" int kvc_qstats_accumulate(kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens,
+                                     int64_t token_stride, int heads, int head_dim, int rotary_dim, void* state,
+                                     size_t state_bytes) {
+  return launch_accumulate(stream, dtype, q, n_tokens, token_stride, heads, head_dim, rotary_dim, state, state_bytes,
+                           false);
+}
+
+extern "C" int kvc_qstats_start(kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens, int64_t token_stride,
+                                int heads, int head_dim, int rotary_dim, void* state, size_t state_bytes) {
+  return launch_accumulate(stream, dtype, q, n_tokens, token_stride, heads, head_dim, rotary_dim, state, state_bytes,
+                           true);
+}
+
 extern "C" int kvc_qstats_finish(kvc_stream_t stream, int heads, int head_dim, int rotary_dim, const void* state,
                                  double* real_sum, double* imag_sum, double* abs_sum, double* pass_sum) {
   if (!shape_ok(heads, head_dim, rotary_dim))
@@ -242,7 +297,7 @@ extern "C" int kvc_qstats_finish(kvc_stream_t stream, int heads, int head_dim, i
   if (!state || !real_sum || !imag_sum || !abs_sum || (pass > 0 && !pass_sum))
     return fail(KVC_EINVAL, "kvc_qstats_finish: null pointer");
   const int64_t units = qstats_units(heads, head_dim, rotary_dim);
-  qstats_finish_kernel<<<static_cast<unsigned>(ceil_div(units * 3, 256)), 256, 0, as_stream(stream)>>>(
-      static_cast<const double*>(state), units, heads, rotary_dim / 2, pass, real_sum, imag_sum, abs_sum, pass_sum);
+  qstats_finish_kernel<<<static_cast<unsigned>(ceil_div(units * 3, 64)), 256, 0, as_stream(stream)>>>(
+      static_cast<const double*>(state), qstats_rows(units), units, heads, rotary_dim / 2, pass, real_sum, imag_sum, abs_sum, pass_sum);
   return launch_status("kvc_qstats_finish");
 }

@@ -339,14 +339,18 @@ class LayerAccumulator:
         if rows.stride(1) != 1:
             rows = rows.contiguous()
         lib = _native.load()
-        if self._state is None:
+        n_tokens = int(rows.shape[0])
+        state = self._state
+        if state is None:
             state_bytes = int(lib.kvc_qstats_state_bytes(heads, head_dim, rotary_dim))
             if state_bytes == 0:
                 raise ValueError("rotary_dim must be positive, even and no larger than head_dim")
-            self._state = torch.zeros(state_bytes, dtype=torch.uint8, device=device)
-        n_tokens = int(rows.shape[0])
+            # The first tokens' launch stores every row of the state.
+            make = torch.empty if n_tokens else torch.zeros
+            state = make(state_bytes, dtype=torch.uint8, device=device)
         if n_tokens:
-            rc = lib.kvc_qstats_accumulate(
+            entry = "kvc_qstats_start" if self._state is None else "kvc_qstats_accumulate"
+            rc = getattr(lib, entry)(
                 torch.cuda.current_stream(device).cuda_stream,
                 _kernel_dtype(rows.dtype),
                 int(rows.data_ptr()),
@@ -355,11 +359,12 @@ class LayerAccumulator:
                 heads,
                 head_dim,
                 rotary_dim,
-                int(self._state.data_ptr()),
-                int(self._state.numel()),
+                int(state.data_ptr()),
+                int(state.numel()),
             )
-            _native.check(rc, "kvc_qstats_accumulate")
+            _native.check(rc, entry)
             self._stale = True
+        self._state = state
         self.count += n_tokens
 
     def _totals(self) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor | None] | None:
