@@ -358,3 +358,35 @@ def test_compaction_order_choice_and_forced_order(hip_device, order) -> None:
     ipipe.select_step(ibatch)
     with pytest.raises(ValueError, match="repeat_in_place"):
         ipipe.settle_compaction(ibatch)
+
+
+@pytest.mark.parametrize("n_seq", [1, 2, 5])
+def test_batch_descriptors_of_one_copy(hip_device, n_seq) -> None:
+    """Every descriptor of a batch, odd and even sequence counts, built behind
+    queued work on a side stream, with the pinned block reused in between; and
+    no capture of the copy."""
+    from kvcompress_mi355x.methods.triattention.pipeline import Batch
+
+    lens = [300 + 1000 * i for i in range(n_seq)]
+    starts = [(1 << 33) + i for i in range(n_seq)]
+    tables = [torch.arange(-(-n // 128)) + 7 * i for i, n in enumerate(lens)]
+    stream = torch.cuda.Stream()
+    batches = []
+    with torch.cuda.stream(stream):
+        busy = torch.randn(2048, 2048, device=hip_device)
+        for _ in range(20):
+            busy = busy @ busy / 64.0
+            batches.append(Batch.build(hip_device, lens, starts, tables, [t[:2] for t in tables], budget=200))
+    stream.synchronize()
+    offsets = torch.tensor([0] + lens).cumsum(0)
+    counts = torch.tensor([0] + [t.numel() for t in tables]).cumsum(0)
+    for b in batches:
+        assert b.seq_lens.dtype == torch.int32 and b.seq_lens.cpu().tolist() == lens
+        assert b.token_offsets.cpu().tolist() == offsets.tolist() and b.round_starts.cpu().tolist() == starts
+        assert b.src_offsets.cpu().tolist() == counts.tolist() and b.dst_offsets.cpu().tolist() == [2 * i for i in range(n_seq + 1)]
+        assert b.src_ids.cpu().tolist() == torch.cat(tables).tolist()
+    graph = torch.cuda.CUDAGraph()
+    device_tables = [t.to(hip_device) for t in tables]
+    with pytest.raises(RuntimeError, match="capture"):
+        with torch.cuda.graph(graph, stream=stream):
+            Batch.build(hip_device, lens, starts, device_tables)

@@ -61,6 +61,7 @@ import torch
 
 from . import __version__, _native
 from .methods.base import ModelShape
+from .methods.triattention._device import stream_handle
 from .methods.triattention.config import TriAttentionConfig
 from .methods.triattention.stats import SUPPORTED_MODEL_TYPES, CalibrationStats
 from .model import model_shape_from_config
@@ -329,7 +330,8 @@ class LayerAccumulator:
         elif self._shape != (heads, head_dim, rotary_dim):
             raise RuntimeError("a layer accumulator cannot change its attention shape")
         if self._device is None:
-            self._device = _hip_device(self.device if self.device is not None else projected.device)
+            on_device = self.device is None and projected.is_cuda
+            self._device = projected.device if on_device else _hip_device(self.device if self.device is not None else projected.device)
         device = self._device
         rows = projected.detach().reshape(-1, expected)
         if rows.dtype not in (torch.bfloat16, torch.float16, torch.float32):
@@ -351,7 +353,7 @@ class LayerAccumulator:
         if n_tokens:
             entry = "kvc_qstats_start" if self._state is None else "kvc_qstats_accumulate"
             rc = getattr(lib, entry)(
-                torch.cuda.current_stream(device).cuda_stream,
+                stream_handle(device),
                 _kernel_dtype(rows.dtype),
                 int(rows.data_ptr()),
                 n_tokens,
@@ -377,7 +379,7 @@ class LayerAccumulator:
             sums = (empty(freq), empty(freq), empty(freq), empty(pass_dim) if pass_dim else None)
             _native.call(
                 "kvc_qstats_finish",
-                torch.cuda.current_stream(self._device).cuda_stream,
+                stream_handle(self._device),
                 heads,
                 head_dim,
                 rotary_dim,

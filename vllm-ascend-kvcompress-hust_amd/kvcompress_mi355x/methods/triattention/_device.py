@@ -30,7 +30,10 @@ def require_contiguous(tensor: torch.Tensor, name: str) -> None:
 
 
 def stream_handle(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream's HIP handle, without building a Stream object for
+    each of a step's launches."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(tensor: torch.Tensor | None) -> int | None:
@@ -86,8 +89,8 @@ def pointer_table(tensors: list[torch.Tensor], device: torch.device) -> torch.Te
     return torch.tensor(signed, dtype=torch.int64, device=device)
 
 
-def ragged(rows: list[torch.Tensor | list[int] | tuple[int, ...]], device: torch.device) -> tuple[torch.Tensor, torch.Tensor, list[int]]:
-    """Concatenate int64 rows; return (offsets [n+1], flat ids, host lengths)."""
+def ragged_ids(rows: list[torch.Tensor | list[int] | tuple[int, ...]], device: torch.device) -> tuple[torch.Tensor, list[int]]:
+    """Concatenate int64 rows; return (flat ids, host lengths)."""
     lengths: list[int] = []
     parts: list[torch.Tensor] = []
     for row in rows:
@@ -95,11 +98,49 @@ def ragged(rows: list[torch.Tensor | list[int] | tuple[int, ...]], device: torch
         t = t.to(device=device, dtype=torch.int64).reshape(-1)
         parts.append(t)
         lengths.append(int(t.numel()))
+    flat = torch.cat(parts) if parts else torch.empty(0, dtype=torch.int64, device=device)
+    return flat.contiguous(), lengths
+
+
+def prefix_offsets(lengths: list[int]) -> list[int]:
     offsets = [0]
     for n in lengths:
-        offsets.append(offsets[-1] + n)
-    flat = torch.cat(parts) if parts else torch.empty(0, dtype=torch.int64, device=device)
-    return torch.tensor(offsets, dtype=torch.int64, device=device), flat.contiguous(), lengths
+        offsets.append(offsets[-1] + int(n))
+    return offsets
+
+
+def ragged(rows: list[torch.Tensor | list[int] | tuple[int, ...]], device: torch.device) -> tuple[torch.Tensor, torch.Tensor, list[int]]:
+    """Concatenate int64 rows; return (offsets [n+1], flat ids, host lengths)."""
+    flat, lengths = ragged_ids(rows, device)
+    return torch.tensor(prefix_offsets(lengths), dtype=torch.int64, device=device), flat, lengths
+
+
+def pack_words(columns: list[list[int]], lengths32: list[int], device: torch.device) -> tuple[list[torch.Tensor], torch.Tensor]:
+    """Host lists as device tensors (int64 columns, then one of int32), cut from
+    one buffer that a single copy fills.  The copy reads pinned memory and is
+    queued on the current stream, so a batch waits for no earlier work (five
+    pageable copies took a tenth of a one-request compression); torch keeps
+    the pinned block from reuse until the copy has run.  A graph would copy
+    the block again at each replay, so capture is refused, as a pageable copy
+    is."""
+    if any(not -(1 << 31) <= int(n) < (1 << 31) for n in lengths32):
+        raise OverflowError("sequence lengths must fit 32 bits")
+    words = [int(v) for column in columns for v in column]
+    low = [int(n) & 0xFFFFFFFF for n in lengths32] + [0] * (len(lengths32) % 2)
+    for i in range(0, len(low), 2):
+        word = low[i] | low[i + 1] << 32
+        words.append(word - (1 << 64) if word >> 63 else word)
+    if device.type == "cuda":
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("batch descriptors cannot be copied to the device under graph capture")
+        flat = torch.tensor(words, dtype=torch.int64, pin_memory=True).to(device, non_blocking=True)
+    else:
+        flat = torch.tensor(words, dtype=torch.int64, device=device)
+    out, at = [], 0
+    for column in columns:
+        out.append(flat[at : at + len(column)])
+        at += len(column)
+    return out, flat[at:].view(torch.int32)[: len(lengths32)]
 
 
 class DescriptorCache:

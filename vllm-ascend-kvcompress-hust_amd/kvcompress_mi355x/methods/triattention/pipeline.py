@@ -128,33 +128,33 @@ class Batch:
         n = len(seq_lens)
         if n == 0 or len(round_starts) != n or len(source_tables) != n:
             raise ValueError("a batch needs matching lengths, round starts and source tables")
-        src_off, src_ids, src_lens = dev.ragged(list(source_tables), device)
+        src_ids, src_lens = dev.ragged_ids(list(source_tables), device)
         for length, blocks in zip(seq_lens, src_lens):
             if length < 0 or blocks * block_size < length:
                 raise ValueError("source block table does not cover the sequence")
-        dst_off = dst_ids = None
+        columns = [dev.prefix_offsets(seq_lens), round_starts, dev.prefix_offsets(src_lens)]
+        dst_ids = None
         if destination_tables is not None:
             if len(destination_tables) != n:
                 raise ValueError("one destination table per sequence")
-            dst_off, dst_ids, dst_lens = dev.ragged(list(destination_tables), device)
+            dst_ids, dst_lens = dev.ragged_ids(list(destination_tables), device)
+            columns.append(dev.prefix_offsets(dst_lens))
             if budget is not None:
                 need = (budget + block_size - 1) // block_size
                 if any(d < need for d in dst_lens):
                     raise ValueError("destination table too short for the budget")
-        offsets = [0]
-        for length in seq_lens:
-            offsets.append(offsets[-1] + int(length))
+        (token_offsets, round_starts_dev, src_off, *rest), seq_lens_dev = dev.pack_words(columns, seq_lens, device)
         return cls(
             n_seq=n,
             seq_lens_host=[int(x) for x in seq_lens],
             round_starts_host=[int(x) for x in round_starts],
             src_lengths_host=src_lens,
-            seq_lens=torch.tensor(seq_lens, dtype=torch.int32, device=device),
-            token_offsets=torch.tensor(offsets, dtype=torch.int64, device=device),
-            round_starts=torch.tensor(round_starts, dtype=torch.int64, device=device),
+            seq_lens=seq_lens_dev,
+            token_offsets=token_offsets,
+            round_starts=round_starts_dev,
             src_offsets=src_off,
             src_ids=src_ids,
-            dst_offsets=dst_off,
+            dst_offsets=rest[0] if rest else None,
             dst_ids=dst_ids,
         )
 
