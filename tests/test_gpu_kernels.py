@@ -759,6 +759,32 @@ def test_select_score_distributions(hip_device, kind) -> None:
             np.testing.assert_array_equal(keep[0].cpu().numpy(), _stable_keep_np(part.numpy(), keep_count, 0, 0, 1, "global"))
 
 
+@pytest.mark.parametrize(
+    "kind", ["normal", "outlier", "past-float32", "few-ulps", "two-values", "constant", "full-bin", "unresolved", "signed-zeros", "sorted"]
+)
+def test_select_split_score_distributions(hip_device, kind) -> None:
+    # The chunked form: bins of a sampled range, candidates ranked against each
+    # other (up to 512) or by radix passes (up to 4096), or radix passes over the
+    # segment; lengths around one chunk (4096), the sample (1024), 32 chunks
+    # and longer chunks, misaligned starts, keep counts from one to all but one.
+    _, selection, _ = _kvc()
+    g = torch.Generator().manual_seed(len(kind))
+    lens = [2, 1027, 4096, 4099, 20011, 131073, 290000]
+    parts = [torch.sort(torch.randn(n, generator=g)).values if kind == "sorted" else _score_distribution(kind, n, g) for n in lens]
+    offsets = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    d_scores = torch.cat(parts).to(hip_device)
+    for i, (n, part) in enumerate(zip(lens, parts)):
+        for keep_count in sorted({1, 2, n // 50 + 1, n // 2, n - 1} - {0}):
+            seq_lens = torch.tensor([n], dtype=torch.int32, device=hip_device)
+            token_offsets = torch.tensor(offsets[i : i + 2], dtype=torch.int64, device=hip_device)
+            keep = torch.full((1, keep_count), -7, dtype=torch.int64, device=hip_device)
+            selection.select_keep_indices_batched(
+                d_scores, seq_lens, token_offsets, [n], keep, budget=keep_count, protected_prefix=0, protected_recent=0,
+                segments=1, policy="global", shape="split",
+            )
+            np.testing.assert_array_equal(keep[0].cpu().numpy(), _stable_keep_np(part.numpy(), keep_count, 0, 0, 1, "global"))
+
+
 def test_select_split_rejects_a_small_workspace(hip_device) -> None:
     _, selection, _ = _kvc()
     scores = torch.randn(50000, device=hip_device)

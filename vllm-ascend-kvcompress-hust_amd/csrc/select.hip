@@ -15,13 +15,11 @@
 //    passes where they do not separate the scores).  Right for batches of many
 //    sequences.
 //  * kvc_select_keep_split: a job's segment is cut into chunks of >= 4096 keys,
-//    one 256-thread workgroup each.  Every radix pass is a launch: workgroups
-//    add their chunk histograms into the pass's histogram in the workspace;
-//    every workgroup of a later launch picks the earlier passes' digits
-//    itself from those finished histograms (no workgroup waits for another).
-//    Then one launch counts each chunk's keys > T and == T and one emits,
-//    each chunk starting from the counts of the chunks before it.  Right for
-//    a few long sequences, which would otherwise run on a few CUs.
+//    one 256-thread workgroup each, in three launches (no workgroup waits for
+//    another inside one): every chunk's histogram over value bins, the chunks'
+//    keys of the bin that holds the threshold, and the emission, each chunk
+//    starting from the counts of the chunks before it.  Right for a few long
+//    sequences, which would otherwise run on a few CUs.
 // Both produce the same indices.
 //
 // Segments follow select_keep_indices (tri/selection.py:108-196): the protected
@@ -38,7 +36,7 @@ namespace {
 constexpr int kSelThreads = 1024;   // one workgroup per job
 constexpr int kSplitThreads = 256;  // split path: one workgroup per chunk
 constexpr int kSplitChunk = 4096;   // keys per chunk, at least
-constexpr int kSplitMaxChunks = 64;
+constexpr int kSplitMaxChunks = 32;
 constexpr int kSelUnroll = 4;  // float4 words per thread in flight in a histogram pass
 constexpr int kEmitWords = 2;  // float4 words per thread per emission tile
 constexpr int kSelPeel = 1;    // dominant digits counted with one atomic per wave
@@ -457,17 +455,17 @@ struct Picked {
   uint32_t thresh, need_eq, ties;  // key of the K-th largest score, its ties to keep, all its ties
 };
 
-// The threshold by four radix passes over the scores.  Out of line, as
-// select_long below: what most calls run stays small in the instruction cache.
-__device__ __noinline__ Picked radix_threshold(const float* sc, int64_t start, int64_t stop, uint32_t need) {
-  __shared__ uint32_t whist[kSelThreads / 64][256];
+// The threshold by four radix passes over the scores, by a workgroup of T threads.
+template <int T>
+__device__ __forceinline__ Picked radix_pick(const float* sc, int64_t start, int64_t stop, uint32_t need) {
+  __shared__ uint32_t whist[T / 64][256];
   __shared__ uint32_t hist[256];
   __shared__ uint32_t s_digit, s_need;
   Picked p{0u, need, 0u};
   uint32_t mask = 0;
   for (int pass = 0; pass < 4; ++pass) {
     const int shift = 24 - 8 * pass;
-    range_histogram<kSelThreads>(sc, start, stop, p.thresh, mask, shift, whist, hist);
+    range_histogram<T>(sc, start, stop, p.thresh, mask, shift, whist, hist);
     if (threadIdx.x < 64) pick_digit(hist, p.need_eq, &s_digit, &s_need);
     __syncthreads();
     p.thresh |= s_digit << shift;
@@ -477,6 +475,12 @@ __device__ __noinline__ Picked radix_threshold(const float* sc, int64_t start, i
     __syncthreads();
   }
   return p;
+}
+
+// Out of line, as select_long below: what most calls run stays small in the
+// instruction cache.
+__device__ __noinline__ Picked radix_threshold(const float* sc, int64_t start, int64_t stop, uint32_t need) {
+  return radix_pick<kSelThreads>(sc, start, stop, need);
 }
 
 // Keeps the `keep` largest scores of [start, stop), their indices written from
@@ -644,15 +648,36 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(SelectArgs a) {
 
 // ------------------------------------------------------ split over chunks --
 
-// Per-job scratch of the split path (in the caller's workspace): the job's
-// keep count and liveness (set by the reset launch), each radix pass's
-// histogram (the chunks' atomic sums) and each chunk's counts of keys > T and
-// == T.
+// The threshold of a long segment, in three launches (seven when four radix
+// passes named it, a clear before and a count after: 4 x 130816 scores 37.7 us
+// against 19.7 now).  Bins are equal cells of a range taken from a sample, a
+// little wider at the top, so no launch has to find the range first: any range
+// is right, since scores past it count in the end bins, and the bins only have
+// to keep the order of the keys.  Every chunk stores a histogram of its own
+// (no atomics, nothing to clear), every chunk of the second launch adds them
+// all, and the threshold's bin holds some hundred keys, ranked exactly.  More
+// than kSplitCand keys there are usually ties of one key, which is then the
+// threshold; if not, every chunk's workgroup makes radix passes over the whole
+// segment.
+constexpr int kSplitBins = 1024;
+constexpr int kSplitCand = 4096;
+constexpr int kSplitRanked = 512;  // candidates ranked against each other; more take radix passes over them
+constexpr int kSplitSamples = 1024;
+static_assert(kSplitBins == 4 * kSplitThreads, "a thread owns four bins");
+
+// Per-job scratch (in the caller's workspace), written before it is read by
+// every call.
 struct SplitState {
-  uint32_t need, live, pad[2];
-  uint32_t hist[4][256];
-  uint32_t counts[kSplitMaxChunks][2];
+  float lo, scale;             // bin of x: (x - lo) * scale
+  uint32_t rank, count;        // the threshold's rank from the top of its bin, keys in that bin
+  uint32_t least[kSplitMaxChunks];   // smallest and largest key of the bin in a
+  uint32_t most[kSplitMaxChunks];    // chunk, where the bin is too full for cand
+  uint32_t above[kSplitMaxChunks];   // a chunk's keys in higher bins
+  uint32_t before[kSplitMaxChunks];  // candidates of the chunks before
+  uint32_t hist[kSplitMaxChunks][kSplitBins];
+  float cand[kSplitCand];      // the bin's scores, chunk after chunk
 };
+static_assert(sizeof(SplitState) % 16 == 0, "jobs' states stay aligned");
 
 __host__ __device__ inline int64_t split_chunk_len(int64_t len) {
   int64_t cs = (len + kSplitMaxChunks - 1) / kSplitMaxChunks;
@@ -668,132 +693,243 @@ __device__ __forceinline__ SplitState* split_state(const SelectArgs& a, int b, i
   return static_cast<SplitState*>(a.state) + static_cast<int64_t>(b) * a.segments + seg;
 }
 
-// grid (segments, n_seq): protected windows, whole segments, and the job's
-// scratch reset (the workspace may hold the previous call's values).
-__global__ __launch_bounds__(kSplitThreads) void select_split_init_kernel(SelectArgs a) {
-  const int b = blockIdx.y, seg = blockIdx.x, tid = threadIdx.x;
-  SplitState* st = split_state(a, b, seg);
-  const Job j = make_job(a, b, seg);
-  int64_t* out = a.keep + static_cast<int64_t>(b) * a.keep_stride;
-  const bool live = fill_fixed(a, j, seg, out, tid, kSplitThreads);
-  uint32_t* words = reinterpret_cast<uint32_t*>(st);
-  for (int i = tid; i < static_cast<int>(sizeof(SplitState) / 4); i += kSplitThreads) words[i] = 0;
+// Order-preserving bin of a score.  Infinities and NaNs go by their key (sign
+// set: below every score); a scale of zero puts every finite score in bin 0.
+__device__ __forceinline__ int split_bin(float x, float lo, float scale) {
+  if (!(fabsf(x) <= 3.402823466e38f)) return (float_key(x) >> 31) ? kSplitBins - 1 : 0;
+  return static_cast<int>(fminf(fmaxf((x - lo) * scale, 0.0f), static_cast<float>(kSplitBins - 1)));
+}
+
+// The chunk of this workgroup (grid: chunks, segments, n_seq).
+struct Chunk {
+  Job j;
+  int c;
+  int chunks;
+  int64_t start, stop;
+  bool live;  // the job needs a threshold and the chunk exists
+};
+
+__device__ __forceinline__ Chunk make_chunk(const SelectArgs& a) {
+  Chunk k;
+  k.c = blockIdx.x;
+  k.j = make_job(a, blockIdx.z, blockIdx.y);
+  const int64_t len = k.j.s.stop - k.j.s.start;
+  k.chunks = split_chunks(len);
+  k.live = k.j.exists && k.j.s.keep > 0 && len > k.j.s.keep && k.c < k.chunks;
+  const int64_t cs = split_chunk_len(len);
+  k.start = k.j.s.start + k.c * cs;
+  k.stop = min(k.j.s.stop, k.start + cs);
+  return k;
+}
+
+// Launch 1: protected windows and segments kept whole (chunk 0), the bins'
+// range, the chunk's histogram.
+__global__ __launch_bounds__(kSplitThreads) void select_split_bins_kernel(SelectArgs a) {
+  __shared__ __attribute__((aligned(16))) uint32_t bins[kSplitBins];
+  __shared__ float s_lo[kSplitThreads / 64], s_hi[kSplitThreads / 64];
+  const int tid = threadIdx.x;
+  const Chunk k = make_chunk(a);
+  if (k.c == 0)
+    fill_fixed(a, k.j, blockIdx.y, a.keep + static_cast<int64_t>(blockIdx.z) * a.keep_stride, tid, kSplitThreads);
+  if (!k.live) return;  // the whole workgroup
+  const float* sc = a.scores + a.token_offsets[blockIdx.z];
+  const int64_t len = k.j.s.stop - k.j.s.start;
+  for (int i = tid; i < kSplitBins; i += kSplitThreads) bins[i] = 0;
+  float lo = INFINITY, hi = -INFINITY;
+  float x[kSplitSamples / kSplitThreads];
+#pragma unroll
+  for (int u = 0; u < kSplitSamples / kSplitThreads; ++u)
+    x[u] = sc[k.j.s.start + (tid + kSplitThreads * u) * len / kSplitSamples];
+#pragma unroll
+  for (int u = 0; u < kSplitSamples / kSplitThreads; ++u) {
+    const bool finite = fabsf(x[u]) <= 3.402823466e38f;
+    lo = fminf(lo, finite ? x[u] : INFINITY);
+    hi = fmaxf(hi, finite ? x[u] : -INFINITY);
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    lo = fminf(lo, __shfl_xor(lo, off));
+    hi = fmaxf(hi, __shfl_xor(hi, off));
+  }
+  if ((tid & 63) == 0) {
+    s_lo[tid >> 6] = lo;
+    s_hi[tid >> 6] = hi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kSplitThreads / 64; ++w) {
+    lo = fminf(lo, s_lo[w]);
+    hi = fmaxf(hi, s_hi[w]);
+  }
+  const float width = hi - lo;
+  lo -= 0.125f * width;
+  float scale = kSplitBins / (1.625f * width);
+  if (!(width > 0.0f && scale > 0.0f && scale < INFINITY && fabsf(lo) < INFINITY)) {
+    lo = 0.0f;
+    scale = 0.0f;
+  }
+  for_each_score<kSplitThreads>(sc, k.start, k.stop, [&](float v) { atomicAdd(&bins[split_bin(v, lo, scale)], 1u); });
+  __syncthreads();
+  SplitState* st = split_state(a, blockIdx.z, blockIdx.y);
+  reinterpret_cast<uint4*>(st->hist[k.c])[tid] = reinterpret_cast<const uint4*>(bins)[tid];
+  if (k.c == 0 && tid == 0) {
+    st->lo = lo;
+    st->scale = scale;
+  }
+}
+
+// Launch 2: the threshold's bin from all chunks' histograms; the chunk's keys
+// of that bin and its number of keys in higher ones.
+__global__ __launch_bounds__(kSplitThreads) void select_split_candidates_kernel(SelectArgs a) {
+  __shared__ uint32_t s_wave[kSplitThreads / 64];
+  __shared__ uint32_t s_bin, s_rank, s_count, s_before, s_filled, s_least, s_most;
+  const int tid = threadIdx.x;
+  const Chunk k = make_chunk(a);
+  if (!k.live) return;
+  if (tid == 0) {
+    s_least = 0xffffffffu;
+    s_most = 0;
+  }
+  SplitState* st = split_state(a, blockIdx.z, blockIdx.y);
+  const uint32_t keep = static_cast<uint32_t>(k.j.s.keep);
+  const float lo = st->lo, scale = st->scale;
+  // Thread t owns bins top - 4t .. top - 4t - 3: thread order is falling order.
+  const int word = kSplitThreads - 1 - tid;
+  uint32_t all[4] = {0, 0, 0, 0}, pre[4] = {0, 0, 0, 0}, own[4] = {0, 0, 0, 0};
+  uint4 h[kSplitMaxChunks];  // every load in flight at once
+#pragma unroll
+  for (int c = 0; c < kSplitMaxChunks; ++c) h[c] = reinterpret_cast<const uint4*>(st->hist[min(c, k.chunks - 1)])[word];
+#pragma unroll
+  for (int c = 0; c < kSplitMaxChunks; ++c) {
+    const uint32_t v[4] = {h[c].w, h[c].z, h[c].y, h[c].x};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      all[q] += c < k.chunks ? v[q] : 0u;
+      pre[q] += c < k.c ? v[q] : 0u;
+      own[q] = c == k.c ? v[q] : own[q];
+    }
+  }
+  if (tid == 0) s_filled = 0;
+  uint32_t total;
+  uint32_t above = block_exclusive_scan<kSplitThreads>(all[0] + all[1] + all[2] + all[3], s_wave, &total);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (above < keep && keep <= above + all[q]) {
+      s_bin = static_cast<uint32_t>(kSplitBins - 1 - 4 * tid - q);
+      s_rank = keep - above;
+      s_count = all[q];
+      s_before = pre[q];
+    }
+    above += all[q];
+  }
+  __syncthreads();
+  const int bin = static_cast<int>(s_bin);
+  const uint32_t count = s_count, before = s_before;
+  uint32_t higher = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) higher += kSplitBins - 1 - 4 * tid - q > bin ? own[q] : 0u;
+  uint32_t above_here;
+  block_exclusive_scan<kSplitThreads>(higher, s_wave, &above_here);
+  if (tid == 0) {
+    st->above[k.c] = above_here;
+    st->before[k.c] = before;
+    if (k.c == 0) {
+      st->rank = s_rank;
+      st->count = count;
+    }
+  }
+  const float* sc = a.scores + a.token_offsets[blockIdx.z];
+  if (count <= kSplitCand) {
+    for_each_score<kSplitThreads>(sc, k.start, k.stop, [&](float x) {
+      if (split_bin(x, lo, scale) == bin) st->cand[before + atomicAdd(&s_filled, 1u)] = x;
+    });
+    return;
+  }
+  uint32_t least = 0xffffffffu, most = 0;
+  for_each_score<kSplitThreads>(sc, k.start, k.stop, [&](float x) {
+    if (split_bin(x, lo, scale) == bin) {
+      least = min(least, float_key(x));
+      most = max(most, float_key(x));
+    }
+  });
+  atomicMin(&s_least, least);
+  atomicMax(&s_most, most);
   __syncthreads();
   if (tid == 0) {
-    st->live = live ? 1u : 0u;
-    st->need = live ? static_cast<uint32_t>(j.s.keep) : 0u;
+    st->least[k.c] = s_least;
+    st->most[k.c] = s_most;
   }
 }
 
-// The radix prefix (want, mask) and the number of keys still needed inside
-// it after `passes` passes: each pass's digit picked from that pass's
-// histogram, complete since an earlier launch, exactly as the last pass of
-// that histogram would have picked it.  The histograms are read together,
-// then walked in LDS.  Every thread calls it; the results are in `out` (LDS)
-// on return.
-struct Threshold {
-  uint32_t want, mask, need, digit;
-};
-__device__ void derive_threshold(const SplitState* st, int passes, uint32_t (*s_hist)[256], Threshold* out) {
-  const int tid = threadIdx.x;
-  for (int i = tid; i < passes * 256; i += kSplitThreads) (&s_hist[0][0])[i] = (&st->hist[0][0])[i];
-  if (tid == 0) *out = Threshold{0u, 0u, st->need, 0u};
-  __syncthreads();
-  for (int q = 0; q < passes; ++q) {
-    if (tid < 64) {
-      const uint32_t need = out->need;  // read by every lane before one lane writes
-      pick_digit(s_hist[q], need, &out->digit, &out->need);
-    }
-    __syncthreads();
-    if (tid == 0) {
-      const int shift = 24 - 8 * q;
-      out->want |= out->digit << shift;
-      out->mask |= 0xFFu << shift;
-    }
-    __syncthreads();
-  }
-}
-
-// grid (chunks, segments, n_seq): one radix pass.  Each workgroup derives the
-// prefix of the passes before (from their histograms) and adds its chunk's
-// histogram of the matching keys into the job's; no workgroup waits for
-// another inside the launch.
-__global__ __launch_bounds__(kSplitThreads) void select_split_pass_kernel(SelectArgs a, int pass) {
-  __shared__ uint32_t whist[kSplitThreads / 64][256];
-  __shared__ uint32_t hist[256];
-  __shared__ uint32_t s_prev[3][256];
-  __shared__ Threshold s_th;
-  const int c = blockIdx.x, seg = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
-  SplitState* st = split_state(a, b, seg);
-  if (!st->live) return;  // the whole workgroup reads the same word
-  const Job j = make_job(a, b, seg);
-  const int64_t len = j.s.stop - j.s.start;
-  const int chunks = split_chunks(len);
-  if (c >= chunks) return;
-  const int64_t cs = split_chunk_len(len);
-  const int64_t c0 = j.s.start + c * cs, c1 = min(j.s.stop, c0 + cs);
-  derive_threshold(st, pass, s_prev, &s_th);
-  const int shift = 24 - 8 * pass;
-  const float* sc = a.scores + a.token_offsets[b];
-  range_histogram<kSplitThreads>(sc, c0, c1, s_th.want, s_th.mask, shift, whist, hist);
-  for (int i = tid; i < 256; i += kSplitThreads)
-    if (hist[i]) atomicAdd(&st->hist[pass][i], hist[i]);
-}
-
-// grid (chunks, segments, n_seq): each chunk's keys > T and == T.
-__global__ __launch_bounds__(kSplitThreads) void select_split_count_kernel(SelectArgs a) {
-  __shared__ uint32_t s_wave[kSplitThreads / 64];
-  __shared__ uint32_t s_prev[4][256];
-  __shared__ Threshold s_th;
-  const int c = blockIdx.x, seg = blockIdx.y, b = blockIdx.z;
-  SplitState* st = split_state(a, b, seg);
-  if (!st->live) return;
-  const Job j = make_job(a, b, seg);
-  const int64_t len = j.s.stop - j.s.start;
-  if (c >= split_chunks(len)) return;
-  const int64_t cs = split_chunk_len(len);
-  const int64_t c0 = j.s.start + c * cs, c1 = min(j.s.stop, c0 + cs);
-  derive_threshold(st, 4, s_prev, &s_th);
-  const uint32_t thresh = s_th.want;
-  const float* sc = a.scores + a.token_offsets[b];
-  uint32_t g = 0, e = 0;
-  for_each_score<kSplitThreads>(sc, c0, c1, [&](float x) {
-    const uint32_t k = float_key(x);
-    g += k > thresh;
-    e += k == thresh;
-  });
-  uint32_t total_g, total_e;
-  block_exclusive_scan<kSplitThreads>(g, s_wave, &total_g);
-  block_exclusive_scan<kSplitThreads>(e, s_wave, &total_e);
-  if (threadIdx.x == 0) {
-    st->counts[c][0] = total_g;
-    st->counts[c][1] = total_e;
-  }
-}
-
-// grid (chunks, segments, n_seq): ordered emission of each chunk.
+// Launch 3: the threshold among the candidates, and the chunk's ordered emission.
 __global__ __launch_bounds__(kSplitThreads) void select_split_emit_kernel(SelectArgs a) {
+  __shared__ __attribute__((aligned(16))) float cand[kSplitCand];
+  __shared__ __attribute__((aligned(16))) uint32_t keys[kSplitRanked];
   __shared__ uint32_t s_wave[kSplitThreads / 64];
-  __shared__ uint32_t s_prev[4][256];
-  __shared__ Threshold s_th;
-  const int c = blockIdx.x, seg = blockIdx.y, b = blockIdx.z;
-  SplitState* st = split_state(a, b, seg);
-  if (!st->live) return;
-  const Job j = make_job(a, b, seg);
-  const int64_t len = j.s.stop - j.s.start;
-  if (c >= split_chunks(len)) return;
-  const int64_t cs = split_chunk_len(len);
-  const int64_t c0 = j.s.start + c * cs, c1 = min(j.s.stop, c0 + cs);
-  uint32_t g0 = 0, e0 = 0;
-  for (int i = 0; i < c; ++i) {
-    g0 += st->counts[i][0];
-    e0 += st->counts[i][1];
+  __shared__ Picked s_picked;
+  const int tid = threadIdx.x;
+  const Chunk k = make_chunk(a);
+  if (!k.live) return;
+  const SplitState* st = split_state(a, blockIdx.z, blockIdx.y);
+  const float* sc = a.scores + a.token_offsets[blockIdx.z];
+  const uint32_t count = st->count, rank = st->rank;
+  Picked p;
+  uint32_t g = 0, e = 0;  // this thread's share of the keys > and == the threshold before the chunk
+  const uint32_t before = st->before[k.c];
+  uint32_t least = 0xffffffffu, most = 0;
+  if (count > kSplitCand)
+    for (int c = 0; c < k.chunks; ++c) {
+      least = min(least, st->least[c]);
+      most = max(most, st->most[c]);
+    }
+  if (count <= kSplitCand) {
+    for (uint32_t i = tid; i < count; i += kSplitThreads) cand[i] = st->cand[i];
+    if (count <= kSplitRanked) {
+      const uint32_t padded = (count + 3) & ~3u;  // with the smallest key, corrected below
+      for (uint32_t i = tid; i < padded; i += kSplitThreads) keys[i] = i < count ? float_key(st->cand[i]) : 0u;
+      __syncthreads();
+      for (uint32_t i = tid; i < count; i += kSplitThreads) {
+        const uint32_t mine = keys[i];
+        uint32_t more = 0, same = mine == 0u ? count - padded : 0u;
+        for (uint32_t q = 0; q < padded; q += 4) {
+          const uint4 other = *reinterpret_cast<const uint4*>(keys + q);
+          more += (other.x > mine) + (other.y > mine) + (other.z > mine) + (other.w > mine);
+          same += (other.x == mine) + (other.y == mine) + (other.z == mine) + (other.w == mine);
+        }
+        if (more < rank && rank <= more + same) s_picked = Picked{mine, rank - more, same};  // equal keys write the same
+      }
+      __syncthreads();
+      p = s_picked;
+    } else {
+      __syncthreads();
+      p = radix_pick<kSplitThreads>(cand, 0, count, rank);
+    }
+    for (uint32_t i = tid; i < before; i += kSplitThreads) {
+      const uint32_t key = float_key(cand[i]);
+      g += key > p.thresh;
+      e += key == p.thresh;
+    }
+    if (tid < k.c) g += st->above[tid];
+  } else if (least == most) {  // ties of one key fill the bin
+    p = Picked{least, rank, count};
+    if (tid < k.c) g += st->above[tid];
+    if (tid == 0) e = before;
+  } else {
+    p = radix_pick<kSplitThreads>(sc, k.j.s.start, k.j.s.stop, static_cast<uint32_t>(k.j.s.keep));
+    if (k.c > 0)
+      for_each_score<kSplitThreads>(sc, k.j.s.start, k.start, [&](float x) {
+        const uint32_t key = float_key(x);
+        g += key > p.thresh;
+        e += key == p.thresh;
+      });
   }
-  derive_threshold(st, 4, s_prev, &s_th);
-  int64_t* out = a.keep + static_cast<int64_t>(b) * a.keep_stride;
-  // Whether a later chunk holds ties is not known here: ties count apart.
-  const Keep kp{s_th.want, s_th.need, false, out, static_cast<int>(j.out_base), a.budget};
-  emit_range<kSplitThreads>(kp, a.scores + a.token_offsets[b], c0, c1, g0, e0, s_wave);
+  uint32_t g0, e0;
+  block_exclusive_scan<kSplitThreads>(g, s_wave, &g0);
+  block_exclusive_scan<kSplitThreads>(e, s_wave, &e0);
+  int64_t* out = a.keep + static_cast<int64_t>(blockIdx.z) * a.keep_stride;
+  const Keep kp{p.thresh, p.need_eq, p.ties == p.need_eq, out, static_cast<int>(k.j.out_base), a.budget};
+  // With every tie kept, both kinds count in the first number.
+  emit_range<kSplitThreads>(kp, sc, k.start, k.stop, kp.all_ties ? g0 + e0 : g0, kp.all_ties ? 0u : e0, s_wave);
 }
 
 int check_select_args(const char* who, int n_seq, int max_seq_len, const int32_t* seq_lens,
@@ -875,15 +1011,11 @@ extern "C" int kvc_select_keep_split(kvc_stream_t stream, int n_seq, int max_seq
   // A segment is at most the whole sequence.
   const int chunks = split_chunks(max_seq_len);
   hipStream_t st = as_stream(stream);
-  select_split_init_kernel<<<dim3(sa.segments, n_seq), kSplitThreads, 0, st>>>(sa);
-  if (int rc = launch_status("kvc_select_keep_split(init)")) return rc;
   const dim3 grid(static_cast<unsigned>(chunks), static_cast<unsigned>(sa.segments), static_cast<unsigned>(n_seq));
-  for (int pass = 0; pass < 4; ++pass) {
-    select_split_pass_kernel<<<grid, kSplitThreads, 0, st>>>(sa, pass);
-    if (int rc = launch_status("kvc_select_keep_split(pass)")) return rc;
-  }
-  select_split_count_kernel<<<grid, kSplitThreads, 0, st>>>(sa);
-  if (int rc = launch_status("kvc_select_keep_split(count)")) return rc;
+  select_split_bins_kernel<<<grid, kSplitThreads, 0, st>>>(sa);
+  if (int rc = launch_status("kvc_select_keep_split(bins)")) return rc;
+  select_split_candidates_kernel<<<grid, kSplitThreads, 0, st>>>(sa);
+  if (int rc = launch_status("kvc_select_keep_split(candidates)")) return rc;
   select_split_emit_kernel<<<grid, kSplitThreads, 0, st>>>(sa);
   return launch_status("kvc_select_keep_split(emit)");
 }

@@ -16,12 +16,14 @@ from . import _device as dev
 
 POLICY_CODES = {"global": _native.POLICY_GLOBAL, "v3": _native.POLICY_V3}
 
-# kvc_select_keep runs one workgroup per (sequence, segment), about 10 us plus
-# 0.7 us per 1K scores of the longest segment; kvc_select_keep_split (seven
-# launches, chunks spread over the chip) takes 50-65 us for up to a few dozen
-# segments: 4 x 130816 scores 66 us against 100 us, 16 x 16256 53 us against
-# 23 us.  The crossover is near 64K scores per segment.
-SPLIT_MIN_SEGMENT = 65536
+# kvc_select_keep runs one workgroup per (sequence, segment), 11 us for 16K
+# scores and about 0.35 us per further 1K of the longest segment;
+# kvc_select_keep_split (three launches, chunks spread over the chip) takes
+# 18-23 us for a few segments of up to 256K scores and up to 37 for 32 of them:
+# 1 x 49152 scores 18.5 us against 25.4, 4 x 131072 19.7 against 54, 16 x 32768
+# 19.8 against 20.0, 1 x 16384 17 against 11.  At 32K the two are level; the
+# line is above it, where the chunks win with 32 jobs too (65536: 27 against 32).
+SPLIT_MIN_SEGMENT = 49152
 SPLIT_MAX_JOBS = 32
 
 
