@@ -27,7 +27,7 @@
 // 256-token spans; its four waves walk interleaved 16-token tiles of a span.
 // The per-offset fragments (bf16 or fp16 hi/lo, 1 KB per 32 rotary dims and
 // chunk) are staged in LDS once per workgroup; each fragment read feeds two
-// key tiles (one in the three-waves-per-SIMD form).  Workgroups that share a
+// key tiles (one at 256 dims).  Workgroups that share a
 // key span but not a query-head group are placed eight apart in the grid, on
 // the same XCD, so the second read of the keys is an L2 hit.  Raw scores and partial sums have the mean scorer's
 // layout, so kvc_head_stats and kvc_aggregate are shared.
@@ -249,18 +249,23 @@ struct MaxGeometry {
   int64_t tail_base;
 };
 
-// One tile per fragment pass at three waves per SIMD, or two tiles per pass
-// at two: the first keeps more key loads in flight, the second halves the
-// fragment reads per product.
-template <int NK, bool ONE_TILE>
+// Two key tiles per fragment pass (one at 256 dims).  LEAN, the form for 128
+// dims without tail chunks: one fragment buffer whose words are replaced by
+// the next head's as their products issue, so that two tiles fit three waves
+// per SIMD.  Scoring and aggregating 8 x 16384 tokens x 6 layers, 16 offsets, 5
+// query heads: 495 us with one tile and the heads under run-time branches, 488
+// with the heads' number known, 482 with two tiles (half the LDS reads; about
+// 420 of it is this kernel: the matrix cores take 118 us, the vector ALUs about
+// as much, the LDS reads 100, the mixed reads and writes of HBM 330).
+template <int NK, bool LEAN>
 struct MaxTiling {
-  static constexpr int T = ONE_TILE || NK >= 8 ? 1 : 2;
-  static constexpr int kWavesPerSimd = ONE_TILE ? 3 : 1;  // 1: no request
+  static constexpr int T = NK >= 8 ? 1 : 2;
+  static constexpr int kWavesPerSimd = LEAN ? 3 : 1;  // 1: no request
 };
 
-template <int NK, int NF, int NCH, bool F16, bool IL, bool ONE_TILE>
+template <int NK, int NF, int NCH, bool F16, bool IL, bool LEAN, int GC>
 __global__ __launch_bounds__(kScoreThreads)
-__attribute__((amdgpu_waves_per_eu(MaxTiling<NK, ONE_TILE>::kWavesPerSimd))) void score_max_kernel(
+__attribute__((amdgpu_waves_per_eu(MaxTiling<NK, LEAN>::kWavesPerSimd))) void score_max_kernel(
     ScoreArgs a, MaxGeometry geo, int qpk, const u32x4* __restrict__ rest_frags, const float* __restrict__ rest_scale,
     const u32x4* __restrict__ off_frags, const float* __restrict__ off_scale) {
   typedef MfmaElem<F16> E;
@@ -285,19 +290,19 @@ __attribute__((amdgpu_waves_per_eu(MaxTiling<NK, ONE_TILE>::kWavesPerSimd))) voi
   const int n = a.seq_lens[b];
   if (tile_first * kScoreTile >= n) return;  // whole workgroup leaves together
   const int g0 = gg * geo.gpg;
-  const int gcnt = min(geo.gpg, qpk - g0);
+  const int gcnt = GC > 0 ? GC : min(geo.gpg, qpk - g0);
   if (gcnt <= 0) return;
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar, as a tile's address below
   const int r = lane & 15;   // token of the tile (B column / D column)
   const int kb = lane >> 4;  // K block of the operands, row block of D
   const int64_t col0 = ((static_cast<int64_t>(b) * a.n_layers + layer) * a.kv_heads + head) * qpk;
   constexpr int kFragPerG = NCH * NR * 2 * 64;
   // Shared tail chunks exist for head_dim >= 128 only (at 64 dims their code
-  // would cost the kernel its third wave per SIMD), and not in the one-tile
+  // would cost the kernel its third wave per SIMD), and not in the lean
   // form, which the launcher picks only without them.
-  constexpr bool kTail = NCH == 1 && !F16 && NK >= 4 && !ONE_TILE;
+  constexpr bool kTail = NCH == 1 && !F16 && NK >= 4 && !LEAN;
 
   // Stage this group's per-offset fragments.
   {
@@ -357,7 +362,7 @@ __attribute__((amdgpu_waves_per_eu(MaxTiling<NK, ONE_TILE>::kWavesPerSimd))) voi
   const int64_t* bt = a.block_ids + a.block_offsets[b];
   const int64_t n_blocks = a.block_offsets[b + 1] - a.block_offsets[b];
   const int64_t row_elems = static_cast<int64_t>(a.kv_heads) * a.head_dim;
-  const int64_t lane_off = static_cast<int64_t>(head) * a.head_dim + 8 * kb;
+  const int64_t head_off = static_cast<int64_t>(head) * a.head_dim;
   const int64_t tok_base = a.token_offsets[b];
   float* raw_out = a.raw + layer * a.raw_layer_stride;
   __syncthreads();  // fragments staged
@@ -392,27 +397,27 @@ __attribute__((amdgpu_waves_per_eu(MaxTiling<NK, ONE_TILE>::kWavesPerSimd))) voi
   // span re-read its last tile and rows past the sequence read whatever their
   // page holds: a token is a column of every product here, so those rows only
   // reach scores that are never stored.  Unresolved pages read as zeros.
+  const uint32_t lane_bytes = (static_cast<uint32_t>(r) * static_cast<uint32_t>(row_elems) + 8 * kb) * 2;
   auto load_tile = [&](const SpanPages& pg, int st0, int st1, int mt, u32x4 (&ka)[NK]) {
     const int smt = (st1 - st0 + 15) / 16;
-    const int mt_read = mt < smt ? mt : smt - 1;
-    const int rel = mt_read * 16 + r;
-    const int t = st0 + rel;
+    const int rel = min(mt, smt - 1) * 16;
     bool page_ok = false;
     KVC_GLOBAL const uint16_t* pbase = pg.page(rel, &page_ok);
-    KVC_GLOBAL const uint16_t* row =
-        page_ok ? pbase + static_cast<int64_t>(t & (kBlockSize - 1)) * row_elems + lane_off
-                : reinterpret_cast<KVC_GLOBAL const uint16_t*>(gptr(kZeroKeys));
+    // (pages' first tokens are span-aligned, so rel places the tile in its page)
+    KVC_GLOBAL const uint16_t* first = pbase + static_cast<int64_t>(rel & (kBlockSize - 1)) * row_elems + head_off;
+    KVC_GLOBAL const char* at =
+        reinterpret_cast<KVC_GLOBAL const char*>(page_ok ? first : reinterpret_cast<KVC_GLOBAL const uint16_t*>(gptr(kZeroKeys)));
+    const uint32_t off = page_ok ? lane_bytes : 0u;
 #pragma unroll
-    for (int j = 0; j < NK; ++j) ka[j] = load_k(reinterpret_cast<KVC_GLOBAL const u32x4*>(row + 32 * j));
+    for (int j = 0; j < NK; ++j) ka[j] = load_k(reinterpret_cast<KVC_GLOBAL const u32x4*>(at + off + 64 * j));
   };
 
   // Wave w scores tiles w, w+4, w+8, w+12 of every span in groups of T tiles
   // (T = 2: each fragment read feeds two tiles; T = 1 for head_dim 256,
-  // whose key registers would otherwise leave one wave per SIMD, and for the
-  // three-waves-per-SIMD form).  The keys of the next group, also across a
+  // whose key registers would otherwise leave one wave per SIMD).  The keys of the next group, also across a
   // span boundary and the span's epilogue, are in flight while a group is
   // scored.
-  constexpr int T = MaxTiling<NK, ONE_TILE>::T;
+  constexpr int T = MaxTiling<NK, LEAN>::T;
   constexpr int kGroups = 4 / T;
   static_assert(kScoreTile == 16 * 4 * kStreams, "four tiles per wave cover a span");
   static_assert(kGroups % 2 == 0, "a span's first group lands in buffer 0");
@@ -474,9 +479,9 @@ __attribute__((amdgpu_waves_per_eu(MaxTiling<NK, ONE_TILE>::kWavesPerSimd))) voi
 #pragma unroll
       for (int u = 0; u < T; ++u) rest[u] = rest_tile(kk[u]);
       // Fragment registers: two buffers (the next item's fragments are read
-      // while this item's products run), or, in the one-tile form, one buffer
+      // while this item's products run), or, in the lean form, one buffer
       // whose words are replaced by the next item's as their products issue.
-      constexpr int kBufs = ONE_TILE ? 1 : 2;
+      constexpr int kBufs = LEAN ? 1 : 2;
       vec_t wbuf[kBufs][2 * NR];
       load_w(0, wbuf[0]);
       f32x4 tv[T];
@@ -496,18 +501,25 @@ __attribute__((amdgpu_waves_per_eu(MaxTiling<NK, ONE_TILE>::kWavesPerSimd))) voi
             const int it = (4 * q + j) * NCH + c;
             if (4 * q + j < gcnt) {
               f32x4 res[T];
-              if constexpr (ONE_TILE) {
+              if constexpr (LEAN) {
                 const u32x4* wl = lds_frag + (min(it + 1, n_items - 1) * NR) * 128 + lane;
-                f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+                f32x4 acc[T][2];
+#pragma unroll
+                for (int u = 0; u < T; ++u) acc[u][0] = acc[u][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int st = 0; st < NR; ++st) {
 #pragma unroll
                   for (int h = 0; h < 2; ++h) {
-                    acc[h] = E::mfma(wbuf[0][2 * st + h], __builtin_bit_cast(vec_t, kk[0][st]), acc[h]);
+#pragma unroll
+                    for (int u = 0; u < T; ++u) {
+                      const int chain = T == 1 ? h : 0;
+                      acc[u][chain] = E::mfma(wbuf[0][2 * st + h], __builtin_bit_cast(vec_t, kk[u][st]), acc[u][chain]);
+                    }
                     wbuf[0][2 * st + h] = __builtin_bit_cast(vec_t, wl[st * 128 + h * 64]);
                   }
                 }
-                res[0] = acc[0] + acc[1];
+#pragma unroll
+                for (int u = 0; u < T; ++u) res[u] = T == 1 ? acc[u][0] + acc[u][1] : acc[u][0];
               } else {
                 load_w(it + 1, wbuf[(it + 1) & 1]);
                 chunk_products(wbuf[it & 1], res);
@@ -788,27 +800,43 @@ ValuMaxKernel pick_valu_max(int nch) {
 
 using MaxKernel = void (*)(ScoreArgs, MaxGeometry, int, const u32x4*, const float*, const u32x4*, const float*);
 
+// Lean form: the number of query heads of a workgroup that holds all of a
+// KV head's is known at compile time, so the heads' products and maxima are
+// scheduled across each other; 0: any number.
+template <int NF, bool F16, bool IL>
+MaxKernel pick_max_heads(int heads) {
+  switch (heads) {
+    case 1: return score_max_kernel<4, NF, 1, F16, IL, true, 1>;
+    case 2: return score_max_kernel<4, NF, 1, F16, IL, true, 2>;
+    case 3: return score_max_kernel<4, NF, 1, F16, IL, true, 3>;
+    case 4: return score_max_kernel<4, NF, 1, F16, IL, true, 4>;
+    case 5: return score_max_kernel<4, NF, 1, F16, IL, true, 5>;
+    case 6: return score_max_kernel<4, NF, 1, F16, IL, true, 6>;
+    default: return score_max_kernel<4, NF, 1, F16, IL, true, 0>;
+  }
+}
+
 template <int NCH, bool F16, bool IL>
-MaxKernel pick_max_chunks(int nk, int nf, bool one_tile) {
-  if (one_tile) {  // head_dim 128, one chunk per query head, no tail chunks
+MaxKernel pick_max_chunks(int nk, int nf, bool lean, int heads) {
+  if (lean) {  // head_dim 128, one chunk per query head, no tail chunks
     if (NCH != 1 || nk != 4) return nullptr;
-    return nf == 1 ? score_max_kernel<4, 1, 1, F16, IL, true> : nf == 2 ? score_max_kernel<4, 2, 1, F16, IL, true> : nullptr;
+    return nf == 1 ? pick_max_heads<1, F16, IL>(heads) : nf == 2 ? pick_max_heads<2, F16, IL>(heads) : nullptr;
   }
   switch (nk * 16 + nf) {
-    case 2 * 16 + 1: return score_max_kernel<2, 1, NCH, F16, IL, false>;
-    case 4 * 16 + 1: return score_max_kernel<4, 1, NCH, F16, IL, false>;
-    case 4 * 16 + 2: return score_max_kernel<4, 2, NCH, F16, IL, false>;
-    case 8 * 16 + 1: return score_max_kernel<8, 1, NCH, F16, IL, false>;
-    case 8 * 16 + 2: return score_max_kernel<8, 2, NCH, F16, IL, false>;
-    case 8 * 16 + 4: return score_max_kernel<8, 4, NCH, F16, IL, false>;
+    case 2 * 16 + 1: return score_max_kernel<2, 1, NCH, F16, IL, false, 0>;
+    case 4 * 16 + 1: return score_max_kernel<4, 1, NCH, F16, IL, false, 0>;
+    case 4 * 16 + 2: return score_max_kernel<4, 2, NCH, F16, IL, false, 0>;
+    case 8 * 16 + 1: return score_max_kernel<8, 1, NCH, F16, IL, false, 0>;
+    case 8 * 16 + 2: return score_max_kernel<8, 2, NCH, F16, IL, false, 0>;
+    case 8 * 16 + 4: return score_max_kernel<8, 4, NCH, F16, IL, false, 0>;
     default: return nullptr;
   }
 }
 
 template <bool F16, bool IL>
-MaxKernel pick_max_typed(int nk, int nf, int nch, bool one_tile) {
-  if (nch == 1) return pick_max_chunks<1, F16, IL>(nk, nf, one_tile);
-  if (nch == 2) return pick_max_chunks<2, F16, IL>(nk, nf, one_tile);
+MaxKernel pick_max_typed(int nk, int nf, int nch, bool lean, int heads) {
+  if (nch == 1) return pick_max_chunks<1, F16, IL>(nk, nf, lean, heads);
+  if (nch == 2) return pick_max_chunks<2, F16, IL>(nk, nf, lean, heads);
   return nullptr;
 }
 
@@ -857,15 +885,8 @@ int launch_max_scorer(hipStream_t stream, const ScoreShape& s, int dtype, int n_
       geo.tail_base = cols_total * nr * 128;
     }
   }
-  // One tile per pass at three waves per SIMD where that measured faster: 128
-  // dims with one chunk per query head and no tail (16 offsets, Qwen2.5-14B
-  // shape: 1.03 against 1.13 ms; with a tail chunk it is 9% slower).
-  const bool one_tile = nk == 4 && nch == 1 && geo.tail_n == 0;
-  MaxKernel kern =
-      f16 ? (fa.interleaved ? pick_max_typed<true, true>(nk, nf, nch, one_tile) : pick_max_typed<true, false>(nk, nf, nch, one_tile))
-          : (fa.interleaved ? pick_max_typed<false, true>(nk, nf, nch, one_tile)
-                            : pick_max_typed<false, false>(nk, nf, nch, one_tile));
-  if (!kern) return fail(KVC_EINVAL, "kvc_score_paged_max: no scorer for head_dim %d rotary_dim %d", s.head_dim, s.rotary_dim);
+  // The lean form serves 128 dims with one chunk per query head and no tail.
+  const bool lean = nk == 4 && nch == 1 && geo.tail_n == 0;
   const int per_g = geo.nch * nr * 2 * kOffsetFragBytes;
   int gpg = kMaxFragLds / per_g;
   if (geo.tail_n > 0) gpg = s.qpk;
@@ -875,6 +896,12 @@ int launch_max_scorer(hipStream_t stream, const ScoreShape& s, int dtype, int n_
   if (gpg > s.qpk) gpg = s.qpk;
   geo.groups = (s.qpk + gpg - 1) / gpg;
   geo.gpg = (s.qpk + geo.groups - 1) / geo.groups;
+  const int heads = geo.groups == 1 ? s.qpk : 0;
+  MaxKernel kern = f16 ? (fa.interleaved ? pick_max_typed<true, true>(nk, nf, nch, lean, heads)
+                                         : pick_max_typed<true, false>(nk, nf, nch, lean, heads))
+                       : (fa.interleaved ? pick_max_typed<false, true>(nk, nf, nch, lean, heads)
+                                         : pick_max_typed<false, false>(nk, nf, nch, lean, heads));
+  if (!kern) return fail(KVC_EINVAL, "kvc_score_paged_max: no scorer for head_dim %d rotary_dim %d", s.head_dim, s.rotary_dim);
   const int64_t items = ceil_div(s.max_tiles, kMaxSpans) * s.kv_heads;
   const int64_t gx = ceil_div(items, 8) * 8 * geo.groups;
   if (gx > 0x7fffffff) return fail(KVC_EINVAL, "kvc_score_paged_max: grid too large");
