@@ -535,6 +535,41 @@ def test_aggregate_finalize_non_finite_matches_oracle(hip_device, layer_mode) ->
 
 
 @pytest.mark.parametrize("layer_mode", ["mean", "max"])
+@pytest.mark.parametrize("layers,heads", [(1, 4), (3, 16), (2, 20), (5, 32), (4, 64)])
+def test_aggregate_whole_rows_match_single_floats(hip_device, layers, heads, layer_mode) -> None:
+    """Token-major rows of whole 16-byte words against the same scores shifted
+    by one float (read one by one): idle lanes, odd layer counts, several turns
+    over the heads, ragged tails, NaN and infinite scores, layer maxima."""
+    from kvcompress_mi355x import _native
+    from kvcompress_mi355x.methods.triattention import _device as dev
+
+    g = torch.Generator().manual_seed(layers * 100 + heads)
+    lens = [1, 63, 200]
+    total = sum(lens)
+    raw = torch.randn(layers, total, heads, generator=g)
+    raw[0, 3, heads - 1], raw[layers - 1, 70, 0], raw[0, 100, 1] = float("nan"), float("inf"), float("-inf")
+    mean = torch.randn(layers, len(lens), heads, generator=g).to(hip_device)
+    var = torch.rand(layers, len(lens), heads, generator=g).to(hip_device)
+    seq_lens = torch.tensor(lens, dtype=torch.int32, device=hip_device)
+    tok_off = torch.tensor([0, 1, 64, total], dtype=torch.int64, device=hip_device)
+    shifted = torch.empty(raw.numel() + 1, device=hip_device)
+    shifted[1:] = raw.flatten().to(hip_device)
+    mode = _native.LAYER_MEAN if layer_mode == "mean" else _native.LAYER_MAX
+    out = []
+    for base in (raw.to(hip_device), shifted[1:]):
+        agg = torch.full((total + 1,), 5.0, device=hip_device)
+        per_layer = torch.full((layers, total), 5.0, device=hip_device)
+        head = (dev.stream_handle(hip_device), layers, heads, len(lens), max(lens), dev.ptr(seq_lens), dev.ptr(tok_off),
+                dev.ptr(base), total * heads, heads, 1, dev.ptr(mean), dev.ptr(var), len(lens) * heads, heads)
+        _native.call("kvc_aggregate", *head, mode, _native.AGG_FINALIZE, dev.ptr(agg))
+        _native.call("kvc_layer_head_max", *head, 0, dev.ptr(per_layer), total)
+        out.append((agg.cpu(), per_layer.cpu()))
+    assert float(out[0][0][total]) == 5.0
+    torch.testing.assert_close(out[0][0], out[1][0], rtol=0, atol=0, equal_nan=True)
+    torch.testing.assert_close(out[0][1], out[1][1], rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("layer_mode", ["mean", "max"])
 @pytest.mark.parametrize("layers,heads", [(1, 17), (3, 7), (6, 40), (2, 1), (8, 64), (64, 33)])
 def test_aggregate_few_tokens_bit_identical(hip_device, layers, heads, layer_mode) -> None:
     # Batches of few tokens share 32 tokens between a workgroup's waves; a

@@ -495,6 +495,76 @@ __device__ __forceinline__ float quad_max_nan(float v) {
   return v;
 }
 
+// Token-major scores whose rows are whole, aligned 16-byte words: L lanes a
+// token, each reading four adjacent heads at a time, two tokens and two layers
+// in flight, so a wave instruction covers whole rows and a mean or scale word
+// serves eight scores.  The one-float form below reads 16 tokens x 4 heads an
+// instruction, one layer after the other: 18.0 us for 8 x 2k-16k tokens x 4
+// layers x 32 heads (33 MB), 15.2 here, a third of it the divisions.
+template <int L>
+__global__ __launch_bounds__(kAggThreads) void aggregate_rows_kernel(AggArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float dyn[];
+  constexpr int kSlots = kAggThreads / L;
+  const int n_stats = a.n_layers * a.n_heads;
+  const int b = blockIdx.y;
+  const int n = a.seq_lens[b];
+  if (static_cast<int64_t>(blockIdx.x) * 2 * kSlots >= n) return;
+  load_layer_stats(a, b, dyn, dyn + n_stats);
+  __syncthreads();
+  const int q = threadIdx.x & (L - 1);
+  const int t0 = blockIdx.x * 2 * kSlots + threadIdx.x / L;
+  const bool rsqrt_form = (a.flags & KVC_AGG_RSQRT) != 0;
+  int64_t tok[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) tok[i] = a.token_offsets[b] + min(t0 + i * kSlots, n - 1);
+  float total[2] = {0.0f, 0.0f};
+  for (int l0 = 0; l0 < a.n_layers; l0 += 2) {
+    float best[2][2];  // [layer][token]
+#pragma unroll
+    for (int d = 0; d < 2; ++d) best[d][0] = best[d][1] = -INFINITY;
+    for (int h = 4 * q; h < a.n_heads; h += 4 * L) {
+      float4 x[2][2];
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          x[d][i] = *reinterpret_cast<const float4*>(a.raw + min(l0 + d, a.n_layers - 1) * a.raw_layer_stride +
+                                                     tok[i] * a.raw_token_stride + h);
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        const int at = min(l0 + d, a.n_layers - 1) * a.n_heads + h;
+        const float4 m = *reinterpret_cast<const float4*>(dyn + at);
+        const float4 s = *reinterpret_cast<const float4*>(dyn + n_stats + at);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          best[d][i] = max_nan(best[d][i], normalise(x[d][i].x, m.x, s.x, rsqrt_form));
+          best[d][i] = max_nan(best[d][i], normalise(x[d][i].y, m.y, s.y, rsqrt_form));
+          best[d][i] = max_nan(best[d][i], normalise(x[d][i].z, m.z, s.z, rsqrt_form));
+          best[d][i] = max_nan(best[d][i], normalise(x[d][i].w, m.w, s.w, rsqrt_form));
+        }
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      if (l0 + d >= a.n_layers) break;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float v = quad_max_nan(best[d][i]);
+        if (L == 8) v = max_nan(v, dpp_row_half_mirror(v));
+        if (a.layer_out_stride) {
+          if (q == 0 && t0 + i * kSlots < n) a.agg[(l0 + d) * a.layer_out_stride + tok[i]] = v;
+        } else {
+          total[i] = combine_layers(total[i], v, l0 + d, a, tok[i]);
+        }
+      }
+    }
+  }
+  if (q != 0 || a.layer_out_stride) return;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (t0 + i * kSlots < n) a.agg[tok[i]] = finalize(total[i], a);
+}
+
 __global__ __launch_bounds__(kAggThreads) void aggregate_kernel(AggArgs a) {
   extern __shared__ float dyn[];
   float* s_mean = dyn;
@@ -1006,6 +1076,14 @@ int launch_aggregate(const char* who, kvc_stream_t stream, int n_layers, int n_h
     }
     dim3 grid(static_cast<unsigned>(ceil_div(max_seq_len, kAggTokPerBlock)), static_cast<unsigned>(n_seq));
     aggregate_tokens_kernel<<<grid, kAggThreads, lds, as_stream(stream)>>>(aa);
+    return launch_status(who);
+  }
+  if (raw_head_stride == 1 && n_heads % 4 == 0 && raw_token_stride % 4 == 0 && raw_layer_stride % 4 == 0 &&
+      reinterpret_cast<uintptr_t>(raw) % 16 == 0) {
+    // Four lanes hold 16 heads of a token; past that eight, in turns past 32.
+    const int lanes = n_heads <= 16 ? 4 : 8;
+    dim3 grid(static_cast<unsigned>(ceil_div(max_seq_len, 2 * kAggThreads / lanes)), static_cast<unsigned>(n_seq));
+    (lanes == 4 ? aggregate_rows_kernel<4> : aggregate_rows_kernel<8>)<<<grid, kAggThreads, lds, as_stream(stream)>>>(aa);
     return launch_status(who);
   }
   dim3 grid(static_cast<unsigned>(ceil_div(max_seq_len, kAggTokensPerBlock)), static_cast<unsigned>(n_seq));
