@@ -178,6 +178,20 @@ int kvc_head_stats(kvc_stream_t stream, int n_layers, int kv_heads, int head_dim
                    int qpk, int n_seq, int max_seq_len, const int32_t* seq_lens,
                    const void* workspace, size_t workspace_bytes, float* mean, float* var);
 
+/* kvc_mean_phases, kvc_score_paged and kvc_head_stats of one batch in one call,
+ * the phases formed by the launch that folds the weights (phase_cos, phase_sin:
+ * [n_seq][n_layers][rotary_dim/2], written as kvc_mean_phases does).  Same
+ * arguments, checks and results as the three.  No counterpart in the reference. */
+int kvc_score_batch(kvc_stream_t stream, int dtype, int n_layers, const uint64_t* k_layer_ptrs, int64_t num_pages,
+                    int64_t page_stride, int kv_heads, int head_dim, int rotary_dim, int qpk, int rope_style,
+                    int n_seq, int max_seq_len, const int32_t* seq_lens, const int64_t* token_offsets,
+                    const int64_t* block_offsets, const int64_t* block_ids, const float* q_real,
+                    const float* q_imag, const float* freq_scale, const float* extra_coef,
+                    const float* q_pass, const int64_t* round_starts, const float* offsets, int n_offsets,
+                    const float* omega, float* phase_cos, float* phase_sin, float* raw,
+                    int64_t raw_layer_stride, int64_t raw_token_stride, int64_t raw_head_stride,
+                    void* workspace, size_t workspace_bytes, float* mean, float* var);
+
 /* kvc_score_paged followed by kvc_head_stats, with the scorer's scratch (folded
  * weights and per-tile partial sums) in a static 64 MiB device array that the
  * library holds on every device it runs on until the process ends, instead of

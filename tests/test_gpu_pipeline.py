@@ -390,3 +390,40 @@ def test_batch_descriptors_of_one_copy(hip_device, n_seq) -> None:
     with pytest.raises(RuntimeError, match="capture"):
         with torch.cuda.graph(graph, stream=stream):
             Batch.build(hip_device, lens, starts, device_tables)
+
+
+@pytest.mark.parametrize("shape", [(8, 2, 128, 128, torch.bfloat16), (12, 4, 96, 96, torch.float16), (8, 1, 192, 192, torch.bfloat16),
+                                   (16, 2, 256, 256, torch.bfloat16)])
+def test_batch_scoring_equals_its_three_calls(hip_device, shape) -> None:
+    """kvc_score_batch against kvc_mean_phases, kvc_score_paged and
+    kvc_head_stats on the same batch, bit for bit (matrix-core shapes of two and
+    three words, the vector scorer, heads split over workgroups and not)."""
+    from kvcompress_mi355x import _native, workloads
+    from kvcompress_mi355x.methods.triattention import _device as dev
+
+    heads, kv, dim, rotary, dtype = shape
+    spec = workloads.config_spec(2, n_layers=3, score_layer_stride=1, seq_lens=(1500, 700, 2049), budget=512, recent=64, head_dim=dim,
+                                 rotary_dim=rotary, num_attention_heads=heads, num_kv_heads=kv, max_model_len=65536)
+    cache = workloads.build_synthetic_cache(spec, hip_device, seed=7)
+    if dtype != cache.k_caches[0].dtype:
+        cache.k_caches = [c.to(dtype) for c in cache.k_caches]
+        cache.v_caches = [c.to(dtype) for c in cache.v_caches]
+    p, batch = workloads.build_pipeline(cache)
+    p.raw.fill_(3.0)
+    p.score(batch)
+    got = [t.clone() for t in (p.phase_cos, p.phase_sin, p.raw, *p.head_statistics(batch))]
+    t, stream, n = p.tables, dev.stream_handle(p.device), batch.n_seq
+    p.raw.fill_(3.0)
+    p.phase_cos.zero_()
+    _native.call("kvc_mean_phases", stream, n, t.n_layers, t.freq, dev.ptr(batch.round_starts), dev.ptr(t.offsets), t.offsets.numel(),
+                 dev.ptr(t.omega), dev.ptr(p.phase_cos), dev.ptr(p.phase_sin))
+    size = (t.n_layers, p.kv_heads, p.head_dim, t.rotary_dim, t.qpk)
+    _native.call("kvc_score_paged", stream, dev.cache_dtype_code(p.dtype), t.n_layers, dev.ptr(p.scoring_ptrs), p.num_pages, p.page_stride,
+                 *size[1:], dev.rope_style_code(t.rope_style), n, max(batch.seq_lens_host), dev.ptr(batch.seq_lens),
+                 dev.ptr(batch.token_offsets), dev.ptr(batch.src_offsets), dev.ptr(batch.src_ids), dev.ptr(t.q_real), dev.ptr(t.q_imag),
+                 dev.ptr(t.freq_scale), dev.ptr(t.extra), dev.ptr(t.q_pass), dev.ptr(p.phase_cos), dev.ptr(p.phase_sin),
+                 t.n_layers * t.freq, dev.ptr(p.raw), *p.raw_strides(), dev.ptr(p.workspace), p.workspace_bytes)
+    _native.call("kvc_head_stats", stream, *size, n, max(batch.seq_lens_host), dev.ptr(batch.seq_lens), dev.ptr(p.workspace),
+                 p.workspace_bytes, dev.ptr(p.mean), dev.ptr(p.var))
+    for have, want in zip(got, (p.phase_cos, p.phase_sin, p.raw, *p.head_statistics(batch))):
+        assert torch.equal(have, want)

@@ -72,8 +72,13 @@ extern "C" int kvc_score_paged_noalloc(kvc_stream_t stream, int dtype, int n_lay
                                        int64_t raw_token_stride, int64_t raw_head_stride, float* mean, float* var) {
   // Size and output checks come first: nothing is launched for a call that is
   // going to be rejected.
-  const size_t need = kvc_score_workspace_bytes(n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq, max_seq_len);
-  if (need == 0) return fail(KVC_EINVAL, "kvc_score_paged_noalloc: unsupported shape");
+  ScoreShape s;
+  if (!make_shape(&s, n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq, max_seq_len))
+    return fail(KVC_EINVAL, "kvc_score_paged_noalloc: unsupported shape");
+  // The matrix cores' three words a weight take more room than the vector
+  // scorer's floats; a batch that only the latter fit is scored by it.
+  s.vector_only = workspace_bytes(s) > kNoallocScratchBytes;
+  const size_t need = workspace_bytes(s);
   if (need > kNoallocScratchBytes)
     return fail(KVC_EINVAL,
                 "kvc_score_paged_noalloc: this batch needs %zu bytes of scratch, more than the %zu bytes (64 MiB) "
@@ -86,12 +91,12 @@ extern "C" int kvc_score_paged_noalloc(kvc_stream_t stream, int dtype, int n_lay
   // Nothing in the scratch has to start at zero: the fold writes every weight
   // the scorer reads, the scorer writes the partial sums of every tile that
   // holds tokens, and kvc_head_stats reads only those tiles.
-  if (int rc = kvc_score_paged(stream, dtype, n_layers, k_layer_ptrs, num_pages, page_stride, kv_heads, head_dim,
+  if (int rc = score_paged(s.vector_only, nullptr, stream, dtype, n_layers, k_layer_ptrs, num_pages, page_stride, kv_heads, head_dim,
                                rotary_dim, qpk, rope_style, n_seq, max_seq_len, seq_lens, token_offsets, block_offsets,
                                block_ids, q_real, q_imag, freq_scale, extra_coef, q_pass, phase_cos, phase_sin,
                                phase_seq_stride, raw, raw_layer_stride, raw_token_stride, raw_head_stride, ws,
                                kNoallocScratchBytes))
     return rc;
-  return kvc_head_stats(stream, n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq, max_seq_len, seq_lens, ws,
+  return head_stats(s.vector_only, stream, n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq, max_seq_len, seq_lens, ws,
                         kNoallocScratchBytes, mean, var);
 }

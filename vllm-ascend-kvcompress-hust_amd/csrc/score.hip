@@ -37,17 +37,8 @@ namespace {
 
 // ------------------------------------------------------------- phase tables --
 
-// One group of `width` lanes (the offset count rounded up to a power of two,
-// at most 32) per (sequence, layer, frequency); lane o evaluates offset o (then
-// o + width, ...), so a thread waits for one cosine/sine instead of one per
-// offset.  The phase argument is formed exactly as the torch path does in
-// float32, (offset + round_start) * omega, and its cosine/sine are evaluated in
-// double and rounded once, so the table agrees with a correctly rounded float32
-// evaluation.  Lane 0 of the group sums the rounded values sequentially in
-// offset order in float32 and divides by the offset count, as the torch path's
-// mean over the offset axis.
-constexpr int kPhaseMaxLanes = 32;
-
+// One group of `width` lanes per (sequence, layer, frequency), so a thread
+// waits for one cosine/sine instead of one per offset (mean_phase).
 __global__ __launch_bounds__(256) void mean_phases_kernel(int n_seq, int n_layers, int n_freq, int width,
                                                           const int64_t* __restrict__ round_starts,
                                                           const float* __restrict__ offsets, int n_offsets,
@@ -58,28 +49,10 @@ __global__ __launch_bounds__(256) void mean_phases_kernel(int n_seq, int n_layer
   const int64_t per_seq = static_cast<int64_t>(n_layers) * n_freq;
   if (idx >= per_seq * n_seq) return;  // the whole lane group leaves together
   const int64_t b = idx / per_seq;
-  const int64_t lf = idx - b * per_seq;
-  const float rs = static_cast<float>(round_starts[b]);
-  const float w = omega[lf];
-  float c = 0.0f, s = 0.0f;
-  for (int o0 = 0; o0 < n_offsets; o0 += width) {
-    const int o = o0 + lane;
-    float co = 0.0f, so = 0.0f;
-    if (o < n_offsets) {
-      const float x = __fmul_rn(__fadd_rn(offsets[o], rs), w);
-      co = static_cast<float>(cos(static_cast<double>(x)));
-      so = static_cast<float>(sin(static_cast<double>(x)));
-    }
-    const int count = min(width, n_offsets - o0);
-    for (int j = 0; j < count; ++j) {
-      c = __fadd_rn(c, __shfl(co, j, width));
-      s = __fadd_rn(s, __shfl(so, j, width));
-    }
-  }
+  const float2 m = mean_phase(lane, width, static_cast<float>(round_starts[b]), omega[idx - b * per_seq], offsets, n_offsets);
   if (lane == 0) {
-    const float n = static_cast<float>(n_offsets);
-    phase_cos[idx] = __fdiv_rn(c, n);
-    phase_sin[idx] = __fdiv_rn(s, n);
+    phase_cos[idx] = m.x;
+    phase_sin[idx] = m.y;
   }
 }
 
@@ -784,8 +757,7 @@ extern "C" int kvc_mean_phases(kvc_stream_t stream, int n_seq, int n_layers, int
   if (!round_starts || !offsets || !omega || !phase_cos || !phase_sin)
     return fail(KVC_EINVAL, "kvc_mean_phases: null pointer");
   const int64_t total = static_cast<int64_t>(n_seq) * n_layers * n_freq;
-  int width = 1;
-  while (width < n_offsets && width < kPhaseMaxLanes) width <<= 1;
+  const int width = phase_lanes(n_offsets);
   if (ceil_div(total * width, 256) > 0x7fffffff) return fail(KVC_EINVAL, "kvc_mean_phases: grid too large");
   mean_phases_kernel<<<static_cast<unsigned>(ceil_div(total * width, 256)), 256, 0, as_stream(stream)>>>(
       n_seq, n_layers, n_freq, width, round_starts, offsets, n_offsets, omega, phase_cos, phase_sin);
@@ -844,7 +816,7 @@ namespace {
 // Checks and argument blocks shared by kvc_score_paged and kvc_score_paged_max.
 // `phase_bytes_ok` is false when the caller's phase tables cannot be read by
 // this entry (checked by the caller).  Returns 0 or a C-ABI error code.
-int score_setup(const char* who, int dtype, int n_layers, const uint64_t* k_layer_ptrs, int64_t num_pages,
+int score_setup(const char* who, bool vector_only, int dtype, int n_layers, const uint64_t* k_layer_ptrs, int64_t num_pages,
                 int64_t page_stride, int kv_heads, int head_dim, int rotary_dim, int qpk, int rope_style, int n_seq,
                 int max_seq_len, const int32_t* seq_lens, const int64_t* token_offsets, const int64_t* block_offsets,
                 const int64_t* block_ids, const float* q_real, const float* q_imag, const float* freq_scale,
@@ -858,6 +830,7 @@ int score_setup(const char* who, int dtype, int n_layers, const uint64_t* k_laye
                 "rotary_dim=%d qpk=%d n_seq=%d); rotary_dim and head_dim-rotary_dim must be "
                 "multiples of 16, qpk <= 8",
                 who, n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq);
+  s->vector_only = vector_only;
   if (dtype != KVC_DTYPE_BF16 && dtype != KVC_DTYPE_FP16)
     return fail(KVC_EINVAL, "%s: dtype must be bf16 or fp16", who);
   if (rope_style != KVC_ROPE_HALF && rope_style != KVC_ROPE_INTERLEAVED)
@@ -922,7 +895,7 @@ int score_setup(const char* who, int dtype, int n_layers, const uint64_t* k_laye
 }  // namespace
 }  // namespace kvc
 
-extern "C" int kvc_score_paged(kvc_stream_t stream, int dtype, int n_layers,
+int kvc::score_paged(bool vector_only, const PhaseArgs* phases, kvc_stream_t stream, int dtype, int n_layers,
                                const uint64_t* k_layer_ptrs, int64_t num_pages,
                                int64_t page_stride, int kv_heads, int head_dim, int rotary_dim,
                                int qpk, int rope_style, int n_seq, int max_seq_len,
@@ -938,18 +911,24 @@ extern "C" int kvc_score_paged(kvc_stream_t stream, int dtype, int n_layers,
   FoldArgs fa;
   ScoreArgs sa;
   const size_t need = make_shape(&s, n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq, max_seq_len)
-                          ? workspace_bytes(s)
+                          ? (s.vector_only = vector_only, workspace_bytes(s))
                           : 0;
-  if (int rc = score_setup("kvc_score_paged", dtype, n_layers, k_layer_ptrs, num_pages, page_stride, kv_heads,
+  if (int rc = score_setup("kvc_score_paged", vector_only, dtype, n_layers, k_layer_ptrs, num_pages, page_stride, kv_heads,
                            head_dim, rotary_dim, qpk, rope_style, n_seq, max_seq_len, seq_lens, token_offsets,
                            block_offsets, block_ids, q_real, q_imag, freq_scale, extra_coef, q_pass, phase_cos,
                            phase_sin, phase_seq_stride, raw, raw_layer_stride, raw_token_stride, raw_head_stride,
                            workspace, workspace_bytes_given, need, &s, &fa, &sa))
     return rc;
+  const bool matrix = mfma_scorer_supported(s, dtype, rope_style);
+  if (phases && (s.max_tiles == 0 || !matrix)) {
+    if (int rc = kvc_mean_phases(stream, n_seq, n_layers, s.freq, phases->round_starts, phases->offsets,
+                                 phases->n_offsets, phases->omega, phases->phase_cos, phases->phase_sin))
+      return rc;
+  }
   if (s.max_tiles == 0) return 0;
   hipStream_t st = as_stream(stream);
 
-  if (mfma_scorer_supported(s, dtype, rope_style)) return launch_mfma_scorer(st, s, dtype, fa, sa, workspace);
+  if (matrix) return launch_mfma_scorer(st, s, dtype, phases, fa, sa, workspace);
 
   const int64_t fold_threads = static_cast<int64_t>(n_seq) * n_layers * kv_heads * s.units;
   fold_weights_kernel<<<static_cast<unsigned>(ceil_div(fold_threads, 64)), 64, 0, st>>>(fa);
@@ -969,6 +948,25 @@ extern "C" int kvc_score_paged(kvc_stream_t stream, int dtype, int n_layers,
     return fail(KVC_EINVAL, "kvc_score_paged: too many sequences or layers for one launch");
   kern<<<grid, kScoreThreads, 0, st>>>(sa);
   return launch_status("kvc_score_paged");
+}
+
+extern "C" int kvc_score_paged(kvc_stream_t stream, int dtype, int n_layers,
+                               const uint64_t* k_layer_ptrs, int64_t num_pages,
+                               int64_t page_stride, int kv_heads, int head_dim, int rotary_dim,
+                               int qpk, int rope_style, int n_seq, int max_seq_len,
+                               const int32_t* seq_lens, const int64_t* token_offsets,
+                               const int64_t* block_offsets, const int64_t* block_ids,
+                               const float* q_real, const float* q_imag, const float* freq_scale,
+                               const float* extra_coef, const float* q_pass,
+                               const float* phase_cos, const float* phase_sin,
+                               int64_t phase_seq_stride, float* raw, int64_t raw_layer_stride,
+                               int64_t raw_token_stride, int64_t raw_head_stride, void* workspace,
+                               size_t workspace_bytes_given) {
+    return score_paged(false, nullptr, stream, dtype, n_layers, k_layer_ptrs, num_pages, page_stride, kv_heads,
+                     head_dim, rotary_dim, qpk, rope_style, n_seq, max_seq_len, seq_lens, token_offsets,
+                     block_offsets, block_ids, q_real, q_imag, freq_scale, extra_coef, q_pass, phase_cos, phase_sin,
+                     phase_seq_stride, raw, raw_layer_stride, raw_token_stride, raw_head_stride, workspace,
+                     workspace_bytes_given);
 }
 
 extern "C" size_t kvc_score_max_workspace_bytes(int n_layers, int kv_heads, int head_dim, int rotary_dim, int qpk,
@@ -995,7 +993,7 @@ extern "C" int kvc_score_paged_max(kvc_stream_t stream, int dtype, int n_layers,
   const size_t need = make_shape(&s, n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq, max_seq_len)
                           ? max_workspace_bytes(s, n_offsets)
                           : 0;
-  if (int rc = score_setup("kvc_score_paged_max", dtype, n_layers, k_layer_ptrs, num_pages, page_stride, kv_heads,
+  if (int rc = score_setup("kvc_score_paged_max", false, dtype, n_layers, k_layer_ptrs, num_pages, page_stride, kv_heads,
                            head_dim, rotary_dim, qpk, rope_style, n_seq, max_seq_len, seq_lens, token_offsets,
                            block_offsets, block_ids, q_real, q_imag, freq_scale, extra_coef, q_pass, offset_cos,
                            offset_sin, phase_seq_stride, raw, raw_layer_stride, raw_token_stride, raw_head_stride,
@@ -1009,13 +1007,14 @@ extern "C" int kvc_score_paged_max(kvc_stream_t stream, int dtype, int n_layers,
   return launch_max_scorer(as_stream(stream), s, dtype, n_offsets, fa, sa, workspace);
 }
 
-extern "C" int kvc_head_stats(kvc_stream_t stream, int n_layers, int kv_heads, int head_dim,
+int kvc::head_stats(bool vector_only, kvc_stream_t stream, int n_layers, int kv_heads, int head_dim,
                               int rotary_dim, int qpk, int n_seq, int max_seq_len,
                               const int32_t* seq_lens, const void* workspace,
                               size_t workspace_bytes_given, float* mean, float* var) {
   ScoreShape s;
   if (!make_shape(&s, n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq, max_seq_len))
     return fail(KVC_EINVAL, "kvc_head_stats: unsupported shape");
+  s.vector_only = vector_only;
   if (!seq_lens || !workspace || !mean || !var)
     return fail(KVC_EINVAL, "kvc_head_stats: null pointer");
   if (workspace_bytes_given < workspace_bytes(s))
@@ -1027,6 +1026,36 @@ extern "C" int kvc_head_stats(kvc_stream_t stream, int n_layers, int kv_heads, i
   head_stats_kernel<<<static_cast<unsigned>(ceil_div(total * 64, 256)), 256, 0, as_stream(stream)>>>(
       n_layers, n_seq, n_heads, s.max_tiles > 0 ? s.max_tiles : 1, seq_lens, partials, mean, var);
   return launch_status("kvc_head_stats");
+}
+
+extern "C" int kvc_head_stats(kvc_stream_t stream, int n_layers, int kv_heads, int head_dim,
+                              int rotary_dim, int qpk, int n_seq, int max_seq_len,
+                              const int32_t* seq_lens, const void* workspace,
+                              size_t workspace_bytes_given, float* mean, float* var) {
+    return head_stats(false, stream, n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq, max_seq_len, seq_lens,
+                    workspace, workspace_bytes_given, mean, var);
+}
+
+extern "C" int kvc_score_batch(kvc_stream_t stream, int dtype, int n_layers, const uint64_t* k_layer_ptrs, int64_t num_pages,
+                              int64_t page_stride, int kv_heads, int head_dim, int rotary_dim, int qpk, int rope_style,
+                              int n_seq, int max_seq_len, const int32_t* seq_lens, const int64_t* token_offsets,
+                              const int64_t* block_offsets, const int64_t* block_ids, const float* q_real,
+                              const float* q_imag, const float* freq_scale, const float* extra_coef,
+                              const float* q_pass, const int64_t* round_starts, const float* offsets, int n_offsets,
+                              const float* omega, float* phase_cos, float* phase_sin, float* raw,
+                              int64_t raw_layer_stride, int64_t raw_token_stride, int64_t raw_head_stride,
+                              void* workspace, size_t workspace_bytes_given, float* mean, float* var) {
+  if (n_offsets <= 0) return fail(KVC_EINVAL, "kvc_score_batch: n_offsets must be positive");
+  if (!round_starts || !offsets || !omega || !mean || !var) return fail(KVC_EINVAL, "kvc_score_batch: null pointer");
+  const PhaseArgs phases = {round_starts, offsets, n_offsets, omega, phase_cos, phase_sin};
+  if (int rc = score_paged(false, &phases, stream, dtype, n_layers, k_layer_ptrs, num_pages, page_stride, kv_heads,
+                           head_dim, rotary_dim, qpk, rope_style, n_seq, max_seq_len, seq_lens, token_offsets,
+                           block_offsets, block_ids, q_real, q_imag, freq_scale, extra_coef, q_pass, phase_cos, phase_sin,
+                           static_cast<int64_t>(n_layers) * (rotary_dim / 2), raw, raw_layer_stride, raw_token_stride,
+                           raw_head_stride, workspace, workspace_bytes_given))
+    return rc;
+  return head_stats(false, stream, n_layers, kv_heads, head_dim, rotary_dim, qpk, n_seq, max_seq_len, seq_lens, workspace,
+                    workspace_bytes_given, mean, var);
 }
 
 namespace kvc {

@@ -1,6 +1,8 @@
 // Scorer definitions shared by the VALU (score.hip) and MFMA (score_mfma.hip) kernels.
 #pragma once
 
+#include <math.h>
+
 #include "kvc_common.h"
 
 namespace kvc {
@@ -51,6 +53,7 @@ struct ScoreShape {
   int n_layers, kv_heads, head_dim, rotary_dim, qpk;
   int freq, pass, units_rot, units, group_shift;
   int n_seq, max_tiles;
+  bool vector_only;  // three-word shapes: the vector scorer and its smaller weights
 };
 
 inline bool make_shape(ScoreShape* s, int n_layers, int kv_heads, int head_dim, int rotary_dim, int qpk,
@@ -80,6 +83,7 @@ inline bool make_shape(ScoreShape* s, int n_layers, int kv_heads, int head_dim, 
   // token slot stay idle.
   const int groups_per_wg = (kScoreThreads / 64) * (64 >> shift);
   if (groups_per_wg < kv_heads) return false;
+  s->vector_only = false;
   s->n_seq = n_seq;
   s->max_tiles = static_cast<int>(ceil_div(max_seq_len, kScoreTile));
   return true;
@@ -108,7 +112,7 @@ inline bool mfma_two_words(const ScoreShape& s) {
          (s.freq == 32 || s.freq == 64 || s.freq == 128);
 }
 inline bool mfma_shape(const ScoreShape& s) {
-  return mfma_two_words(s) || (s.head_dim <= 256 && s.rotary_dim <= 128);
+  return mfma_two_words(s) || (!s.vector_only && s.head_dim <= 256 && s.rotary_dim <= 128);
 }
 inline MfmaSteps mfma_steps(const ScoreShape& s) {
   MfmaSteps m;
@@ -177,6 +181,53 @@ struct FoldArgs {
   float* weights;  // [n_seq][n_layers][kv_heads][units][3][qpk][8]
 };
 
+// Where a call also forms the mean phases it folds (kvc_mean_phases' arguments).
+struct PhaseArgs {
+  const int64_t* round_starts;
+  const float* offsets;
+  int n_offsets;
+  const float* omega;
+  float* phase_cos;  // [n_seq][n_layers][F]
+  float* phase_sin;
+};
+
+// Lanes a phase mean is spread over: the offset count rounded up to a power of
+// two, at most 32.
+constexpr int kPhaseMaxLanes = 32;
+inline int phase_lanes(int n_offsets) {
+  int width = 1;
+  while (width < n_offsets && width < kPhaseMaxLanes) width <<= 1;
+  return width;
+}
+
+// Mean cosine and sine of (offset + round_start) * omega over the offsets, by an
+// aligned group of `width` lanes, each evaluating offsets lane, lane + width,
+// ...  The argument is formed exactly as the torch path does in float32 and its
+// cosine/sine are evaluated in double and rounded once, so the table agrees
+// with a correctly rounded float32 evaluation; the rounded values are summed in
+// offset order in float32 and divided by the offset count, as the torch path's
+// mean over the offset axis.  Every lane of the group returns both.
+__device__ __forceinline__ float2 mean_phase(int lane, int width, float round_start, float omega,
+                                             const float* __restrict__ offsets, int n_offsets) {
+  float c = 0.0f, s = 0.0f;
+  for (int o0 = 0; o0 < n_offsets; o0 += width) {
+    const int o = o0 + lane;
+    float co = 0.0f, so = 0.0f;
+    if (o < n_offsets) {
+      const float x = __fmul_rn(__fadd_rn(offsets[o], round_start), omega);
+      co = static_cast<float>(cos(static_cast<double>(x)));
+      so = static_cast<float>(sin(static_cast<double>(x)));
+    }
+    const int count = min(width, n_offsets - o0);
+    for (int j = 0; j < count; ++j) {
+      c = __fadd_rn(c, __shfl(co, j, width));
+      s = __fadd_rn(s, __shfl(so, j, width));
+    }
+  }
+  const float n = static_cast<float>(n_offsets);
+  return make_float2(__fdiv_rn(c, n), __fdiv_rn(s, n));
+}
+
 struct ScoreArgs {
   const uint64_t* k_layer_ptrs;
   int64_t num_pages, page_stride;
@@ -193,11 +244,25 @@ struct ScoreArgs {
   double* partials;  // [n_layers][n_seq][max_tiles][kv_heads*QPK][2]
 };
 
+// kvc_score_paged and kvc_head_stats (score.hip), with the weight layout and
+// scorer that `vector_only` asks for.  `phases`: form the phase tables as well
+// (phase_cos/phase_sin are then its outputs).
+int score_paged(bool vector_only, const PhaseArgs* phases, kvc_stream_t stream, int dtype, int n_layers, const uint64_t* k_layer_ptrs,
+                int64_t num_pages, int64_t page_stride, int kv_heads, int head_dim, int rotary_dim, int qpk,
+                int rope_style, int n_seq, int max_seq_len, const int32_t* seq_lens, const int64_t* token_offsets,
+                const int64_t* block_offsets, const int64_t* block_ids, const float* q_real, const float* q_imag,
+                const float* freq_scale, const float* extra_coef, const float* q_pass, const float* phase_cos,
+                const float* phase_sin, int64_t phase_seq_stride, float* raw, int64_t raw_layer_stride,
+                int64_t raw_token_stride, int64_t raw_head_stride, void* workspace, size_t workspace_bytes_given);
+int head_stats(bool vector_only, kvc_stream_t stream, int n_layers, int kv_heads, int head_dim, int rotary_dim, int qpk,
+               int n_seq, int max_seq_len, const int32_t* seq_lens, const void* workspace,
+               size_t workspace_bytes_given, float* mean, float* var);
+
 // MFMA scorer (score_mfma.hip): whether it serves this shape, and its launch
 // (weight fold into bf16 or fp16 hi/lo fragments + scoring).  Returns a C-ABI code.
 bool mfma_scorer_supported(const ScoreShape& s, int dtype, int rope_style);
-int launch_mfma_scorer(hipStream_t stream, const ScoreShape& s, int dtype, const FoldArgs& fa, const ScoreArgs& sa,
-                       void* weights);
+int launch_mfma_scorer(hipStream_t stream, const ScoreShape& s, int dtype, const PhaseArgs* phases, const FoldArgs& fa,
+                       const ScoreArgs& sa, void* weights);
 // Max-over-offsets scorer (score_max.hip): fold of the per-offset fragments,
 // magnitude/pass fold (zero_rotary) and scoring.  `fa.phase_cos/phase_sin`
 // are the per-offset tables [n_seq][n_layers][n_offsets][F].

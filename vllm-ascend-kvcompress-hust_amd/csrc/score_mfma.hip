@@ -85,22 +85,22 @@ inline MfmaGeometry geometry(const ScoreShape& s) {
 
 // ---------------------------------------------------------------- fold ------
 
-// One thread per (sequence, layer, KV head, fragment, live lane): the lane's
-// eight bf16 values of one fragment.  Only the lanes of live query heads
-// (g < qpk) are stored, packed as [fragment][kb][g]; the scorer zeroes the
-// B columns of the other lanes, so a wave reads qpk/16 of a full fragment.  Linear weight of head dim d for query head g
+// Fragments hold the eight 16-bit values of each lane of live query heads
+// (g < qpk), packed as [fragment][kb][g]; the scorer zeroes the B columns of
+// the other lanes, so a wave reads qpk/16 of a full fragment.  Weight for query head g
 // (tri/scoring.py:70-81, 117-119 folded with the phase means):
 //   real part of frequency f      : sqrt(fss) (qr c - qi s)
 //   imaginary part of frequency f : sqrt(fss) (qi c + qr s)
 //   pass dim p                    : q_pass[p]
 // Magnitude weight of frequency f: sqrt(fss) * extra.  Fragment terms*j + k
-// holds word k of K step j (linear steps, then magnitude steps): the bf16 of
-// what the words before it leave of the weight.
+// holds word k of K step j (linear steps, then magnitude steps): the rounding
+// of what the words before it leave of the weight.
+//
 // Folded weight of K-step element (step, kb, e) for query head g of
-// (sequence b, layer, KV head): see fold_mfma_kernel.  Elements past the
+// a (sequence, layer, KV head) whose phases are pc, ps.  Elements past the
 // frequencies or the pass dims (dead lanes of a kind's last step) are zero.
-__device__ __forceinline__ float folded_weight(const FoldArgs& a, int nk, int nf, int b, int layer, int64_t row,
-                                              int step, int kb, int e) {
+__device__ __forceinline__ float folded_weight(const FoldArgs& a, const float* pc, const float* ps, int nk, int nf,
+                                              int64_t row, int step, int kb, int e) {
   if (step < 2 * nf) {
     if (a.zero_rotary) return 0.0f;
     // Half style: steps 0 .. nf-1 real, nf .. 2nf-1 imaginary parts of 32
@@ -109,8 +109,6 @@ __device__ __forceinline__ float folded_weight(const FoldArgs& a, int nk, int nf
     const bool real = a.interleaved ? (i & 1) == 0 : step < nf;
     const int f = a.interleaved ? i >> 1 : (step < nf ? i : i - 32 * nf);
     if (f >= a.freq) return 0.0f;
-    const float* pc = a.phase_cos + b * a.phase_seq_stride + static_cast<int64_t>(layer) * a.freq;
-    const float* ps = a.phase_sin + b * a.phase_seq_stride + static_cast<int64_t>(layer) * a.freq;
     const int64_t o = row * a.freq + f;
     const float qr = a.q_real[o], qi = a.q_imag[o], sc = a.scale[o];
     const float c = pc[f], sn = ps[f];
@@ -127,101 +125,144 @@ __device__ __forceinline__ float folded_weight(const FoldArgs& a, int nk, int nf
   return a.scale[o] * a.extra[o];
 }
 
-__global__ void fold_mfma_kernel(FoldArgs a, int nk, int nf, int terms, uint16_t* __restrict__ frags) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int n_frag = terms * (nk + nf);
-  const int packed = 4 * a.qpk;  // live lanes per fragment
-  const int64_t total = static_cast<int64_t>(a.n_seq) * a.n_layers * a.kv_heads * n_frag * packed;
-  if (idx >= total) return;
-  const int pl = static_cast<int>(idx % packed);
-  int64_t r = idx / packed;
-  const int frag = static_cast<int>(r % n_frag);
-  r /= n_frag;
-  const int head = static_cast<int>(r % a.kv_heads);
-  r /= a.kv_heads;
-  const int layer = static_cast<int>(r % a.n_layers);
-  const int b = static_cast<int>(r / a.n_layers);
-  const int g = pl % a.qpk;
-  const int kb = pl / a.qpk;
-  const int64_t row = ((static_cast<int64_t>(layer) * a.kv_heads + head) * a.qpk + g);
-  const int step = frag / terms;
-  const int term = frag - step * terms;
-  uint16_t out[8];
+// The 16-bit words of the eight weights w, word k to dst + k * stride.
+template <bool F16>
+__device__ __forceinline__ void store_words(float (&w)[8], int terms, uint16_t* dst, int64_t stride) {
+  for (int k = 0; k < terms; ++k) {
+    u32x4 out;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    float w = folded_weight(a, nk, nf, b, layer, row, step, kb, e);
-    uint32_t word = bf16_bits(w);
-    for (int k = 0; k < term; ++k) {
-      w -= bf16_value(word);
-      word = bf16_bits(w);
+    for (int i = 0; i < 4; ++i) {
+      uint32_t word = 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float& v = w[2 * i + h];
+        uint32_t bits;
+        if (F16) {
+          bits = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
+          if (terms == 3 && k == 0) bits &= MfmaElem<true>::kLeadMask;
+          v -= static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(bits)));
+        } else {
+          bits = bf16_bits(v) & 0xffffu;
+          v -= bf16_value(bits);
+        }
+        word |= bits << (16 * h);
+      }
+      out[i] = word;
     }
-    out[e] = static_cast<uint16_t>(word);
+    *reinterpret_cast<u32x4*>(dst + k * stride) = out;
   }
-  uint16_t* dst = frags + (((((static_cast<int64_t>(b) * a.n_layers + layer) * a.kv_heads + head) * n_frag + frag) * packed) + pl) * 8;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) dst[e] = out[e];
 }
 
-// fp16 fragments: one wave per (sequence, layer, KV head, query head g), 256
-// threads per workgroup.  Lane l < 4*(nk+nf) owns K step l/4, row block l%4:
-// its eight weights (magnitude weights times 1/kMagScale), then the column's
-// largest magnitude over the wave picks the power-of-two scale 2^s that brings
-// it to [2^13, 2^14) (s in [-126, 126]; none when it is 0, inf or NaN).  The
-// lane writes the fp16 words of 2^s w, each of what the ones before it leave,
-// in the packed layout of fold_mfma_kernel; lane 0 writes 2^-s.
-__global__ __launch_bounds__(256) void fold_mfma_f16_kernel(FoldArgs a, int nk, int nf, int terms,
-                                                            uint16_t* __restrict__ frags,
-                                                            float* __restrict__ inv_scale) {
-  const int64_t col = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  const int64_t cols = static_cast<int64_t>(a.n_seq) * a.n_layers * a.kv_heads * a.qpk;
-  if (col >= cols) return;  // whole wave
-  const int lane = threadIdx.x & 63;
-  const int g = static_cast<int>(col % a.qpk);
-  int64_t r = col / a.qpk;
-  const int head = static_cast<int>(r % a.kv_heads);
-  r /= a.kv_heads;
-  const int layer = static_cast<int>(r % a.n_layers);
-  const int b = static_cast<int>(r / a.n_layers);
-  const int64_t row = ((static_cast<int64_t>(layer) * a.kv_heads + head) * a.qpk + g);
-  const bool active = lane < 4 * (nk + nf);
-  const int step = lane >> 2, kb = lane & 3;
-  float w[8];
-  float big = 0.0f;
+// The fragments of `heads` KV heads of one (sequence b, layer) for `threads`
+// threads starting at `first`, phases pc, ps.  bf16: a thread a live lane of a K step.  fp16: a wave
+// a column (KV head, query head g); lane l < 4*(nk+nf) owns K step l/4, row
+// block l%4: its eight weights (magnitude weights times 1/kMagScale), then the
+// column's largest magnitude over the wave picks the power-of-two scale 2^s
+// that brings it to [2^13, 2^14) (s in [-126, 126]; none when it is 0, inf or
+// NaN), the words are those of 2^s w, and lane 0 writes 2^-s.
+template <bool F16>
+__device__ __forceinline__ void fold_layer(const FoldArgs& a, const float* pc, const float* ps, int b, int layer, int nk,
+                                           int nf, int terms, uint16_t* frags, float* inv_scale, int head_begin, int heads,
+                                           int first, int threads) {
+  const int packed = 4 * a.qpk;  // live lanes per fragment
+  const int steps = nk + nf;
+  const int64_t head0 = (static_cast<int64_t>(b) * a.n_layers + layer) * a.kv_heads;
+  const int items = F16 ? heads * a.qpk * 64 : heads * steps * packed;
+  for (int idx = first; idx < items; idx += threads) {
+    int head, g, step, kb;
+    bool active = true;
+    if (F16) {
+      const int lane = idx & 63, col = idx >> 6;
+      head = col / a.qpk;
+      g = col - head * a.qpk;
+      step = lane >> 2;
+      kb = lane & 3;
+      active = step < steps;
+    } else {
+      const int r = idx / packed, pl = idx - r * packed;
+      head = r / steps;
+      step = r - head * steps;
+      kb = pl / a.qpk;
+      g = pl - kb * a.qpk;
+    }
+    head += head_begin;
+    const int64_t row = (static_cast<int64_t>(layer) * a.kv_heads + head) * a.qpk + g;
+    float w[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    w[e] = active ? folded_weight(a, nk, nf, b, layer, row, step, kb, e) : 0.0f;
-    if (step >= nk) w[e] *= 1.0f / MfmaElem<true>::kMagScale;
-    big = fmaxf(big, fabsf(w[e]));
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) big = fmaxf(big, __shfl_xor(big, off));
-  int sh = 0;
-  if (big > 0.0f && big <= 3.4e38f) {
-    int ex;
-    (void)frexpf(big, &ex);  // big < 2^ex
-    sh = 14 - ex;
-    sh = sh < -126 ? -126 : (sh > 126 ? 126 : sh);
-  }
-  if (active) {
-    const int n_frag = terms * (nk + nf);
-    const int packed = 4 * a.qpk;
-    const int64_t base =
-        (((static_cast<int64_t>(b) * a.n_layers + layer) * a.kv_heads + head) * n_frag + terms * step) * packed +
-        kb * a.qpk + g;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) w[e] = ldexpf(w[e], sh);
-    for (int k = 0; k < terms; ++k) {
-      uint16_t* dst = frags + (base + k * packed) * 8;
+    for (int e = 0; e < 8; ++e) w[e] = active ? folded_weight(a, pc, ps, nk, nf, row, step, kb, e) : 0.0f;
+    if (F16) {
+      float big = 0.0f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        uint16_t bits = __builtin_bit_cast(uint16_t, static_cast<_Float16>(w[e]));
-        if (terms == 3 && k == 0) bits &= MfmaElem<true>::kLeadMask;
-        dst[e] = bits;
-        w[e] -= static_cast<float>(__builtin_bit_cast(_Float16, bits));
+        if (step >= nk) w[e] *= 1.0f / MfmaElem<true>::kMagScale;
+        big = fmaxf(big, fabsf(w[e]));
+      }
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) big = fmaxf(big, __shfl_xor(big, off));
+      int sh = 0;
+      if (big > 0.0f && big <= 3.4e38f) {
+        int ex;
+        (void)frexpf(big, &ex);  // big < 2^ex
+        sh = 14 - ex;
+        sh = sh < -126 ? -126 : (sh > 126 ? 126 : sh);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w[e] = ldexpf(w[e], sh);
+      if ((idx & 63) == 0) inv_scale[(head0 + head) * a.qpk + g] = ldexpf(1.0f, -sh);
+    }
+    if (active)
+      store_words<F16>(w, terms, frags + (((head0 + head) * terms * steps + terms * step) * packed + kb * a.qpk + g) * 8,
+                       packed * 8);
+  }
+}
+
+// grid (blocks, layers, sequences): phases from the caller's tables.
+constexpr int kFoldThreads = 256;
+template <bool F16>
+__global__ __launch_bounds__(kFoldThreads) void fold_mfma_kernel(FoldArgs a, int nk, int nf, int terms,
+                                                                 uint16_t* __restrict__ frags,
+                                                                 float* __restrict__ inv_scale) {
+  const int layer = blockIdx.y, b = blockIdx.z;
+  const int64_t at = b * a.phase_seq_stride + static_cast<int64_t>(layer) * a.freq;
+  fold_layer<F16>(a, a.phase_cos + at, a.phase_sin + at, b, layer, nk, nf, terms, frags, inv_scale, 0,
+                  a.kv_heads, blockIdx.x * kFoldThreads + threadIdx.x, gridDim.x * kFoldThreads);
+}
+
+// grid (layers, sequences, head splits): a workgroup forms its (sequence,
+// layer)'s mean phases, which every head shares, in LDS (and split 0 in the
+// caller's tables), and folds its KV heads' weights from them.  One workgroup's
+// scattered loads of the statistics bound it, so the heads are split until some
+// 512 workgroups share them, each forming the phases again.  As two launches this was
+// 4.2 + 6.2 us for one sequence x 6 layers of 40 heads, and the gap between
+// them; in one workgroup a layer 10.6, with the heads split 8.1.  16 sequences:
+// 4.9 + 8.6 before, 12.9 now.
+constexpr int kFoldPhaseThreads = 1024;
+constexpr int kFoldMaxFreq = 128;
+template <bool F16>
+__global__ __launch_bounds__(kFoldPhaseThreads) void fold_phases_kernel(FoldArgs a, PhaseArgs ph, int width, int nk, int nf,
+                                                                        int terms, uint16_t* __restrict__ frags,
+                                                                        float* __restrict__ inv_scale) {
+  __shared__ float s_cos[kFoldMaxFreq], s_sin[kFoldMaxFreq];
+  const int layer = blockIdx.x, b = blockIdx.y;
+  const float rs = static_cast<float>(ph.round_starts[b]);
+  const int64_t at = (static_cast<int64_t>(b) * a.n_layers + layer) * a.freq;
+  for (int i = threadIdx.x; i < a.freq * width; i += kFoldPhaseThreads) {  // whole lane groups
+    const int f = i / width, lane = i & (width - 1);
+    const float2 m = mean_phase(lane, width, rs, ph.omega[static_cast<int64_t>(layer) * a.freq + f], ph.offsets, ph.n_offsets);
+    if (lane == 0) {
+      s_cos[f] = m.x;
+      s_sin[f] = m.y;
+      if (blockIdx.z == 0) {
+        ph.phase_cos[at + f] = m.x;
+        ph.phase_sin[at + f] = m.y;
       }
     }
   }
-  if (lane == 0) inv_scale[col] = ldexpf(1.0f, -sh);
+  __syncthreads();
+  const int per = (a.kv_heads + gridDim.z - 1) / gridDim.z;
+  const int head = blockIdx.z * per;
+  fold_layer<F16>(a, s_cos, s_sin, b, layer, nk, nf, terms, frags, inv_scale, head, min(per, a.kv_heads - head),
+                  threadIdx.x, kFoldPhaseThreads);
 }
 
 // --------------------------------------------------------------- score ------
@@ -608,42 +649,54 @@ bool mfma_scorer_supported(const ScoreShape& s, int dtype, int rope_style) {
   return pick(s, dtype, rope_style) != nullptr;
 }
 
-int64_t mfma_fold_items(const ScoreShape& s, int dtype) {
+namespace {
+// Workgroups a (sequence, layer) is folded by.
+unsigned fold_blocks(const ScoreShape& s, int dtype) {
   const MfmaGeometry geo = geometry(s);
-  const int64_t cols = static_cast<int64_t>(s.n_seq) * s.n_layers * s.kv_heads * s.qpk;
-  // fp16: one wave per weight column, four per workgroup; bf16: one thread per
-  // live lane of every fragment.
-  if (dtype == KVC_DTYPE_FP16) return ceil_div(cols, 4) * 256;
-  return ceil_div(cols * geo.terms * (geo.nk + geo.nf) * 4, 256) * 256;
+  const int cols = s.kv_heads * s.qpk;
+  return static_cast<unsigned>(ceil_div(dtype == KVC_DTYPE_FP16 ? cols * 64 : cols * 4 * (geo.nk + geo.nf), kFoldThreads));
+}
+}  // namespace
+
+int64_t mfma_fold_items(const ScoreShape& s, int dtype) {
+  return static_cast<int64_t>(fold_blocks(s, dtype)) * kFoldThreads * s.n_layers * s.n_seq;
 }
 
 int launch_mfma_fold(hipStream_t stream, const ScoreShape& s, int dtype, const FoldArgs& fa, void* weights) {
   const MfmaGeometry geo = geometry(s);
   const int64_t items = mfma_fold_items(s, dtype);
-  if (items > kMaxDispatchItems)
+  if (items > kMaxDispatchItems || s.n_seq > 65535 || s.n_layers > 65535)
     return fail(KVC_EINVAL, "kvc_score_paged: the weight fold's %lld work-items exceed one dispatch",
                 static_cast<long long>(items));
   uint16_t* frags = static_cast<uint16_t*>(weights);
   float* inv_scale = reinterpret_cast<float*>(static_cast<char*>(weights) + mfma_fragment_only_bytes(s));
-  const unsigned blocks = static_cast<unsigned>(items / 256);
-  if (dtype == KVC_DTYPE_FP16) {
-    fold_mfma_f16_kernel<<<blocks, 256, 0, stream>>>(fa, geo.nk, geo.nf, geo.terms, frags, inv_scale);
-  } else {
-    fold_mfma_kernel<<<blocks, 256, 0, stream>>>(fa, geo.nk, geo.nf, geo.terms, frags);
-  }
+  const dim3 grid(fold_blocks(s, dtype), static_cast<unsigned>(s.n_layers), static_cast<unsigned>(s.n_seq));
+  (dtype == KVC_DTYPE_FP16 ? fold_mfma_kernel<true> : fold_mfma_kernel<false>)<<<grid, kFoldThreads, 0, stream>>>(
+      fa, geo.nk, geo.nf, geo.terms, frags, inv_scale);
   return launch_status("kvc_score_paged(fold)");
 }
 
-int launch_mfma_scorer(hipStream_t stream, const ScoreShape& s, int dtype, const FoldArgs& fa, const ScoreArgs& sa,
-                       void* weights) {
+int launch_mfma_scorer(hipStream_t stream, const ScoreShape& s, int dtype, const PhaseArgs* phases, const FoldArgs& fa,
+                       const ScoreArgs& sa, void* weights) {
   const MfmaGeometry geo = geometry(s);
   MfmaKernel kern = pick(s, dtype, fa.interleaved ? KVC_ROPE_INTERLEAVED : KVC_ROPE_HALF);
   if (!kern) return fail(KVC_EINVAL, "kvc_score_paged: no MFMA scorer for head_dim %d rotary_dim %d", s.head_dim, s.rotary_dim);
-  if (int rc = launch_mfma_fold(stream, s, dtype, fa, weights)) return rc;
-  const uint16_t* frags = static_cast<const uint16_t*>(weights);
-  const float* inv_scale = reinterpret_cast<const float*>(static_cast<const char*>(weights) + mfma_fragment_only_bytes(s));
   if (s.n_seq > 65535 || s.n_layers > 65535)
     return fail(KVC_EINVAL, "kvc_score_paged: too many sequences or layers for one launch");
+  if (phases) {
+    uint16_t* out = static_cast<uint16_t*>(weights);
+    float* scale = reinterpret_cast<float*>(static_cast<char*>(weights) + mfma_fragment_only_bytes(s));
+    const int64_t splits = ceil_div(512, static_cast<int64_t>(s.n_layers) * s.n_seq);
+    const dim3 grid(static_cast<unsigned>(s.n_layers), static_cast<unsigned>(s.n_seq),
+                    static_cast<unsigned>(splits < s.kv_heads ? splits : s.kv_heads));
+    (dtype == KVC_DTYPE_FP16 ? fold_phases_kernel<true> : fold_phases_kernel<false>)<<<grid, kFoldPhaseThreads, 0, stream>>>(
+        fa, *phases, phase_lanes(phases->n_offsets), geo.nk, geo.nf, geo.terms, out, scale);
+    if (int rc = launch_status("kvc_score_paged(phases and fold)")) return rc;
+  } else if (int rc = launch_mfma_fold(stream, s, dtype, fa, weights)) {
+    return rc;
+  }
+  const uint16_t* frags = static_cast<const uint16_t*>(weights);
+  const float* inv_scale = reinterpret_cast<const float*>(static_cast<const char*>(weights) + mfma_fragment_only_bytes(s));
   const int64_t gx = static_cast<int64_t>(s.max_tiles) * geo.head_groups;
   if (gx > 0x7fffffff) return fail(KVC_EINVAL, "kvc_score_paged: grid too large");
   dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(s.n_seq), static_cast<unsigned>(s.n_layers));

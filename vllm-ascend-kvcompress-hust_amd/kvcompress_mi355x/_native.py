@@ -63,6 +63,14 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
             _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i32, _i64, _p, _i64, _i64, _i64, _p, _sz,
         ],
     ),
+    "kvc_score_batch": (
+        _i32,
+        [
+            _p, _i32, _i32, _p, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32,
+            _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p,
+            _i32, _p, _p, _p, _p, _i64, _i64, _i64, _p, _sz, _p, _p,
+        ],
+    ),
     "kvc_head_stats": (_i32, [_p, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _p, _p, _sz, _p, _p]),
     "kvc_score_paged_noalloc": (
         _i32,

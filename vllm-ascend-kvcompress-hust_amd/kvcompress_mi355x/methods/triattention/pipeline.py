@@ -324,28 +324,7 @@ class CompressionPipeline:
         stream = dev.stream_handle(self.device)
         max_len = max(batch.seq_lens_host)
         n_off = int(t.offsets.numel())
-        max_mode = self.score_aggregation == "max"
-        _native.call(
-            "kvc_offset_phases" if max_mode else "kvc_mean_phases",
-            stream,
-            batch.n_seq,
-            t.n_layers,
-            t.freq,
-            dev.ptr(batch.round_starts),
-            dev.ptr(t.offsets),
-            n_off,
-            dev.ptr(t.omega),
-            dev.ptr(self.phase_cos),
-            dev.ptr(self.phase_sin),
-        )
-        phase_args = (
-            (dev.ptr(self.phase_cos), dev.ptr(self.phase_sin), n_off, t.n_layers * n_off * t.freq)
-            if max_mode
-            else (dev.ptr(self.phase_cos), dev.ptr(self.phase_sin), t.n_layers * t.freq)
-        )
-        _native.call(
-            "kvc_score_paged_max" if max_mode else "kvc_score_paged",
-            stream,
+        shape = (
             dev.cache_dtype_code(self.dtype),
             t.n_layers,
             dev.ptr(self.scoring_ptrs),
@@ -367,27 +346,22 @@ class CompressionPipeline:
             dev.ptr(t.freq_scale),
             dev.ptr(t.extra),
             dev.ptr(t.q_pass),
-            *phase_args,
-            dev.ptr(self.raw),
-            *self.raw_strides(),
-            dev.ptr(self.workspace),
-            self.workspace_bytes,
+        )
+        phases = (dev.ptr(self.phase_cos), dev.ptr(self.phase_sin))
+        offsets = (dev.ptr(batch.round_starts), dev.ptr(t.offsets), n_off, dev.ptr(t.omega))
+        raw = (dev.ptr(self.raw), *self.raw_strides())
+        workspace = (dev.ptr(self.workspace), self.workspace_bytes)
+        stats = (dev.ptr(self.mean), dev.ptr(self.var))
+        if self.score_aggregation == "mean":
+            _native.call("kvc_score_batch", stream, *shape, *offsets, *phases, *raw, *workspace, *stats)
+            return
+        _native.call("kvc_offset_phases", stream, batch.n_seq, t.n_layers, t.freq, *offsets, *phases)
+        _native.call(
+            "kvc_score_paged_max", stream, *shape, *phases, n_off, t.n_layers * n_off * t.freq, *raw, *workspace
         )
         _native.call(
-            "kvc_head_stats",
-            stream,
-            t.n_layers,
-            self.kv_heads,
-            self.head_dim,
-            t.rotary_dim,
-            t.qpk,
-            batch.n_seq,
-            max_len,
-            dev.ptr(batch.seq_lens),
-            dev.ptr(self.workspace),
-            self.workspace_bytes,
-            dev.ptr(self.mean),
-            dev.ptr(self.var),
+            "kvc_head_stats", stream, t.n_layers, self.kv_heads, self.head_dim, t.rotary_dim, t.qpk, batch.n_seq, max_len,
+            dev.ptr(batch.seq_lens), *workspace, *stats,
         )
 
     def aggregate(self, batch: Batch) -> None:
