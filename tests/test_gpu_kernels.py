@@ -250,6 +250,10 @@ PART_SHAPES = [
     (2, 3, 256, 224, "half", torch.bfloat16, 290),
     (1, 6, 256, 208, "interleaved", torch.bfloat16, 1),
     (8, 2, 112, 48, "half", torch.float16, 1000),
+    (8, 3, 112, 48, "half", torch.float16, 1000),
+    (2, 4, 256, 16, "half", torch.float16, 300),
+    (1, 4, 256, 96, "interleaved", torch.bfloat16, 257),
+    (2, 3, 96, 96, "interleaved", torch.float16, 129),
 ]
 
 

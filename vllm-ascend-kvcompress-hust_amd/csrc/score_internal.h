@@ -111,8 +111,18 @@ inline bool mfma_two_words(const ScoreShape& s) {
   return mfma_full_steps(s) && (s.head_dim == 64 || s.head_dim == 128 || s.head_dim == 256) &&
          (s.freq == 32 || s.freq == 64 || s.freq == 128);
 }
+// The three-word products cost the same for any number of query heads up to 8,
+// the vector scorer about 10 us more a head, so few heads stay with it.
+// Phases, fold, scores and statistics of 8 x 8192 tokens x 2 layers, 4 KV heads,
+// 1 / 2 / 3 / 4 / 8 query heads each, vector against matrix: 96 dims 34 / 39 / 45 /
+// 52 / 91 against 40 / 40 / 41 / 41 / 44 us, 256 dims with 16 rotary 58 / 65 / 76 / 89
+// / 156 against 85 / 86 / 87 / 87 / 91; 11 x 770 tokens x 6 layers, 96 dims: 32 / 37 /
+// 44 / 51 / 89 against 42 / 43 / 44 / 43 / 47.
 inline bool mfma_shape(const ScoreShape& s) {
-  return mfma_two_words(s) || (!s.vector_only && s.head_dim <= 256 && s.rotary_dim <= 128);
+  if (mfma_two_words(s)) return true;
+  if (s.vector_only || s.head_dim > 256 || s.rotary_dim > 128) return false;
+  const int steps = 2 * ((s.freq + 31) / 32) + (s.pass + 31) / 32;
+  return s.qpk >= (steps >= 6 ? 4 : 3);
 }
 inline MfmaSteps mfma_steps(const ScoreShape& s) {
   MfmaSteps m;
