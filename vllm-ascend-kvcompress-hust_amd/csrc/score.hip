@@ -468,15 +468,17 @@ __device__ __forceinline__ float quad_max_nan(float v) {
   return v;
 }
 
-// Token-major scores whose rows are whole, aligned 16-byte words: L lanes a
+// Token-major scores whose rows are whole, aligned 16-byte words: eight lanes a
 // token, each reading four adjacent heads at a time, two tokens and two layers
 // in flight, so a wave instruction covers whole rows and a mean or scale word
 // serves eight scores.  The one-float form below reads 16 tokens x 4 heads an
 // instruction, one layer after the other: 18.0 us for 8 x 2k-16k tokens x 4
 // layers x 32 heads (33 MB), 15.2 here, a third of it the divisions.
-template <int L>
+constexpr int kAggRowLanes = 8;
+
 __global__ __launch_bounds__(kAggThreads) void aggregate_rows_kernel(AggArgs a) {
   extern __shared__ __attribute__((aligned(16))) float dyn[];
+  constexpr int L = kAggRowLanes;
   constexpr int kSlots = kAggThreads / L;
   const int n_stats = a.n_layers * a.n_heads;
   const int b = blockIdx.y;
@@ -523,7 +525,7 @@ __global__ __launch_bounds__(kAggThreads) void aggregate_rows_kernel(AggArgs a) 
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         float v = quad_max_nan(best[d][i]);
-        if (L == 8) v = max_nan(v, dpp_row_half_mirror(v));
+        v = max_nan(v, dpp_row_half_mirror(v));
         if (a.layer_out_stride) {
           if (q == 0 && t0 + i * kSlots < n) a.agg[(l0 + d) * a.layer_out_stride + tok[i]] = v;
         } else {
@@ -1107,12 +1109,12 @@ int launch_aggregate(const char* who, kvc_stream_t stream, int n_layers, int n_h
     aggregate_tokens_kernel<<<grid, kAggThreads, lds, as_stream(stream)>>>(aa);
     return launch_status(who);
   }
-  if (raw_head_stride == 1 && n_heads % 4 == 0 && raw_token_stride % 4 == 0 && raw_layer_stride % 4 == 0 &&
+  if (raw_head_stride == 1 && n_heads > 16 && n_heads % 4 == 0 && raw_token_stride % 4 == 0 && raw_layer_stride % 4 == 0 &&
       reinterpret_cast<uintptr_t>(raw) % 16 == 0) {
-    // Four lanes hold 16 heads of a token; past that eight, in turns past 32.
-    const int lanes = n_heads <= 16 ? 4 : 8;
-    dim3 grid(static_cast<unsigned>(ceil_div(max_seq_len, 2 * kAggThreads / lanes)), static_cast<unsigned>(n_seq));
-    (lanes == 4 ? aggregate_rows_kernel<4> : aggregate_rows_kernel<8>)<<<grid, kAggThreads, lds, as_stream(stream)>>>(aa);
+    // Up to 16 heads leave half of a token's eight lanes idle, and half the
+    // workgroups: 2 us more than the other form at 4 heads x 11 x 770 tokens.
+    dim3 grid(static_cast<unsigned>(ceil_div(max_seq_len, 2 * kAggThreads / kAggRowLanes)), static_cast<unsigned>(n_seq));
+    aggregate_rows_kernel<<<grid, kAggThreads, lds, as_stream(stream)>>>(aa);
     return launch_status(who);
   }
   dim3 grid(static_cast<unsigned>(ceil_div(max_seq_len, kAggTokensPerBlock)), static_cast<unsigned>(n_seq));
