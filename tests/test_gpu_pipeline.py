@@ -427,3 +427,30 @@ def test_batch_scoring_equals_its_three_calls(hip_device, shape) -> None:
                  p.workspace_bytes, dev.ptr(p.mean), dev.ptr(p.var))
     for have, want in zip(got, (p.phase_cos, p.phase_sin, p.raw, *p.head_statistics(batch))):
         assert torch.equal(have, want)
+
+
+def test_batch_built_on_one_stream_and_used_on_another(hip_device) -> None:
+    """A batch built behind queued work on one stream is whole when build
+    returns: a second stream that waits for nothing reads every descriptor and
+    may overwrite the block tables it was built from."""
+    from kvcompress_mi355x.methods.triattention.pipeline import Batch
+
+    lens, starts = [300, 1300, 2300], [11, 12, 13]
+    tables = [(torch.arange(-(-n // 128)) + 7 * i).to(hip_device) for i, n in enumerate(lens)]
+    want = torch.cat(tables).tolist()
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(first):
+        busy = torch.randn(4096, 4096, device=hip_device)
+        for _ in range(40):
+            busy = busy @ busy / 64.0
+        batch = Batch.build(hip_device, lens, starts, tables, [t[:2] for t in tables], budget=200)
+    with torch.cuda.stream(second):
+        for t in tables:
+            t.fill_(-1)
+        copies = [t.cpu().tolist() for t in (batch.seq_lens, batch.token_offsets, batch.round_starts, batch.src_offsets,
+                                             batch.src_ids, batch.dst_offsets)]
+    counts = torch.tensor([0] + [t.numel() for t in tables]).cumsum(0).tolist()
+    assert copies == [lens, [0, 300, 1600, 3900], starts, counts, want, [0, 2, 4, 6]]
+    torch.cuda.synchronize()
+    assert batch.src_ids.tolist() == want

@@ -223,7 +223,7 @@ class TriAttentionMethod(KVCompressionMethod):
         for request in requests:
             dev.require_hip(request.source_block_ids_device, "source_block_ids_device")
             dev.require_hip(request.destination_block_ids_device, "destination_block_ids_device")
-        batch = Batch.build(
+        batch = Batch.queue(
             self.pipeline.device,
             [int(r.physical_num_tokens) for r in requests],
             [int(r.semantic_num_tokens) for r in requests],
@@ -232,8 +232,11 @@ class TriAttentionMethod(KVCompressionMethod):
             block_size=self.cache_block_size,
             budget=self.config.kv_budget,
         )
-        self._select(batch)
-        self.pipeline.compact(batch)
+        try:
+            self._select(batch)
+            self.pipeline.compact(batch)
+        finally:
+            batch.wait()  # the requests' block tables are the caller's again
         return [self._result() for _ in requests]
 
     def _select(self, batch: Batch) -> torch.Tensor:
@@ -245,8 +248,11 @@ class TriAttentionMethod(KVCompressionMethod):
         """Keep indices of one request without materialising (tri/method.py:297-475)."""
         if self.pipeline is None:
             raise RuntimeError("TriAttention method is not bound to KV cache")
-        batch = Batch.build(self.pipeline.device, [int(physical_num_tokens)], [int(round_start)], [source_block_ids])
-        return self._select(batch)[0].clone()
+        batch = Batch.queue(self.pipeline.device, [int(physical_num_tokens)], [int(round_start)], [source_block_ids])
+        try:
+            return self._select(batch)[0].clone()
+        finally:
+            batch.wait()
 
 
 def tensor_parallel_group() -> Any:

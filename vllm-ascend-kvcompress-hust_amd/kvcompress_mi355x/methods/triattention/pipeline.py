@@ -90,7 +90,12 @@ class ScoringTables:
 
 @dataclass
 class Batch:
-    """Device descriptors of one batch of sequences."""
+    """Device descriptors of one batch of sequences.
+
+    ``build`` returns when they are written and the block tables it was given
+    are read, so the batch may be used, and the tables changed, on any stream.
+    ``queue`` only puts the copies on the current stream: for callers that use
+    the batch on that stream and call ``wait`` before they hand back the tables."""
 
     n_seq: int
     seq_lens_host: list[int]
@@ -104,6 +109,7 @@ class Batch:
     dst_offsets: torch.Tensor | None
     dst_ids: torch.Tensor | None
     rewrite_buffers: dict = field(default_factory=dict)
+    written: torch.cuda.Event | None = field(default=None, repr=False, compare=False)
 
     @property
     def total_tokens(self) -> int:
@@ -115,6 +121,29 @@ class Batch:
 
     @classmethod
     def build(
+        cls,
+        device: torch.device,
+        seq_lens: list[int],
+        round_starts: list[int],
+        source_tables: list,
+        destination_tables: list | None = None,
+        *,
+        block_size: int = 128,
+        budget: int | None = None,
+    ) -> Batch:
+        batch = cls.queue(
+            device, seq_lens, round_starts, source_tables, destination_tables, block_size=block_size, budget=budget
+        )
+        batch.wait()
+        return batch
+
+    def wait(self) -> None:
+        """Until the device has run the copies that ``queue`` put on its stream."""
+        if self.written is not None:
+            self.written.synchronize()
+
+    @classmethod
+    def queue(
         cls,
         device: torch.device,
         seq_lens: list[int],
@@ -144,6 +173,10 @@ class Batch:
                 if any(d < need for d in dst_lens):
                     raise ValueError("destination table too short for the budget")
         (token_offsets, round_starts_dev, src_off, *rest), seq_lens_dev = dev.pack_words(columns, seq_lens, device)
+        written = None
+        if seq_lens_dev.is_cuda:
+            written = torch.cuda.Event()
+            written.record(torch.cuda.current_stream(device))
         return cls(
             n_seq=n,
             seq_lens_host=[int(x) for x in seq_lens],
@@ -156,6 +189,7 @@ class Batch:
             src_ids=src_ids,
             dst_offsets=rest[0] if rest else None,
             dst_ids=dst_ids,
+            written=written,
         )
 
 
