@@ -574,3 +574,30 @@ def test_compaction_form_waits_for_events_and_capture():
     assert choice.chosen == "layer_major"
     captured = CompactionFormChoice(event_factory=lambda: None, capturing=lambda: True)
     assert captured.next_call() == ("layer_major", None) and captured._next == 0
+
+
+def test_launches_refuse_host_tensors(monkeypatch):
+    """A launch on host tensors ends with a ValueError before the kernel call,
+    whatever the current stream's handle is."""
+    from kvcompress_mi355x import _native
+    from kvcompress_mi355x.methods.triattention import _device as dev
+    from kvcompress_mi355x.methods.triattention import cache, selection
+
+    launched = []
+    monkeypatch.setattr(_native, "call", lambda entry, *args: launched.append(entry))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 64)
+    assert dev.stream_handle(torch.device("cuda")) == dev.stream_handle(torch.device("cuda", 1)) == 64
+    with pytest.raises(ValueError, match="HIP device"):
+        dev.stream_handle(torch.device("cpu"))
+    lens, offsets = torch.tensor([300], dtype=torch.int32), torch.tensor([0, 300])
+    keep = torch.zeros((1, 100), dtype=torch.int64)
+    with pytest.raises(ValueError, match="HIP device"):
+        selection.select_keep_indices_batched(
+            torch.zeros(300), lens, offsets, [300], keep, budget=100, protected_prefix=0, protected_recent=0, segments=1,
+            policy="global")
+    with pytest.raises(ValueError, match="HIP device"):
+        cache.compact_layers(
+            offsets, offsets, num_pages=3, page_stride=128, row_elems=1, seq_lens=lens, src_block_offsets=offsets,
+            src_block_ids=offsets, dst_block_offsets=None, dst_block_ids=None, keep=keep, budget=100)
+    assert launched == []
