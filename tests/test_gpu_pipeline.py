@@ -454,3 +454,13 @@ def test_batch_built_on_one_stream_and_used_on_another(hip_device) -> None:
     assert copies == [lens, [0, 300, 1600, 3900], starts, counts, want, [0, 2, 4, 6]]
     torch.cuda.synchronize()
     assert batch.src_ids.tolist() == want
+
+
+def test_batch_built_under_a_default_device(hip_device) -> None:
+    """A caller's default device does not reach the batch's host memory."""
+    from kvcompress_mi355x.methods.triattention.pipeline import Batch
+
+    with torch.device(hip_device):
+        batch = Batch.build(hip_device, [300, 20], [5, 6], [[4, 2, 9], [1]], [[7], [8]], budget=100)
+    assert batch.seq_lens.cpu().tolist() == [300, 20] and batch.src_ids.cpu().tolist() == [4, 2, 9, 1]
+    assert batch.token_offsets.cpu().tolist() == [0, 300, 320] and batch.dst_offsets.cpu().tolist() == [0, 1, 2]

@@ -136,7 +136,9 @@ def pack_words(columns: list[list[int]], lengths32: list[int], device: torch.dev
     if device.type == "cuda":
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("batch descriptors cannot be copied to the device under graph capture")
-        flat = torch.tensor(words, dtype=torch.int64, pin_memory=True).to(device, non_blocking=True)
+        # Host memory whatever the caller's default device is.
+        host = torch.tensor(words, dtype=torch.int64, device="cpu", pin_memory=True)
+        flat = host.to(device, non_blocking=True)
     else:
         flat = torch.tensor(words, dtype=torch.int64, device=device)
     out, at = [], 0
