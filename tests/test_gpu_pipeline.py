@@ -464,3 +464,11 @@ def test_batch_built_under_a_default_device(hip_device) -> None:
         batch = Batch.build(hip_device, [300, 20], [5, 6], [[4, 2, 9], [1]], [[7], [8]], budget=100)
     assert batch.seq_lens.cpu().tolist() == [300, 20] and batch.src_ids.cpu().tolist() == [4, 2, 9, 1]
     assert batch.token_offsets.cpu().tolist() == [0, 300, 320] and batch.dst_offsets.cpu().tolist() == [0, 1, 2]
+
+
+def test_batch_length_past_32_bits_is_a_runtime_error(hip_device) -> None:
+    """The type torch's own conversion to int32 raises."""
+    from kvcompress_mi355x.methods.triattention.pipeline import Batch
+
+    with pytest.raises(RuntimeError, match="32 bits"):
+        Batch.build(hip_device, [1 << 31], [5], [torch.zeros(1 << 24, dtype=torch.int64, device=hip_device)])

@@ -127,7 +127,7 @@ def pack_words(columns: list[list[int]], lengths32: list[int], device: torch.dev
     the block again at each replay, so capture is refused, as a pageable copy
     is."""
     if any(not -(1 << 31) <= int(n) < (1 << 31) for n in lengths32):
-        raise OverflowError("sequence lengths must fit 32 bits")
+        raise RuntimeError("sequence lengths must fit 32 bits")
     words = [int(v) for column in columns for v in column]
     low = [int(n) & 0xFFFFFFFF for n in lengths32] + [0] * (len(lengths32) % 2)
     for i in range(0, len(low), 2):
