@@ -824,6 +824,55 @@ def test_select_split_score_distributions(hip_device, kind) -> None:
             np.testing.assert_array_equal(keep[0].cpu().numpy(), _stable_keep_np(part.numpy(), keep_count, 0, 0, 1, "global"))
 
 
+def _hard_scores(kind: str, n: int, g: torch.Generator) -> torch.Tensor:
+    """Scores that one set of value bins does not separate."""
+    x = torch.randn(n, generator=g)
+    at = torch.randperm(n, generator=g)
+    if kind == "both-infinities":
+        x[at[: n // 3]] = float("inf")
+        x[at[n // 3 : 2 * n // 3]] = float("-inf")
+    elif kind == "nans":  # of both signs and other payloads, beside infinities
+        x[at[: n // 4]] = float("nan")
+        bits = torch.tensor([0x7FC00001, -0x400000, 0x7F800000, -0x800000], dtype=torch.int32)
+        x.view(torch.int32)[at[n // 4 : n // 2]] = bits.repeat(n // 8 + 1)[: n // 2 - n // 4]
+    elif kind == "heavy-tail":
+        x = torch.tan(1.5707 * (2 * torch.rand(n, generator=g) - 1)) ** 3
+    elif kind == "two-scales":  # outliers, and ones of the rest, in every group of lanes
+        x[at[: n // 5]] *= 1e-8
+        x[at[n // 5 : n // 4]] *= 1e12
+        x[at[n // 4 : n // 4 + 100]] *= 3e37
+    elif kind == "zeros":
+        x = torch.where(x > 0, 0.0, -0.0)
+    elif kind == "subnormal":
+        x = torch.randint(-9, 9, (n,), generator=g) * 2.0**-149
+    elif kind == "trend":
+        x = torch.arange(n) * 1e-3 + 1e-4 * x
+    return x.float()
+
+
+@pytest.mark.parametrize("shape", ["single", "split"])
+@pytest.mark.parametrize("kind", ["both-infinities", "nans", "heavy-tail", "two-scales", "zeros", "subnormal", "trend"])
+def test_select_scores_binned_again(hip_device, kind, shape) -> None:
+    # Lengths around the cached form's limit (16384 scores), one chunk and
+    # longer chunks; keep counts that put the threshold into every kind of bin.
+    _, selection, _ = _kvc()
+    g = torch.Generator().manual_seed(len(kind))
+    for n in (1, 5, 1500, 16384, 16390, 70001) + ((131075,) if shape == "split" else ()):
+        scores = _hard_scores(kind, n + 3, g)[3:]
+        d_scores = torch.cat([torch.zeros(3), scores]).to(hip_device)  # misaligned
+        for keep_count in sorted({1, n // 10 + 1, n // 4 + 7, n // 2, 5 * n // 6, n - 1}):
+            if not 0 < keep_count <= n:
+                continue
+            seq_lens = torch.tensor([n], dtype=torch.int32, device=hip_device)
+            token_offsets = torch.tensor([3, 3 + n], dtype=torch.int64, device=hip_device)
+            keep = torch.full((1, keep_count), -7, dtype=torch.int64, device=hip_device)
+            selection.select_keep_indices_batched(
+                d_scores, seq_lens, token_offsets, [n], keep, budget=keep_count, protected_prefix=0, protected_recent=0,
+                segments=1, policy="global", shape=shape,
+            )
+            np.testing.assert_array_equal(keep[0].cpu().numpy(), _stable_keep_np(scores.numpy(), keep_count, 0, 0, 1, "global"))
+
+
 def test_select_split_rejects_a_small_workspace(hip_device) -> None:
     _, selection, _ = _kvc()
     scores = torch.randn(50000, device=hip_device)

@@ -3,17 +3,16 @@
 // A job is one (sequence, segment).  The segment's scores are mapped to
 // order-preserving 32-bit keys; the exact key T of the K-th largest score and
 // how many scores equal to T are still needed come from a histogram over value
-// bins and an exact ranking inside one bin, or from four 8-bit radix passes
-// (LDS histograms of the keys that still match the selected high digits).
+// bins and an exact ranking inside one bin (binned again while a bin holds too
+// many keys to rank).
 // Emission keeps every key > T plus the first `need` keys == T (ties go to the
 // lowest index), walking the segment in coalesced tiles: prefix sums of packed
 // (greater, equal) counts give every key its output slot, so the output is
 // sorted without a sort.
 //
 // Two launch shapes:
-//  * kvc_select_keep: one 1024-thread workgroup per job (value bins, radix
-//    passes where they do not separate the scores).  Right for batches of many
-//    sequences.
+//  * kvc_select_keep: one 1024-thread workgroup per job.  Right for batches of
+//    many sequences.
 //  * kvc_select_keep_split: a job's segment is cut into chunks of >= 4096 keys,
 //    one 256-thread workgroup each, in three launches (no workgroup waits for
 //    another inside one): every chunk's histogram over value bins, the chunks'
@@ -37,9 +36,8 @@ constexpr int kSelThreads = 1024;   // one workgroup per job
 constexpr int kSplitThreads = 256;  // split path: one workgroup per chunk
 constexpr int kSplitChunk = 4096;   // keys per chunk, at least
 constexpr int kSplitMaxChunks = 32;
-constexpr int kSelUnroll = 4;  // float4 words per thread in flight in a histogram pass
+constexpr int kSelUnroll = 4;  // float4 words per thread in flight in a walk
 constexpr int kEmitWords = 2;  // float4 words per thread per emission tile
-constexpr int kSelPeel = 1;    // dominant digits counted with one atomic per wave
 
 struct SelectArgs {
   int n_seq, budget, prefix, recent, segments, policy;
@@ -122,7 +120,7 @@ __device__ Job make_job(const SelectArgs& a, int b, int seg) {
 }
 
 // Protected windows (the workgroup of segment 0) and segments kept whole.
-// Returns whether the job still needs a radix select.  Output rows are budget
+// Returns whether the job still needs a threshold.  Output rows are budget
 // entries wide; the guards keep a caller that skipped validation (a sequence
 // shorter than the budget) inside its row.
 __device__ bool fill_fixed(const SelectArgs& a, const Job& j, int seg, int64_t* out, int tid, int nthreads) {
@@ -142,9 +140,9 @@ __device__ bool fill_fixed(const SelectArgs& a, const Job& j, int seg, int64_t* 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Calls f(score) for every score in [start, stop), spread over a workgroup of
-// T threads: scalar head up to 16-byte alignment, float4 words kSelUnroll at a
+// T threads: scalar head up to 16-byte alignment, float4 words U at a
 // time (loads issued together), scalar tail.
-template <int T, typename F>
+template <int T, int U = kSelUnroll, typename F>
 __device__ __forceinline__ void for_each_score(const float* sc, int64_t start, int64_t stop, F&& f) {
   const int tid = threadIdx.x;
   const int64_t misalign = (reinterpret_cast<uintptr_t>(sc + start) >> 2) & 3;
@@ -154,15 +152,15 @@ __device__ __forceinline__ void for_each_score(const float* sc, int64_t start, i
   const int64_t body = start + head;
   const int64_t n4 = (stop - body) >> 2;
   const f32x4* v = reinterpret_cast<const f32x4*>(sc + body);
-  for (int64_t w0 = tid; w0 < n4; w0 += static_cast<int64_t>(T) * kSelUnroll) {
-    f32x4 x[kSelUnroll];
+  for (int64_t w0 = tid; w0 < n4; w0 += static_cast<int64_t>(T) * U) {
+    f32x4 x[U];
 #pragma unroll
-    for (int u = 0; u < kSelUnroll; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int64_t w = w0 + static_cast<int64_t>(u) * T;
       x[u] = v[w < n4 ? w : n4 - 1];  // in range; surplus words are ignored below
     }
 #pragma unroll
-    for (int u = 0; u < kSelUnroll; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int64_t w = w0 + static_cast<int64_t>(u) * T;
       if (w < n4) {
 #pragma unroll
@@ -171,6 +169,26 @@ __device__ __forceinline__ void for_each_score(const float* sc, int64_t start, i
     }
   }
   for (int64_t i = body + 4 * n4 + tid; i < stop; i += T) f(sc[i]);
+}
+
+// The same for code that few calls run: one score a load and little code (the
+// first pass over instructions costs more than the walk), except where 256
+// threads walk a whole segment and wait for memory.
+template <int T, typename F>
+__device__ __forceinline__ void for_each_score_rarely(const float* sc, int64_t start, int64_t stop, F&& f) {
+  if constexpr (T < kSelThreads) {
+    for_each_score<T, 8>(sc, start, stop, f);
+  } else {
+#pragma unroll 1
+    for (int64_t i0 = start + threadIdx.x; i0 < stop; i0 += kSelUnroll * T) {
+      float x[kSelUnroll];
+#pragma unroll
+      for (int u = 0; u < kSelUnroll; ++u) x[u] = sc[min(i0 + u * T, stop - 1)];
+#pragma unroll
+      for (int u = 0; u < kSelUnroll; ++u)
+        if (i0 + u * T < stop) f(x[u]);
+    }
+  }
 }
 
 // Exclusive prefix sum over a workgroup of T threads (thread order); *total
@@ -197,74 +215,6 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
   __syncthreads();  // s_wave is reused by the next scan
   *total = all;
   return before + incl - v;
-}
-
-// Counts one key's digit into a wave's LDS histogram.  Scores of similar
-// magnitude share their high digits (the first pass sees little more than the
-// sign and exponent), so most lanes of a wave can hit one or two bins; up to
-// kSelPeel times, the lanes holding the first active lane's digit add their
-// number with a single atomic, and the lanes left count one by one.
-__device__ __forceinline__ void count_digit(uint32_t* hist, uint32_t digit) {
-#pragma unroll
-  for (int p = 0; p < kSelPeel; ++p) {
-    const uint32_t lead = __builtin_amdgcn_readfirstlane(digit);
-    const uint64_t same = __ballot(digit == lead);
-    if (digit == lead) {
-      if (__lane_id() == static_cast<unsigned>(__ffsll(static_cast<unsigned long long>(same)) - 1))
-        atomicAdd(&hist[lead], static_cast<uint32_t>(__popcll(same)));
-      return;
-    }
-  }
-  atomicAdd(&hist[digit], 1u);
-}
-
-// Histogram (digit at `shift`) of the keys in [start, stop) that match
-// (want, mask): each wave counts into whist[wave], then hist = their sum.
-// Every thread of the workgroup calls it; hist is complete on return.
-template <int T>
-__device__ void range_histogram(const float* sc, int64_t start, int64_t stop, uint32_t want, uint32_t mask, int shift,
-                                uint32_t (*whist)[256], uint32_t* hist) {
-  const int tid = threadIdx.x;
-  for (int i = tid; i < (T / 64) * 256; i += T) (&whist[0][0])[i] = 0;
-  __syncthreads();
-  uint32_t* mine = whist[tid >> 6];
-  for_each_score<T>(sc, start, stop, [&](float x) {
-    const uint32_t k = float_key(x);
-    if ((k & mask) == want) count_digit(mine, (k >> shift) & 255u);
-  });
-  __syncthreads();
-  for (int i = tid; i < 256; i += T) {
-    uint32_t c = 0;
-#pragma unroll
-    for (int w = 0; w < T / 64; ++w) c += whist[w][i];
-    hist[i] = c;
-  }
-  __syncthreads();
-}
-
-// Wave 0: the digit whose bin holds the need-th largest matching key, and how
-// many keys of that bin are still needed.  Lane l owns bins 4l..4l+3.
-__device__ __forceinline__ void pick_digit(const uint32_t* hist, uint32_t need, uint32_t* s_digit, uint32_t* s_need) {
-  const int lane = threadIdx.x & 63;
-  const uint32_t c0 = hist[4 * lane], c1 = hist[4 * lane + 1];
-  const uint32_t c2 = hist[4 * lane + 2], c3 = hist[4 * lane + 3];
-  const uint32_t tot = c0 + c1 + c2 + c3;
-  uint32_t incl = tot;  // sum over lanes >= lane
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t v = __shfl_down(incl, off);
-    if (lane + off < 64) incl += v;
-  }
-  uint32_t above = incl - tot;  // matching keys in higher bins
-  const uint32_t cs[4] = {c0, c1, c2, c3};
-#pragma unroll
-  for (int j = 3; j >= 0; --j) {
-    if (above < need && need <= above + cs[j]) {
-      *s_digit = static_cast<uint32_t>(4 * lane + j);
-      *s_need = need - above;
-    }
-    above += cs[j];
-  }
 }
 
 // What the emission keeps: key k iff k > thresh, or k == thresh and fewer than
@@ -432,55 +382,255 @@ __device__ __forceinline__ void emit_range(const Keep& kp, const float* sc, int6
 // emission's layout with as few words a thread as hold the segment.
 constexpr int kCacheWords = 4;
 
-// The threshold by value bins: the scores' range is cut into kBins equal bins,
-// one histogram of which names the bin that holds the K-th largest score; that
-// bin's keys (a few dozen of 16 K aggregated scores) are gathered and ranked
-// exactly against each other.  bin(x) = trunc((x - lo) * scale) is a
-// composition of roundings that never decrease, so bins keep the order of the
-// keys.  One walk over scores that spread over many bins, where a radix pass
-// on the sign and exponent sends most lanes of a wave to the same two
-// counters, four times over.  Scores that defeat it (an infinity or NaN, a
-// range of zero or past float32, or more than kMaxCand keys in the bin: heavy
-// ties, an outlier of 1e30) take the four radix passes instead.  One
-// workgroup's instructions per score bound this kernel (1024 threads on one
-// CU), not its loads.  Microseconds per launch against the radix passes: one
-// 4096-score sequence 7.4 / 11.2, 16 x 16384 11.3 / 18.1, 8 x 65536 in eight v3
-// segments 9.7 / 17.6, one of 65000 31 / 53.
+// The threshold by value bins: a range of the scores is cut into kBins equal
+// bins, one histogram of which names the bin that holds the K-th largest score;
+// that bin's keys (a few dozen of 16 K aggregated scores) are gathered and
+// ranked exactly against each other.  bin(x) = trunc(clamp((hi - x) * scale))
+// is a composition of roundings that never increase, so bins keep the order of
+// the keys, and any range is right: scores past it, infinities among them,
+// count in the end bins.  One walk over scores that spread over many bins,
+// where a radix pass on the sign and exponent sends most lanes of a wave to the
+// same two counters, four times over.  Where the threshold's bin holds more than
+// kMaxCand keys, it is ties of one key (tokens without a score among them) or
+// is cut again (hard_threshold).  One workgroup's instructions per score bound
+// this kernel (1024 threads on one CU), not its loads.
+//
+// Microseconds of one 4096-score sequence, 16 x 16384, one of 40000, against
+// four radix passes: normal scores 7.8 / 11.3 / 23.4 (radix 11.1 / 19.8 / 39.8),
+// with an outlier of 1e30 or one -inf 7.8 / 11.3 / 24, 70% -inf 12.7 / 13.5 / 30
+// (12.2 / 19.8 / 39.7), Cauchy 8.3 / 15.6 / 29 (11 / 19.5 / 39), exp(3 normal)
+// 10.7 / 18.9 / 33 (11 / 18.6 / 38), two values 9.5 / 14.9 / 30 (13 / 25 / 51);
+// only zeros of both signs take longer, 18.5 / 32 / 60 (13 / 25 / 52).
 constexpr int kBins = 2048;
+constexpr int kBinBits = 11;
 constexpr int kMaxCand = 1024;
-static_assert(kBins == 2 * kSelThreads, "a thread owns two bins of the scan");
-static_assert(kMaxCand <= kSelThreads, "a thread ranks one candidate");
+constexpr int kRangeGroups = 16;  // of lanes, see select_segment
+constexpr int kRangeWaves = kSelThreads / 64 / (64 / kRangeGroups);
+static_assert(kBins == 1 << kBinBits && kBins == 2 * kSelThreads, "a thread owns two bins of the scan");
+constexpr int kMaxCompared = 256;  // candidates compared with each other, see rank_candidates
+static_assert(kMaxCompared <= kSplitThreads && kMaxCompared < kMaxCand, "a thread holds one of them");
+
+constexpr uint32_t kMinusInf = 0xff800000u;  // bits; NaNs with the sign set are above
 
 struct Picked {
   uint32_t thresh, need_eq, ties;  // key of the K-th largest score, its ties to keep, all its ties
 };
 
-// The threshold by four radix passes over the scores, by a workgroup of T threads.
-template <int T>
-__device__ __forceinline__ Picked radix_pick(const float* sc, int64_t start, int64_t stop, uint32_t need) {
-  __shared__ uint32_t whist[T / 64][256];
-  __shared__ uint32_t hist[256];
-  __shared__ uint32_t s_digit, s_need;
-  Picked p{0u, need, 0u};
-  uint32_t mask = 0;
-  for (int pass = 0; pass < 4; ++pass) {
-    const int shift = 24 - 8 * pass;
-    range_histogram<T>(sc, start, stop, p.thresh, mask, shift, whist, hist);
-    if (threadIdx.x < 64) pick_digit(hist, p.need_eq, &s_digit, &s_need);
-    __syncthreads();
-    p.thresh |= s_digit << shift;
-    mask |= 0xFFu << shift;
-    p.need_eq = s_need;
-    p.ties = hist[s_digit];
-    __syncthreads();
-  }
-  return p;
+__device__ __forceinline__ float key_float(uint32_t key) {
+  return __uint_as_float((key & 0x80000000u) ? key ^ 0x80000000u : ~key);
 }
 
-// Out of line, as select_long below: what most calls run stays small in the
-// instruction cache.
-__device__ __noinline__ Picked radix_threshold(const float* sc, int64_t start, int64_t stop, uint32_t need) {
-  return radix_pick<kSelThreads>(sc, start, stop, need);
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) <= 3.402823466e38f; }
+
+// Smallest and largest key of a set of scores, smallest and largest finite one.
+struct Range {
+  uint32_t kl, kh;
+  float lo, hi;
+};
+
+// The key with rank `need` from the top of the `count` <= kMaxCand keys of cand
+// (in LDS, 16-byte aligned), written to `out`.  A few dozen keys, the usual
+// number, are compared with each other.  More are held by one wave, 16 a lane
+// at most, which sets the threshold's bits from the top by the number of keys
+// at or above each trial: up to 4 us, where comparing 800 with each other took
+// 25 of the whole workgroup.  Every thread calls it.
+template <int T>
+__device__ __forceinline__ void rank_candidates(uint32_t* cand, uint32_t count, uint32_t need, Picked* out) {
+  constexpr int kWords = kMaxCand / 64;
+  const uint32_t padded = (count + 3) & ~3u;  // with the smallest key, corrected below
+  if (count <= kMaxCompared && threadIdx.x < padded - count) cand[count + threadIdx.x] = 0u;
+  __syncthreads();  // the keys are written
+  if (count <= kMaxCompared) {
+    if (threadIdx.x < count) {
+      const uint32_t mine = cand[threadIdx.x];
+      uint32_t g = 0, e = mine == 0u ? count - padded : 0u;
+      for (uint32_t k = 0; k < padded; k += 4) {
+        const uint4 o = *reinterpret_cast<const uint4*>(cand + k);
+        g += (o.x > mine) + (o.y > mine) + (o.z > mine) + (o.w > mine);
+        e += (o.x == mine) + (o.y == mine) + (o.z == mine) + (o.w == mine);
+      }
+      if (g < need && need <= g + e) *out = Picked{mine, need - g, e};  // equal keys write the same
+    }
+  } else if (threadIdx.x < 64) {
+    const uint32_t lane = threadIdx.x;
+    const int words = static_cast<int>((count + 63) / 64);
+    uint32_t key[kWords];
+#pragma unroll
+    for (int w = 0; w < kWords; ++w) key[w] = 64 * w + lane < count ? cand[64 * w + lane] : 0u;
+    auto at_least = [&](uint32_t trial) {
+      uint32_t n = 0;
+#pragma unroll
+      for (int w = 0; w < kWords; w += 4) {
+        if (w >= words) break;
+#pragma unroll
+        for (int v = w; v < w + 4; ++v) n += static_cast<uint32_t>(__popcll(__ballot(key[v] >= trial)));
+      }
+      return n;
+    };
+    const uint32_t base = __builtin_amdgcn_readfirstlane(key[0]);
+    uint32_t diff = 0;  // bits in which keys differ; those above are the threshold's
+#pragma unroll
+    for (int w = 0; w < kWords; ++w) diff |= 64 * w + lane < count ? key[w] ^ base : 0u;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) diff |= __shfl_xor(diff, off);
+    diff = __builtin_amdgcn_readfirstlane(diff);
+    uint32_t bit = diff ? 0x80000000u >> __clz(static_cast<int>(diff)) : 0u;
+    uint32_t thresh = bit ? base & ~(2 * bit - 1) : base;
+#pragma unroll 1
+    for (; bit; bit >>= 1)
+      if (at_least(thresh | bit) >= need) thresh |= bit;
+    // Padding equals a threshold of zero only.
+    const uint32_t more = diff == 0 || thresh == 0xffffffffu ? 0u : at_least(thresh + 1);
+    const uint32_t from = diff == 0 || thresh == 0u ? count : at_least(thresh);
+    if (lane == 0) *out = Picked{thresh, need - more, from - more};
+  }
+  __syncthreads();
+}
+
+// The union of the threads' ranges, by a workgroup of T threads.
+template <int T>
+__device__ __forceinline__ Range meet_ranges(Range r) {
+  __shared__ Range waves[T / 64];
+  auto meet = [&](int off) {
+    r.kl = min(r.kl, __shfl_xor(r.kl, off));
+    r.kh = max(r.kh, __shfl_xor(r.kh, off));
+    r.lo = fminf(r.lo, __shfl_xor(r.lo, off));
+    r.hi = fmaxf(r.hi, __shfl_xor(r.hi, off));
+  };
+#pragma unroll 1
+  for (int off = 32; off >= 1; off >>= 1) meet(off);
+  if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = r;
+  __syncthreads();
+  r = waves[threadIdx.x & (T / 64 - 1)];
+#pragma unroll 1
+  for (int off = T / 128; off >= 1; off >>= 1) meet(off);
+  __syncthreads();  // written again by the next call
+  return r;
+}
+
+// The range of the scores that `member` accepts, by a workgroup of T threads.
+template <int T, typename F>
+__device__ __forceinline__ Range member_range(const float* sc, int64_t start, int64_t stop, F&& member) {
+  Range r{0xffffffffu, 0u, INFINITY, -INFINITY};
+  for_each_score_rarely<T>(sc, start, stop, [&](float x) {
+    const uint32_t key = float_key(x);
+    if (member(x, key)) {
+      r.kl = min(r.kl, key);
+      r.kh = max(r.kh, key);
+      r.lo = fminf(r.lo, finite(x) ? x : INFINITY);
+      r.hi = fmaxf(r.hi, finite(x) ? x : -INFINITY);
+    }
+  });
+  return meet_ranges<T>(r);
+}
+
+// A workgroup's bins, kBinCopies counters each: lane l counts in copy l %
+// kBinCopies, so that lanes whose scores share a bin (ties, the crowded end of a
+// skewed range) wait for each other in smaller groups.
+constexpr int kBinCopies = 4;
+__device__ __forceinline__ uint32_t* shared_bins() {
+  __shared__ __attribute__((aligned(16))) uint32_t bins[kBins * kBinCopies];
+  return bins;
+}
+__device__ __forceinline__ uint32_t* shared_candidates() {
+  __shared__ __attribute__((aligned(16))) uint32_t cand[kMaxCand];
+  return cand;
+}
+template <int T>
+__device__ __forceinline__ void clear_bins() {
+  for (int i = threadIdx.x; i < kBins; i += T) reinterpret_cast<uint4*>(shared_bins())[i] = make_uint4(0, 0, 0, 0);
+}
+__device__ __forceinline__ void count_bin(int bin) {
+  atomicAdd(&shared_bins()[kBinCopies * bin + (threadIdx.x & (kBinCopies - 1))], 1u);
+}
+__device__ __forceinline__ uint32_t bin_total(int bin) {
+  const uint4 c = reinterpret_cast<const uint4*>(shared_bins())[bin];
+  return c.x + c.y + c.z + c.w;
+}
+
+// The need-th largest of the `count` scores of [start, stop) whose keys lie in
+// [r.kl, r.kh], by a workgroup of T threads: that range is cut into kBins bins
+// until at most kMaxCand keys share the threshold's bin, or it is one key.  Up
+// to twice the bins are equal in value (the end bins hold what is not finite):
+// what an outlier's bin holds spreads well.  Then they are equal in keys, which
+// takes kBinBits bits off the range a turn.
+template <int T>
+__device__ __noinline__ Picked pick_in_range(const float* sc, int64_t start, int64_t stop, uint32_t need, Range r,
+                                             uint32_t count) {
+  constexpr int kOwn = kBins / T;  // bins a thread owns in the scan
+  uint32_t* cand = shared_candidates();
+  __shared__ uint32_t s_wave[T / 64];
+  __shared__ uint32_t s_bin, s_need, s_count, s_filled;
+  __shared__ Picked s_picked;
+  const int tid = threadIdx.x;
+  for (int turn = 0; r.kl != r.kh; ++turn) {
+    const uint32_t kl = r.kl, span = r.kh - r.kl;
+    const float lo = 0.5f * r.lo;  // halves: no range overflows
+    const float scale = (kBins - 2 - 1.0f / 512.0f) / (0.5f * r.hi - lo);
+    const bool values = turn < 2 && r.hi > r.lo && scale > 0.0f && scale < INFINITY;
+    const int shift = max(32 - __clz(static_cast<int>(span)) - kBinBits, 0);
+    auto bin_of = [&](float x, uint32_t key) -> int {
+      if (!values) return static_cast<int>((key - kl) >> shift);
+      if (!finite(x)) return (key >> 31) ? kBins - 1 : 0;
+      return 1 + static_cast<int>((0.5f * x - lo) * scale);
+    };
+    clear_bins<T>();
+    if (tid == 0) s_filled = 0;
+    __syncthreads();
+    for_each_score_rarely<T>(sc, start, stop, [&](float x) {
+      const uint32_t key = float_key(x);
+      if (key - kl <= span) count_bin(bin_of(x, key));
+    });
+    __syncthreads();
+    // Thread order is falling order of the bins.
+    uint32_t c[kOwn], own = 0, total;
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q) own += c[q] = bin_total(kBins - 1 - kOwn * tid - q);
+    uint32_t above = block_exclusive_scan<T>(own, s_wave, &total);
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q) {
+      if (above < need && need <= above + c[q]) {
+        s_bin = static_cast<uint32_t>(kBins - 1 - kOwn * tid - q);
+        s_need = need - above;
+        s_count = c[q];
+      }
+      above += c[q];
+    }
+    __syncthreads();
+    const int bin = static_cast<int>(s_bin);
+    need = s_need;
+    count = s_count;
+    auto member = [&](float x, uint32_t key) { return key - kl <= span && bin_of(x, key) == bin; };
+    if (count <= kMaxCand) {
+      for_each_score_rarely<T>(sc, start, stop, [&](float x) {
+        const uint32_t key = float_key(x);
+        if (member(x, key)) cand[atomicAdd(&s_filled, 1u)] = key;
+      });
+      rank_candidates<T>(cand, count, need, &s_picked);
+      return s_picked;
+    }
+    if (!values && shift == 0) return Picked{kl + static_cast<uint32_t>(bin), need, count};
+    r = member_range<T>(sc, start, stop, member);
+  }
+  return Picked{r.kl, need, count};
+}
+
+// The first bins, from the largest scores down: a NaN counts in bin 0, where it
+// belongs unless its sign is set.
+__device__ __forceinline__ int value_bin(float x, float hi, float scale) {
+  return static_cast<int>(__builtin_amdgcn_fmed3f((hi - x) * scale, 0.0f, static_cast<float>(kBins - 1)));
+}
+
+// The threshold of scores that the first set of bins did not separate: the
+// need-th largest of the `count` scores with keys in [kl, kh], kl and kh among
+// them, or (kl > kh) of all scores.  Out of line, as select_long below: what
+// most calls run stays small in the instruction cache.
+__device__ __noinline__ Picked hard_threshold(const float* sc, int64_t start, int64_t stop, uint32_t need, uint32_t count,
+                                              uint32_t kl, uint32_t kh) {
+  Range r{kl, kh, key_float(kl), key_float(kh)};
+  if (kl > kh || !finite(r.lo) || !finite(r.hi))
+    r = member_range<kSelThreads>(sc, start, stop, [&](float, uint32_t key) { return kl > kh || key - kl <= kh - kl; });
+  return pick_in_range<kSelThreads>(sc, start, stop, need, r, count);
 }
 
 // Keeps the `keep` largest scores of [start, stop), their indices written from
@@ -488,11 +638,12 @@ __device__ __noinline__ Picked radix_threshold(const float* sc, int64_t start, i
 template <bool CACHED>
 __device__ __forceinline__ void select_segment(const float* sc, int64_t start, int64_t stop, uint32_t keep, int64_t* out,
                                                int out_base, int budget) {
-  __shared__ uint32_t bins[kBins];
-  __shared__ uint32_t cand[kMaxCand];
+  uint32_t* cand = shared_candidates();
   __shared__ uint32_t s_bin, s_need, s_count, s_filled;
+  __shared__ Picked s_picked;
   __shared__ uint32_t s_wave[kSelThreads / 64];
-  __shared__ float s_range[3][kSelThreads / 64];
+  __shared__ bool s_odd[kSelThreads / 64];
+  __shared__ float s_range[2][kSelThreads / 64][kRangeGroups];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int64_t misalign = (reinterpret_cast<uintptr_t>(sc + start) >> 2) & 3;
@@ -537,82 +688,122 @@ __device__ __forceinline__ void select_segment(const float* sc, int64_t start, i
     }
   };
 
-  // Range of the scores; `odd` ends as NaN if one of them is not finite.
-  for (int i = tid; i < kBins; i += kSelThreads) bins[i] = 0;
+  // The bins' range, from the smallest and largest score of each of
+  // kRangeGroups groups (every kRangeGroups-th lane): the largest of the
+  // smallest to the smallest of the largest, so that a few outliers or
+  // infinities do not stretch it.  odd: one of the scores is a NaN with its
+  // sign set, which has no place among these bins.
+  clear_bins<kSelThreads>();
   if (tid == 0) s_filled = 0;
-  float lo = INFINITY, hi = -INFINITY, odd = 0.0f;
+  float lo = INFINITY, hi = -INFINITY;
+  uint32_t bits = 0;
   walk([&](float x) {
     lo = fminf(lo, x);
     hi = fmaxf(hi, x);
-    odd = fmaf(x, 0.0f, odd);
+    bits = max(bits, __float_as_uint(x));
   });
+  bool odd = false;
+  if (__any(bits >= kMinusInf)) {  // not from tokens without a score
+    lo = INFINITY;
+    walk([&](float x) { lo = fminf(lo, x == -INFINITY ? INFINITY : x); });
+    odd = __any(bits > kMinusInf);
+  }
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
+  for (int off = 32; off >= kRangeGroups; off >>= 1) {
     lo = fminf(lo, __shfl_xor(lo, off));
     hi = fmaxf(hi, __shfl_xor(hi, off));
-    odd += __shfl_xor(odd, off);
   }
-  if (lane == 0) {
-    s_range[0][wave] = lo;
-    s_range[1][wave] = hi;
-    s_range[2][wave] = odd;
+  if (lane < kRangeGroups) {
+    s_range[0][wave][lane] = lo;
+    s_range[1][wave][lane] = hi;
   }
+  if (lane == 0) s_odd[wave] = odd;
   __syncthreads();
-  lo = s_range[0][0], hi = s_range[1][0], odd = s_range[2][0];
+  odd = __any(s_odd[lane & (kSelThreads / 64 - 1)]);
+  {
+    // Lane l: group l % kRangeGroups, a quarter of the waves.
+    const int group = lane & (kRangeGroups - 1), w0 = (lane / kRangeGroups) * kRangeWaves;
+    lo = s_range[0][w0][group], hi = s_range[1][w0][group];
 #pragma unroll
-  for (int w = 1; w < kSelThreads / 64; ++w) {
-    lo = fminf(lo, s_range[0][w]);
-    hi = fmaxf(hi, s_range[1][w]);
-    odd += s_range[2][w];
+    for (int w = 1; w < kRangeWaves; ++w) {
+      lo = fminf(lo, s_range[0][w0 + w][group]);
+      hi = fmaxf(hi, s_range[1][w0 + w][group]);
+    }
   }
-  // A little below kBins / (hi - lo), so that hi itself rounds to at most the last bin.
-  const float scale = (kBins - 1.0f / 512.0f) / (hi - lo);
-  auto bin_of = [&](float x) { return static_cast<int>((x - lo) * scale); };
+#pragma unroll
+  for (int off = 32; off >= kRangeGroups; off >>= 1) {
+    lo = fminf(lo, __shfl_xor(lo, off));
+    hi = fmaxf(hi, __shfl_xor(hi, off));
+  }
+  if (lo > hi) lo = -INFINITY, hi = INFINITY;  // a group without scores
+  static_assert(kRangeGroups == 16, "a row of lanes holds every group");
+  lo = fmaxf(lo, dpp_quad_xor1(lo)), hi = fminf(hi, dpp_quad_xor1(hi));
+  lo = fmaxf(lo, dpp_quad_xor2(lo)), hi = fminf(hi, dpp_quad_xor2(hi));
+  lo = fmaxf(lo, dpp_row_half_mirror(lo)), hi = fminf(hi, dpp_row_half_mirror(hi));
+  lo = fmaxf(lo, dpp_row_mirror(lo)), hi = fminf(hi, dpp_row_mirror(hi));
+  if (lo > hi) {  // groups apart from each other
+    const float t = lo;
+    lo = hi;
+    hi = t;
+  }
+  const float scale = static_cast<float>(kBins) / (hi - lo);
+  auto bin_of = [&](float x) { return value_bin(x, hi, scale); };
   Picked picked{0u, 0u, 0u};
-  // The same for every thread.  A range past float32 gives a scale of zero.
-  bool found = odd == 0.0f && hi > lo && scale > 0.0f && scale < INFINITY;
+  // The same for every thread.  A range past float32 gives a scale of zero, one
+  // of no width an infinity.
+  bool found = !odd && hi > lo && scale > 0.0f && scale < INFINITY;
+  // Where the bins leave off: the threshold's rank among `among` scores with
+  // keys in [kl, kh] (all scores).
+  uint32_t need = keep, among = static_cast<uint32_t>(stop - start), kl = 0xffffffffu, kh = 0;
   if (found) {
-    walk([&](float x) { atomicAdd(&bins[bin_of(x)], 1u); });
+    walk([&](float x) { count_bin(bin_of(x)); });
     __syncthreads();
-    // Thread t owns bins kBins - 1 - 2t and the one below it: thread order is
-    // falling order of the scores.
-    const uint32_t c0 = bins[kBins - 1 - 2 * tid], c1 = bins[kBins - 2 - 2 * tid];
+    // Thread t owns bins 2t and 2t + 1, in falling order of the scores.
+    const uint32_t c0 = bin_total(2 * tid), c1 = bin_total(2 * tid + 1);
     uint32_t total;
     uint32_t above = block_exclusive_scan<kSelThreads>(c0 + c1, s_wave, &total);
     if (above < keep && keep <= above + c0 + c1) {
       const bool first = keep <= above + c0;
       if (!first) above += c0;
-      s_bin = static_cast<uint32_t>(kBins - 1 - 2 * tid - (first ? 0 : 1));
+      s_bin = static_cast<uint32_t>(2 * tid + (first ? 0 : 1));
       s_need = keep - above;
       s_count = first ? c0 : c1;
     }
     __syncthreads();
     const int bin = static_cast<int>(s_bin);
     const uint32_t count = s_count, rank = s_need;
-    found = count <= kMaxCand;
-    if (found) {
+    if (count <= kMaxCand) {
       walk([&](float x) {
         if (bin_of(x) == bin) cand[atomicAdd(&s_filled, 1u)] = float_key(x);
       });
-      __syncthreads();
-      if (tid < count) {
-        const uint32_t mine = cand[tid];
-        uint32_t g = 0, e = 0;
-        for (uint32_t i = 0; i < count; ++i) {
-          g += cand[i] > mine;
-          e += cand[i] == mine;
+      rank_candidates<kSelThreads>(cand, count, rank, &s_picked);
+      picked = s_picked;
+    } else {
+      // Ties of one key fill the bin, or tokens without a score (-inf), or it
+      // has to be cut again.
+      uint32_t none = 0;
+      walk([&](float x) {
+        if (bin_of(x) == bin) {
+          if (x == -INFINITY) {
+            ++none;
+          } else {
+            kl = min(kl, float_key(x));
+            kh = max(kh, float_key(x));
+          }
         }
-        if (g < rank && rank <= g + e) {  // every candidate equal to the threshold writes the same
-          s_bin = mine;
-          s_need = rank - g;
-          s_count = e;
-        }
-      }
-      __syncthreads();
-      picked = Picked{s_bin, s_need, s_count};
+      });
+      if (none > 0) atomicAdd(&s_filled, none);
+      const Range r = meet_ranges<kSelThreads>(Range{kl, kh, 0.0f, 0.0f});
+      none = s_filled;
+      kl = r.kl;
+      kh = r.kh;
+      need = rank;
+      among = count - none;
+      found = need > among || kl == kh;
+      picked = need > among ? Picked{float_key(-INFINITY), need - among, none} : Picked{kl, need, among};
     }
   }
-  if (!found) picked = radix_threshold(sc, start, stop, keep);
+  if (!found) picked = hard_threshold(sc, start, stop, need, among, kl, kh);
   const Keep kp{picked.thresh, picked.need_eq, picked.ties == picked.need_eq, out, out_base, budget};
   if constexpr (CACHED) {
     uint32_t g_run = 0, e_run = 0;
@@ -657,12 +848,13 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(SelectArgs a) {
 // (no atomics, nothing to clear), every chunk of the second launch adds them
 // all, and the threshold's bin holds some hundred keys, ranked exactly.  More
 // than kSplitCand keys there are usually ties of one key, which is then the
-// threshold; if not, every chunk's workgroup makes radix passes over the whole
-// segment.
+// threshold; if not, every chunk's workgroup bins the whole segment's keys of
+// that bin again.
 constexpr int kSplitBins = 1024;
 constexpr int kSplitCand = 4096;
-constexpr int kSplitRanked = 512;  // candidates ranked against each other; more take radix passes over them
+constexpr int kSplitRanked = 1024;  // candidates ranked against each other; more are binned first
 constexpr int kSplitSamples = 1024;
+static_assert(kSplitRanked <= kMaxCand, "one wave ranks them");
 static_assert(kSplitBins == 4 * kSplitThreads, "a thread owns four bins");
 
 // Per-job scratch (in the caller's workspace), written before it is read by
@@ -885,24 +1077,13 @@ __global__ __launch_bounds__(kSplitThreads) void select_split_emit_kernel(Select
   if (count <= kSplitCand) {
     for (uint32_t i = tid; i < count; i += kSplitThreads) cand[i] = st->cand[i];
     if (count <= kSplitRanked) {
-      const uint32_t padded = (count + 3) & ~3u;  // with the smallest key, corrected below
-      for (uint32_t i = tid; i < padded; i += kSplitThreads) keys[i] = i < count ? float_key(st->cand[i]) : 0u;
-      __syncthreads();
-      for (uint32_t i = tid; i < count; i += kSplitThreads) {
-        const uint32_t mine = keys[i];
-        uint32_t more = 0, same = mine == 0u ? count - padded : 0u;
-        for (uint32_t q = 0; q < padded; q += 4) {
-          const uint4 other = *reinterpret_cast<const uint4*>(keys + q);
-          more += (other.x > mine) + (other.y > mine) + (other.z > mine) + (other.w > mine);
-          same += (other.x == mine) + (other.y == mine) + (other.z == mine) + (other.w == mine);
-        }
-        if (more < rank && rank <= more + same) s_picked = Picked{mine, rank - more, same};  // equal keys write the same
-      }
-      __syncthreads();
+      for (uint32_t i = tid; i < count; i += kSplitThreads) keys[i] = float_key(st->cand[i]);
+      rank_candidates<kSplitThreads>(keys, count, rank, &s_picked);
       p = s_picked;
     } else {
       __syncthreads();
-      p = radix_pick<kSplitThreads>(cand, 0, count, rank);
+      const Range r = member_range<kSplitThreads>(cand, 0, count, [](float, uint32_t) { return true; });
+      p = pick_in_range<kSplitThreads>(cand, 0, count, rank, r, count);
     }
     for (uint32_t i = tid; i < before; i += kSplitThreads) {
       const uint32_t key = float_key(cand[i]);
@@ -915,9 +1096,10 @@ __global__ __launch_bounds__(kSplitThreads) void select_split_emit_kernel(Select
     if (tid < k.c) g += st->above[tid];
     if (tid == 0) e = before;
   } else {
-    p = radix_pick<kSplitThreads>(sc, k.j.s.start, k.j.s.stop, static_cast<uint32_t>(k.j.s.keep));
+    const Range r{least, most, key_float(least), key_float(most)};
+    p = pick_in_range<kSplitThreads>(sc, k.j.s.start, k.j.s.stop, rank, r, count);
     if (k.c > 0)
-      for_each_score<kSplitThreads>(sc, k.j.s.start, k.start, [&](float x) {
+      for_each_score_rarely<kSplitThreads>(sc, k.j.s.start, k.start, [&](float x) {
         const uint32_t key = float_key(x);
         g += key > p.thresh;
         e += key == p.thresh;
