@@ -841,6 +841,9 @@ def _hard_scores(kind: str, n: int, g: torch.Generator) -> torch.Tensor:
         x[at[: n // 5]] *= 1e-8
         x[at[n // 5 : n // 4]] *= 1e12
         x[at[n // 4 : n // 4 + 100]] *= 3e37
+    elif kind == "clipped":  # ties beside a few others in their bin
+        x = x.clamp(-0.5, 0.8)
+        x[at[: n // 20]] += 1e-6
     elif kind == "zeros":
         x = torch.where(x > 0, 0.0, -0.0)
     elif kind == "subnormal":
@@ -851,7 +854,7 @@ def _hard_scores(kind: str, n: int, g: torch.Generator) -> torch.Tensor:
 
 
 @pytest.mark.parametrize("shape", ["single", "split"])
-@pytest.mark.parametrize("kind", ["both-infinities", "nans", "heavy-tail", "two-scales", "zeros", "subnormal", "trend"])
+@pytest.mark.parametrize("kind", ["both-infinities", "nans", "heavy-tail", "two-scales", "clipped", "zeros", "subnormal", "trend"])
 def test_select_scores_binned_again(hip_device, kind, shape) -> None:
     # Lengths around the cached form's limit (16384 scores), one chunk and
     # longer chunks; keep counts that put the threshold into every kind of bin.

@@ -524,12 +524,15 @@ __device__ __forceinline__ Range member_range(const float* sc, int64_t start, in
   return meet_ranges<T>(r);
 }
 
-// A workgroup's bins, kBinCopies counters each: lane l counts in copy l %
-// kBinCopies, so that lanes whose scores share a bin (ties, the crowded end of a
-// skewed range) wait for each other in smaller groups.
-constexpr int kBinCopies = 4;
+// The bins of a workgroup of T threads, kBinCopies counters each: lane l counts
+// in copy l % kBinCopies, so that lanes whose scores share a bin (ties, the
+// crowded end of a skewed range) wait for each other in smaller groups.  One
+// counter where chunks' workgroups share a CU, and its LDS.
+template <int T>
+constexpr int kBinCopies = T == kSelThreads ? 4 : 1;
+template <int T>
 __device__ __forceinline__ uint32_t* shared_bins() {
-  __shared__ __attribute__((aligned(16))) uint32_t bins[kBins * kBinCopies];
+  __shared__ __attribute__((aligned(16))) uint32_t bins[kBins * kBinCopies<T>];
   return bins;
 }
 __device__ __forceinline__ uint32_t* shared_candidates() {
@@ -538,13 +541,18 @@ __device__ __forceinline__ uint32_t* shared_candidates() {
 }
 template <int T>
 __device__ __forceinline__ void clear_bins() {
-  for (int i = threadIdx.x; i < kBins; i += T) reinterpret_cast<uint4*>(shared_bins())[i] = make_uint4(0, 0, 0, 0);
+  for (int i = threadIdx.x; i < kBins * kBinCopies<T> / 4; i += T)
+    reinterpret_cast<uint4*>(shared_bins<T>())[i] = make_uint4(0, 0, 0, 0);
 }
+template <int T>
 __device__ __forceinline__ void count_bin(int bin) {
-  atomicAdd(&shared_bins()[kBinCopies * bin + (threadIdx.x & (kBinCopies - 1))], 1u);
+  atomicAdd(&shared_bins<T>()[kBinCopies<T> * bin + (threadIdx.x & (kBinCopies<T> - 1))], 1u);
 }
+template <int T>
 __device__ __forceinline__ uint32_t bin_total(int bin) {
-  const uint4 c = reinterpret_cast<const uint4*>(shared_bins())[bin];
+  if constexpr (kBinCopies<T> == 1) return shared_bins<T>()[bin];
+  static_assert(kBinCopies<T> == 1 || kBinCopies<T> == 4, "read as one word");
+  const uint4 c = reinterpret_cast<const uint4*>(shared_bins<T>())[bin];
   return c.x + c.y + c.z + c.w;
 }
 
@@ -579,13 +587,13 @@ __device__ __noinline__ Picked pick_in_range(const float* sc, int64_t start, int
     __syncthreads();
     for_each_score_rarely<T>(sc, start, stop, [&](float x) {
       const uint32_t key = float_key(x);
-      if (key - kl <= span) count_bin(bin_of(x, key));
+      if (key - kl <= span) count_bin<T>(bin_of(x, key));
     });
     __syncthreads();
     // Thread order is falling order of the bins.
     uint32_t c[kOwn], own = 0, total;
 #pragma unroll
-    for (int q = 0; q < kOwn; ++q) own += c[q] = bin_total(kBins - 1 - kOwn * tid - q);
+    for (int q = 0; q < kOwn; ++q) own += c[q] = bin_total<T>(kBins - 1 - kOwn * tid - q);
     uint32_t above = block_exclusive_scan<T>(own, s_wave, &total);
 #pragma unroll
     for (int q = 0; q < kOwn; ++q) {
@@ -756,10 +764,10 @@ __device__ __forceinline__ void select_segment(const float* sc, int64_t start, i
   // keys in [kl, kh] (all scores).
   uint32_t need = keep, among = static_cast<uint32_t>(stop - start), kl = 0xffffffffu, kh = 0;
   if (found) {
-    walk([&](float x) { count_bin(bin_of(x)); });
+    walk([&](float x) { count_bin<kSelThreads>(bin_of(x)); });
     __syncthreads();
     // Thread t owns bins 2t and 2t + 1, in falling order of the scores.
-    const uint32_t c0 = bin_total(2 * tid), c1 = bin_total(2 * tid + 1);
+    const uint32_t c0 = bin_total<kSelThreads>(2 * tid), c1 = bin_total<kSelThreads>(2 * tid + 1);
     uint32_t total;
     uint32_t above = block_exclusive_scan<kSelThreads>(c0 + c1, s_wave, &total);
     if (above < keep && keep <= above + c0 + c1) {
@@ -841,15 +849,22 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(SelectArgs a) {
 
 // The threshold of a long segment, in three launches (seven when four radix
 // passes named it, a clear before and a count after: 4 x 130816 scores 37.7 us
-// against 19.7 now).  Bins are equal cells of a range taken from a sample, a
-// little wider at the top, so no launch has to find the range first: any range
-// is right, since scores past it count in the end bins, and the bins only have
-// to keep the order of the keys.  Every chunk stores a histogram of its own
+// against 19.7 now).  Bins are equal cells of a range taken from a sample, so no
+// launch has to find the range first: any range is right, since scores past it
+// count in the last bins, and the bins only have to keep the order of the keys.  Every chunk stores a histogram of its own
 // (no atomics, nothing to clear), every chunk of the second launch adds them
 // all, and the threshold's bin holds some hundred keys, ranked exactly.  More
-// than kSplitCand keys there are usually ties of one key, which is then the
-// threshold; if not, every chunk's workgroup bins the whole segment's keys of
-// that bin again.
+// than kSplitCand keys there are usually ties of one key and a few others: the
+// second launch counts the keys equal to and above one of them.  Where that does
+// not name the threshold, every chunk's workgroup bins the whole segment's keys
+// of that bin again (ten times the usual time, so the bins' range is chosen to
+// make it rare).
+//
+// Microseconds of 4 x 131072 scores, keep 4608 of each, against the seven
+// launches: normal 20 (38.4), an outlier of 1e30 20 (38.5), 70% -inf 21 (38.5),
+// Cauchy 19 (38.4), exp(3 normal) 19 (38.5), two values 25 (39), one value 26
+// (39).  262144 scores of exp(3 normal) of which 100000 are kept, 8000 in the
+// threshold's bin, take 270 (42).
 constexpr int kSplitBins = 1024;
 constexpr int kSplitCand = 4096;
 constexpr int kSplitRanked = 1024;  // candidates ranked against each other; more are binned first
@@ -862,8 +877,14 @@ static_assert(kSplitBins == 4 * kSplitThreads, "a thread owns four bins");
 struct SplitState {
   float lo, scale;             // bin of x: (x - lo) * scale
   uint32_t rank, count;        // the threshold's rank from the top of its bin, keys in that bin
-  uint32_t least[kSplitMaxChunks];   // smallest and largest key of the bin in a
-  uint32_t most[kSplitMaxChunks];    // chunk, where the bin is too full for cand
+  // Where the bin is too full for cand: one of its keys (a sample's, probably the
+  // ties'), and per chunk the keys equal to it and above it, and the smallest and
+  // largest of the others.
+  uint32_t tie, reserved[3];
+  uint32_t equal[kSplitMaxChunks];
+  uint32_t higher[kSplitMaxChunks];
+  uint32_t least[kSplitMaxChunks];
+  uint32_t most[kSplitMaxChunks];
   uint32_t above[kSplitMaxChunks];   // a chunk's keys in higher bins
   uint32_t before[kSplitMaxChunks];  // candidates of the chunks before
   uint32_t hist[kSplitMaxChunks][kSplitBins];
@@ -885,11 +906,15 @@ __device__ __forceinline__ SplitState* split_state(const SelectArgs& a, int b, i
   return static_cast<SplitState*>(a.state) + static_cast<int64_t>(b) * a.segments + seg;
 }
 
-// Order-preserving bin of a score.  Infinities and NaNs go by their key (sign
-// set: below every score); a scale of zero puts every finite score in bin 0.
+// Place of sample i in a segment of len scores.
+__device__ __forceinline__ int64_t sample_at(int64_t i, int64_t len) { return i * len / kSplitSamples; }
+
+// Order-preserving bin of a score.  Infinities and NaNs have the end bins to
+// themselves, by their sign (many tokens without a score are then one key); a
+// scale of zero puts every finite score in bin 1.
 __device__ __forceinline__ int split_bin(float x, float lo, float scale) {
-  if (!(fabsf(x) <= 3.402823466e38f)) return (float_key(x) >> 31) ? kSplitBins - 1 : 0;
-  return static_cast<int>(fminf(fmaxf((x - lo) * scale, 0.0f), static_cast<float>(kSplitBins - 1)));
+  if (!finite(x)) return (float_key(x) >> 31) ? kSplitBins - 1 : 0;
+  return static_cast<int>(fminf(fmaxf((x - lo) * scale, 1.0f), static_cast<float>(kSplitBins - 2)));
 }
 
 // The chunk of this workgroup (grid: chunks, segments, n_seq).
@@ -918,7 +943,7 @@ __device__ __forceinline__ Chunk make_chunk(const SelectArgs& a) {
 // range, the chunk's histogram.
 __global__ __launch_bounds__(kSplitThreads) void select_split_bins_kernel(SelectArgs a) {
   __shared__ __attribute__((aligned(16))) uint32_t bins[kSplitBins];
-  __shared__ float s_lo[kSplitThreads / 64], s_hi[kSplitThreads / 64];
+  __shared__ float s_range[2][kSplitThreads / 64][kRangeGroups];
   const int tid = threadIdx.x;
   const Chunk k = make_chunk(a);
   if (k.c == 0)
@@ -931,31 +956,38 @@ __global__ __launch_bounds__(kSplitThreads) void select_split_bins_kernel(Select
   float x[kSplitSamples / kSplitThreads];
 #pragma unroll
   for (int u = 0; u < kSplitSamples / kSplitThreads; ++u)
-    x[u] = sc[k.j.s.start + (tid + kSplitThreads * u) * len / kSplitSamples];
+    x[u] = sc[k.j.s.start + sample_at(tid + kSplitThreads * u, len)];
 #pragma unroll
   for (int u = 0; u < kSplitSamples / kSplitThreads; ++u) {
-    const bool finite = fabsf(x[u]) <= 3.402823466e38f;
-    lo = fminf(lo, finite ? x[u] : INFINITY);
-    hi = fmaxf(hi, finite ? x[u] : -INFINITY);
+    lo = fminf(lo, finite(x[u]) ? x[u] : INFINITY);
+    hi = fmaxf(hi, finite(x[u]) ? x[u] : -INFINITY);
   }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    lo = fminf(lo, __shfl_xor(lo, off));
-    hi = fmaxf(hi, __shfl_xor(hi, off));
-  }
-  if ((tid & 63) == 0) {
-    s_lo[tid >> 6] = lo;
-    s_hi[tid >> 6] = hi;
+  // Smallest and largest sample of each group of lanes l % kRangeGroups.
+  lo = fminf(lo, __shfl_xor(lo, 32)), hi = fmaxf(hi, __shfl_xor(hi, 32));
+  lo = fminf(lo, __shfl_xor(lo, 16)), hi = fmaxf(hi, __shfl_xor(hi, 16));
+  const int group = tid & (kRangeGroups - 1);
+  if ((tid & 63) < kRangeGroups) {
+    s_range[0][tid >> 6][group] = lo;
+    s_range[1][tid >> 6][group] = hi;
   }
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < kSplitThreads / 64; ++w) {
-    lo = fminf(lo, s_lo[w]);
-    hi = fmaxf(hi, s_hi[w]);
+    lo = fminf(lo, s_range[0][w][group]);
+    hi = fmaxf(hi, s_range[1][w][group]);
   }
-  const float width = hi - lo;
-  lo -= 0.125f * width;
-  float scale = kSplitBins / (1.625f * width);
+  if (lo > hi) lo = -INFINITY, hi = INFINITY;  // a group without scores
+  // The largest of the groups' smallest to the smallest of their largest: a few
+  // outliers do not stretch the range.  Of normal scores it ends at about 1.75
+  // standard deviations.  The bins reach further, above all at the top, where
+  // the threshold of a small budget lies.
+  lo = fmaxf(lo, dpp_quad_xor1(lo)), hi = fminf(hi, dpp_quad_xor1(hi));
+  lo = fmaxf(lo, dpp_quad_xor2(lo)), hi = fminf(hi, dpp_quad_xor2(hi));
+  lo = fmaxf(lo, dpp_row_half_mirror(lo)), hi = fminf(hi, dpp_row_half_mirror(hi));
+  lo = fmaxf(lo, dpp_row_mirror(lo)), hi = fminf(hi, dpp_row_mirror(hi));
+  const float width = fabsf(hi - lo);  // groups apart from each other: hi < lo
+  lo = fminf(lo, hi) - 0.25f * width;
+  float scale = kSplitBins / (3.0f * width);
   if (!(width > 0.0f && scale > 0.0f && scale < INFINITY && fabsf(lo) < INFINITY)) {
     lo = 0.0f;
     scale = 0.0f;
@@ -974,13 +1006,16 @@ __global__ __launch_bounds__(kSplitThreads) void select_split_bins_kernel(Select
 // of that bin and its number of keys in higher ones.
 __global__ __launch_bounds__(kSplitThreads) void select_split_candidates_kernel(SelectArgs a) {
   __shared__ uint32_t s_wave[kSplitThreads / 64];
-  __shared__ uint32_t s_bin, s_rank, s_count, s_before, s_filled, s_least, s_most;
+  __shared__ uint32_t s_bin, s_rank, s_count, s_before, s_filled, s_least, s_most, s_first, s_equal, s_higher;
   const int tid = threadIdx.x;
   const Chunk k = make_chunk(a);
   if (!k.live) return;
   if (tid == 0) {
     s_least = 0xffffffffu;
     s_most = 0;
+    s_first = kSplitSamples;
+    s_equal = 0;
+    s_higher = 0;
   }
   SplitState* st = split_state(a, blockIdx.z, blockIdx.y);
   const uint32_t keep = static_cast<uint32_t>(k.j.s.keep);
@@ -1037,26 +1072,58 @@ __global__ __launch_bounds__(kSplitThreads) void select_split_candidates_kernel(
     });
     return;
   }
-  uint32_t least = 0xffffffffu, most = 0;
+  // The same sample for every chunk: the first in the bin.
+  const int64_t len = k.j.s.stop - k.j.s.start;
+  float x[kSplitSamples / kSplitThreads];
+#pragma unroll
+  for (int u = 0; u < kSplitSamples / kSplitThreads; ++u) x[u] = sc[k.j.s.start + sample_at(tid + kSplitThreads * u, len)];
+#pragma unroll
+  for (int u = kSplitSamples / kSplitThreads - 1; u >= 0; --u) {
+    const uint64_t in = __ballot(split_bin(x[u], lo, scale) == bin);
+    if (in && (tid & 63) == 0) atomicMin(&s_first, static_cast<uint32_t>(tid + kSplitThreads * u + __ffsll(static_cast<unsigned long long>(in)) - 1));
+  }
+  __syncthreads();
+  const uint32_t tie = s_first < kSplitSamples ? float_key(sc[k.j.s.start + sample_at(s_first, len)]) : 0u;
+  uint32_t least = 0xffffffffu, most = 0, equal = 0, above_tie = 0;
   for_each_score<kSplitThreads>(sc, k.start, k.stop, [&](float x) {
     if (split_bin(x, lo, scale) == bin) {
-      least = min(least, float_key(x));
-      most = max(most, float_key(x));
+      const uint32_t key = float_key(x);
+      if (key == tie) {
+        ++equal;
+      } else {
+        above_tie += key > tie;
+        least = min(least, key);
+        most = max(most, key);
+      }
     }
   });
-  atomicMin(&s_least, least);
-  atomicMax(&s_most, most);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    least = min(least, __shfl_xor(least, off));
+    most = max(most, __shfl_xor(most, off));
+    equal += __shfl_xor(equal, off);
+    above_tie += __shfl_xor(above_tie, off);
+  }
+  if ((tid & 63) == 0) {
+    atomicMin(&s_least, least);
+    atomicMax(&s_most, most);
+    atomicAdd(&s_equal, equal);
+    atomicAdd(&s_higher, above_tie);
+  }
   __syncthreads();
   if (tid == 0) {
     st->least[k.c] = s_least;
     st->most[k.c] = s_most;
+    st->equal[k.c] = s_equal;
+    st->higher[k.c] = s_higher;
+    if (k.c == 0) st->tie = tie;
   }
 }
 
 // Launch 3: the threshold among the candidates, and the chunk's ordered emission.
-__global__ __launch_bounds__(kSplitThreads) void select_split_emit_kernel(SelectArgs a) {
+__global__ __launch_bounds__(kSplitThreads, 4) void select_split_emit_kernel(SelectArgs a) {
   __shared__ __attribute__((aligned(16))) float cand[kSplitCand];
-  __shared__ __attribute__((aligned(16))) uint32_t keys[kSplitRanked];
+  uint32_t* keys = shared_candidates();
   __shared__ uint32_t s_wave[kSplitThreads / 64];
   __shared__ Picked s_picked;
   const int tid = threadIdx.x;
@@ -1068,12 +1135,6 @@ __global__ __launch_bounds__(kSplitThreads) void select_split_emit_kernel(Select
   Picked p;
   uint32_t g = 0, e = 0;  // this thread's share of the keys > and == the threshold before the chunk
   const uint32_t before = st->before[k.c];
-  uint32_t least = 0xffffffffu, most = 0;
-  if (count > kSplitCand)
-    for (int c = 0; c < k.chunks; ++c) {
-      least = min(least, st->least[c]);
-      most = max(most, st->most[c]);
-    }
   if (count <= kSplitCand) {
     for (uint32_t i = tid; i < count; i += kSplitThreads) cand[i] = st->cand[i];
     if (count <= kSplitRanked) {
@@ -1091,19 +1152,37 @@ __global__ __launch_bounds__(kSplitThreads) void select_split_emit_kernel(Select
       e += key == p.thresh;
     }
     if (tid < k.c) g += st->above[tid];
-  } else if (least == most) {  // ties of one key fill the bin
-    p = Picked{least, rank, count};
-    if (tid < k.c) g += st->above[tid];
-    if (tid == 0) e = before;
   } else {
-    const Range r{least, most, key_float(least), key_float(most)};
-    p = pick_in_range<kSplitThreads>(sc, k.j.s.start, k.j.s.stop, rank, r, count);
-    if (k.c > 0)
-      for_each_score_rarely<kSplitThreads>(sc, k.j.s.start, k.start, [&](float x) {
-        const uint32_t key = float_key(x);
-        g += key > p.thresh;
-        e += key == p.thresh;
-      });
+    const uint32_t tie = st->tie;
+    uint32_t least = 0xffffffffu, most = 0, equal = 0, higher = 0, equal_before = 0, higher_before = 0;
+    for (int c = 0; c < k.chunks; ++c) {
+      if (c == k.c) equal_before = equal, higher_before = higher;
+      least = min(least, st->least[c]);
+      most = max(most, st->most[c]);
+      equal += st->equal[c];
+      higher += st->higher[c];
+    }
+    if (tid < k.c) g += st->above[tid];
+    if (higher < rank && rank <= higher + equal) {  // the ties' key
+      p = Picked{tie, rank - higher, equal};
+      if (tid == 0) g += higher_before, e = equal_before;
+    } else if (least == most) {  // the others are one key
+      const bool below = least < tie;
+      p = Picked{least, below ? rank - equal : rank, count - equal};
+      if (tid == 0) g += below ? equal_before : 0u, e = before - equal_before;
+    } else {
+      least = min(least, equal > 0 ? tie : least);
+      most = max(most, equal > 0 ? tie : most);
+      const Range r{least, most, key_float(least), key_float(most)};
+      p = pick_in_range<kSplitThreads>(sc, k.j.s.start, k.j.s.stop, rank, r, count);
+      g = 0;
+      if (k.c > 0)
+        for_each_score_rarely<kSplitThreads>(sc, k.j.s.start, k.start, [&](float x) {
+          const uint32_t key = float_key(x);
+          g += key > p.thresh;
+          e += key == p.thresh;
+        });
+    }
   }
   uint32_t g0, e0;
   block_exclusive_scan<kSplitThreads>(g, s_wave, &g0);
