@@ -397,10 +397,11 @@ constexpr int kCacheWords = 4;
 //
 // Microseconds of one 4096-score sequence, 16 x 16384, one of 40000, against
 // four radix passes: normal scores 7.8 / 11.3 / 23.4 (radix 11.1 / 19.8 / 39.8),
-// with an outlier of 1e30 or one -inf 7.8 / 11.3 / 24, 70% -inf 12.7 / 13.5 / 30
-// (12.2 / 19.8 / 39.7), Cauchy 8.3 / 15.6 / 29 (11 / 19.5 / 39), exp(3 normal)
-// 10.7 / 18.9 / 33 (11 / 18.6 / 38), two values 9.5 / 14.9 / 30 (13 / 25 / 51);
-// only zeros of both signs take longer, 18.5 / 32 / 60 (13 / 25 / 52).
+// with an outlier of 1e30 or one -inf 7.8 / 11.3 / 24, 70% -inf 11.4 / 13.6 / 30
+// (12.2 / 19.8 / 39.7), Cauchy 8.2 / 15.6 / 29 (11 / 19.5 / 39), exp(3 normal)
+// 10.7 / 18.7 / 33 (11 / 18.6 / 38), two values 11.3 / 17.9 / 36 (13 / 25 / 51),
+// clipped at one standard deviation 7.7 / 11.6 / 33 (11 / 20 / 47); only zeros
+// of both signs take longer, 18 / 31 / 59 (13 / 25 / 52).
 constexpr int kBins = 2048;
 constexpr int kBinBits = 11;
 constexpr int kMaxCand = 1024;
@@ -647,7 +648,7 @@ template <bool CACHED>
 __device__ __forceinline__ void select_segment(const float* sc, int64_t start, int64_t stop, uint32_t keep, int64_t* out,
                                                int out_base, int budget) {
   uint32_t* cand = shared_candidates();
-  __shared__ uint32_t s_bin, s_need, s_count, s_filled;
+  __shared__ uint32_t s_bin, s_need, s_count, s_filled, s_tie, s_sums[3];
   __shared__ Picked s_picked;
   __shared__ uint32_t s_wave[kSelThreads / 64];
   __shared__ bool s_odd[kSelThreads / 64];
@@ -702,7 +703,7 @@ __device__ __forceinline__ void select_segment(const float* sc, int64_t start, i
   // infinities do not stretch it.  odd: one of the scores is a NaN with its
   // sign set, which has no place among these bins.
   clear_bins<kSelThreads>();
-  if (tid == 0) s_filled = 0;
+  if (tid == 0) s_filled = s_sums[0] = s_sums[1] = s_sums[2] = 0;
   float lo = INFINITY, hi = -INFINITY;
   uint32_t bits = 0;
   walk([&](float x) {
@@ -787,28 +788,56 @@ __device__ __forceinline__ void select_segment(const float* sc, int64_t start, i
       rank_candidates<kSelThreads>(cand, count, rank, &s_picked);
       picked = s_picked;
     } else {
-      // Ties of one key fill the bin, or tokens without a score (-inf), or it
-      // has to be cut again.
-      uint32_t none = 0;
+      // Tokens without a score (-inf) fill the bin, or ties of one key (probably
+      // that of the member found first) beside a few others, or it has to be cut
+      // again.
+      walk([&](float x) {
+        if (x != -INFINITY && bin_of(x) == bin) s_tie = float_key(x);
+      });
+      __syncthreads();
+      const uint32_t tie = s_tie;
+      uint32_t none = 0, equal = 0, higher = 0;
       walk([&](float x) {
         if (bin_of(x) == bin) {
+          const uint32_t key = float_key(x);
           if (x == -INFINITY) {
             ++none;
+          } else if (key == tie) {
+            ++equal;
           } else {
-            kl = min(kl, float_key(x));
-            kh = max(kh, float_key(x));
+            higher += key > tie;
+            kl = min(kl, key);
+            kh = max(kh, key);
           }
         }
       });
-      if (none > 0) atomicAdd(&s_filled, none);
+#pragma unroll 1
+      for (int off = 32; off >= 1; off >>= 1) {
+        none += __shfl_xor(none, off);
+        equal += __shfl_xor(equal, off);
+        higher += __shfl_xor(higher, off);
+      }
+      if (lane == 0) {
+        atomicAdd(&s_sums[0], none);
+        atomicAdd(&s_sums[1], equal);
+        atomicAdd(&s_sums[2], higher);
+      }
       const Range r = meet_ranges<kSelThreads>(Range{kl, kh, 0.0f, 0.0f});
-      none = s_filled;
-      kl = r.kl;
-      kh = r.kh;
+      none = s_sums[0], equal = s_sums[1], higher = s_sums[2];
       need = rank;
       among = count - none;
-      found = need > among || kl == kh;
-      picked = need > among ? Picked{float_key(-INFINITY), need - among, none} : Picked{kl, need, among};
+      found = true;
+      if (need > among) {
+        picked = Picked{float_key(-INFINITY), need - among, none};
+      } else if (higher < need && need <= higher + equal) {
+        picked = Picked{tie, need - higher, equal};
+      } else if (r.kl == r.kh) {  // the others are one key
+        picked = Picked{r.kl, r.kl < tie ? need - equal : need, among - equal};
+      } else {
+        found = false;
+        kl = min(r.kl, tie);
+        kh = max(r.kh, tie);
+      }
     }
   }
   if (!found) picked = hard_threshold(sc, start, stop, need, among, kl, kh);
