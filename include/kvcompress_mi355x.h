@@ -277,9 +277,9 @@ int kvc_select_keep(kvc_stream_t stream, int n_seq, int max_seq_len, const int32
  * that one workgroup per sequence would leave on a few CUs.  Identical output
  * to kvc_select_keep.  No counterpart in the reference beyond
  * select_keep_indices itself.  `workspace`: at least
- * kvc_select_workspace_bytes(n_seq, segments, policy) bytes, 16-byte aligned,
- * any contents; max_seq_len must bound every
- * sequence length. */
+ * kvc_select_workspace_bytes(n_seq, segments, policy) bytes (about 149 KB a
+ * sequence's segment), 16-byte aligned, any contents; max_seq_len must bound
+ * every sequence length. */
 size_t kvc_select_workspace_bytes(int n_seq, int segments, int policy);
 int kvc_select_keep_split(kvc_stream_t stream, int n_seq, int max_seq_len, const int32_t* seq_lens,
                           const int64_t* token_offsets, const float* scores, int budget,

@@ -472,3 +472,21 @@ def test_batch_length_past_32_bits_is_a_runtime_error(hip_device) -> None:
 
     with pytest.raises(RuntimeError, match="32 bits"):
         Batch.build(hip_device, [1 << 31], [5], [torch.zeros(1 << 24, dtype=torch.int64, device=hip_device)])
+
+
+def test_forced_split_selection_beyond_the_rule(hip_device) -> None:
+    """A pipeline holds chunked-selection scratch for the batches the rule sends
+    there, none for these; a forced shape allocates it once and selects the same
+    indices."""
+    from kvcompress_mi355x import workloads
+
+    spec = workloads.config_spec(2, n_layers=2, score_layer_stride=1, seq_lens=(900, 1300, 700, 1200), budget=512, recent=64,
+                                 max_model_len=65536)
+    pipeline, batch = workloads.build_pipeline(workloads.build_synthetic_cache(spec, hip_device, seed=11))
+    assert pipeline.select_ws.numel() == 16
+    keep = pipeline.select_step(batch).clone()
+    assert pipeline.select_ws_forced is None
+    pipeline.select_shape = "split"
+    assert torch.equal(pipeline.select(batch), keep)
+    held = pipeline.select_ws_forced
+    assert torch.equal(pipeline.select(batch), keep) and pipeline.select_ws_forced is held

@@ -601,3 +601,18 @@ def test_launches_refuse_host_tensors(monkeypatch):
             offsets, offsets, num_pages=3, page_stride=128, row_elems=1, seq_lens=lens, src_block_offsets=offsets,
             src_block_ids=offsets, dst_block_offsets=None, dst_block_ids=None, keep=keep, budget=100)
     assert launched == []
+
+
+def test_split_scratch_covers_the_batches_the_rule_sends_there():
+    """Every batch that prefers_split accepts fits the scratch that a pipeline
+    of its capacity holds; where the rule accepts none, none is held."""
+    from kvcompress_mi355x.methods.triattention import selection
+
+    for policy, segments in (("global", 8), ("v3", 1), ("v3", 3), ("v3", 8), ("v3", 40)):
+        windows = dict(protected_prefix=4, protected_recent=128, segments=segments, policy=policy)
+        for max_len in (4096, 49283, 49284, 147583, 147592, 393400, 1 << 20):
+            for max_seqs in (1, 3, 31, 33, 256):
+                cap = selection.split_capacity(max_seqs, max_len, **windows)
+                accepted = [n for n in range(1, max_seqs + 1) if selection.prefers_split([max_len] * n, **windows)]
+                assert cap == max(accepted, default=0), (policy, segments, max_len, max_seqs)
+                assert cap * (segments if policy == "v3" else 1) <= selection.SPLIT_MAX_JOBS

@@ -34,7 +34,14 @@ import torch
 from ... import _native
 from . import _device as dev
 from .cache import compact_layers, compact_workspace_bytes, rewrite_block_tables
-from .selection import POLICY_CODES, prefers_split, select_keep_indices_batched, select_workspace, validate_selection
+from .selection import (
+    POLICY_CODES,
+    prefers_split,
+    select_keep_indices_batched,
+    select_workspace,
+    split_capacity,
+    validate_selection,
+)
 
 
 @dataclass(frozen=True)
@@ -297,7 +304,18 @@ class CompressionPipeline:
         self.var = torch.empty_like(self.mean)
         self.agg = torch.empty(self.max_tokens, dtype=torch.float32, device=dev_)
         self.keep = torch.empty((self.max_seqs, self.budget), dtype=torch.int64, device=dev_)
-        self.select_ws = select_workspace(self.max_seqs, self.segments, self.policy, dev_)
+        # Scratch of the chunked selection for the batches that take it by rule;
+        # a forced shape takes its own (_split_workspace).
+        self.select_ws_seqs = split_capacity(
+            self.max_seqs,
+            self.max_seq_len,
+            protected_prefix=self.protected_prefix,
+            protected_recent=self.protected_recent,
+            segments=self.segments,
+            policy=self.policy,
+        )
+        self.select_ws = select_workspace(self.select_ws_seqs, self.segments, self.policy, dev_)
+        self.select_ws_forced = None
         self.compact_ws = torch.empty(compact_workspace_bytes(self.max_seqs, self.budget), dtype=torch.uint8, device=dev_)
         self.layer_scores = None  # flat per-layer head maxima, viewed [S, tokens]; made on first use
         shape = (s, self.kv_heads, self.head_dim, self.tables.rotary_dim, self.tables.qpk, self.max_seqs, self.max_seq_len)
@@ -499,6 +517,13 @@ class CompressionPipeline:
         tables, freed = self.rewrite(batch)
         return keep, tables, freed
 
+    def _split_workspace(self, n_seq: int) -> torch.Tensor:
+        if n_seq <= self.select_ws_seqs:
+            return self.select_ws
+        if self.select_ws_forced is None:
+            self.select_ws_forced = select_workspace(self.max_seqs, self.segments, self.policy, self.device)
+        return self.select_ws_forced
+
     def select(self, batch: Batch) -> torch.Tensor:
         shape = self.select_shape
         if shape == "auto":
@@ -522,7 +547,7 @@ class CompressionPipeline:
             segments=self.segments,
             policy=self.policy,
             shape=shape,
-            workspace=self.select_ws,
+            workspace=self._split_workspace(batch.n_seq) if shape == "split" else None,
             validate=False,  # select_step and the callers of select validate the batch first
         )
         return self.keep[: batch.n_seq]

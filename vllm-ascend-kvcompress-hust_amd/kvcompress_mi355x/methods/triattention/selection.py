@@ -34,6 +34,18 @@ def prefers_split(seq_lens_host: list[int], *, protected_prefix: int, protected_
     return len(seq_lens_host) * per_seq <= SPLIT_MAX_JOBS and longest // per_seq >= SPLIT_MIN_SEGMENT
 
 
+def split_capacity(
+    max_seqs: int, max_seq_len: int, *, protected_prefix: int, protected_recent: int, segments: int, policy: str
+) -> int:
+    """The most sequences of a batch that ``prefers_split`` can send to the
+    chunked launch shape, for batches of up to ``max_seqs`` sequences of up to
+    ``max_seq_len`` tokens (a job's scratch is 149 KB)."""
+    per_seq = segments if policy == "v3" else 1
+    if (max_seq_len - protected_prefix - protected_recent) // per_seq < SPLIT_MIN_SEGMENT:
+        return 0
+    return min(max_seqs, SPLIT_MAX_JOBS // per_seq)
+
+
 def select_workspace(n_seq: int, segments: int, policy: str, device: torch.device) -> torch.Tensor:
     """Scratch of the chunked launch shape for up to ``n_seq`` sequences."""
     size = int(_native.load().kvc_select_workspace_bytes(n_seq, segments, POLICY_CODES[policy]))
