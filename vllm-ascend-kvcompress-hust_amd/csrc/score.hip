@@ -643,11 +643,25 @@ __global__ __launch_bounds__(kAggThreads) void aggregate_tokens_kernel(AggArgs a
 // 2 x 16384 14.5 / 12.6 / 13.9 against 22.9, 4 x 16384 22.1 / 21.1 / 25.9
 // against 28.2, 8 x 16384 35.7 / 36.8 / 48.2 against 33.0 (per-workgroup
 // statistics loads outweigh the latency once the chip is full).  So eight waves
-// for at most kAggSplitMaxGroups groups of 32 tokens (4 x 16384).
+// for at most kAggSplitMaxGroups groups of 32 tokens (4 x 16384), and for few
+// items, whose chain is short and leaves waves idle, for fewer (split_pays).
 constexpr int kAggSplitWaves = 8;
 constexpr int kAggSliceHeads = kAggTokLanes * kAggHeadUnroll;
 constexpr int kAggMaxItems = 128;  // 16 KB of LDS
 constexpr int64_t kAggSplitMaxGroups = 2048;
+
+// The one-wave form takes about 2.7 us and 1.2 an item of whatever number of
+// groups, this one the more the more groups there are.  Microseconds, this form
+// against the other: 2 items (2 layers x 8 heads) 4.8 / 5.1 at 1024 groups,
+// 6.5 / 5.1 at 1250, 7.5 / 5.2 at 2048; 3 (3 x 16) 6.5 / 6.9 at 1250, 7.3 / 6.9
+// at 1536; 4 (4 x 16) 7.4 / 8.3 at 1536, 8.6 / 8.1 at 2048; 5 (5 x 16) 8.8 / 9.5
+// at 1750, 9.5 / 9.3 at 2048; 6 (6 x 16) 10.1 / 10.7, 8 (4 x 32) 12.8 / 13.5 at
+// 2048.  One layer of up to 24 heads is one group of loads and a remainder: 4.9
+// against 4.5 at 1024 groups (17 heads).
+bool split_pays(int n_layers, int n_heads, int items, int64_t groups) {
+  if (items < 2 || items > kAggMaxItems || (n_layers == 1 && n_heads <= 24)) return false;
+  return groups <= kAggSplitMaxGroups && groups <= 512 + 256 * static_cast<int64_t>(items);
+}
 
 __global__ __launch_bounds__(64 * kAggSplitWaves) void aggregate_split_kernel(AggArgs a, int slices) {
   extern __shared__ float dyn[];
@@ -1099,7 +1113,7 @@ int launch_aggregate(const char* who, kvc_stream_t stream, int n_layers, int n_h
   if (raw_token_stride == 1) {
     const int slices = static_cast<int>(ceil_div(n_heads, kAggSliceHeads));
     const int64_t groups = ceil_div(max_seq_len, 32) * n_seq;
-    if (groups <= kAggSplitMaxGroups && slices * n_layers > 1 && slices * n_layers <= kAggMaxItems) {
+    if (split_pays(n_layers, n_heads, slices * n_layers, groups)) {
       dim3 grid(static_cast<unsigned>(ceil_div(max_seq_len, 32)), static_cast<unsigned>(n_seq));
       aggregate_split_kernel<<<grid, 64 * kAggSplitWaves, lds + slices * n_layers * 32 * sizeof(float), as_stream(stream)>>>(
           aa, slices);
