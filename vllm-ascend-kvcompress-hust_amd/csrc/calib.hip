@@ -25,15 +25,14 @@
 // finish kernel sums a unit's splits in a fixed order: repeated runs give
 // identical sums.
 //
-// Accumulation reads the projections once (HBM, 2-4 bytes per element), but
-// the state is written (and after the first call read) by every call and read
-// by the finish, so its rows are as few as fill the chip: about 760
-// workgroups, three a CU (77 rows for 40 heads of 128 dims: 4.7 MB against
-// 42 MB of 4096 projections).  Of that shape a layer's clear, accumulation and
-// finish took 6.9 + 12.8 + 7.4 us with 128 rows and a cleared state; now
-// 13.1 + 5.0.  640 and 1020 workgroups measured 13.9 and 14.3 us, eight waves
-// a workgroup 14.6; without any store it is 12.0, the latency of one round of
-// loads over a chip that starts and drains.
+// Accumulation reads the projections once (HBM, 2-4 bytes per element): 42 MB
+// for 4096 tokens of 40 heads of 128 dims.  128 rows there are 1280 workgroups,
+// whose first loads are the whole input in flight at once; the rows they write
+// and the finish reads are 7.9 MB.  Microseconds of that shape's first call,
+// later call and finish: 11.3 + 12.2 + 4.0 (a state cleared first, and one
+// thread an entry in the finish: 17.0, 12.0, 5.8).  Each wave 0 alone adds the
+// old sums: with the entries spread over all four waves, coalesced, later calls
+// took 14.1.  Where a row is large, fewer of them fill the chip (qstats_rows).
 
 #include "kvc_common.h"
 
@@ -44,6 +43,7 @@ constexpr int kQsWaves = 4;
 constexpr int kQsThreads = kQsWaves * 64;
 constexpr int kQsUnroll = 8;
 constexpr int kQsMinRows = 32, kQsMaxRows = 128;  // state rows
+constexpr int64_t kQsManyUnits = 3584;            // above: as many rows as 760 workgroups of four-wide lanes
 constexpr int kQsMinSplitTokens = 32;  // tokens per split, at least
 
 struct QStatsArgs {
@@ -73,10 +73,16 @@ __device__ __forceinline__ float widen<float>(float v) {
   return v;
 }
 
-// State rows, the most splits a call makes: 64*4 units x 760 rows' worth.
+// State rows, the most splits a call makes.  First and later calls of 4096
+// tokens, 128 rows against as many as 760 workgroups of 256 units have (us):
+// 40 heads of 128 dims (2560 units, 77 rows) 11.3 + 12.2 against 12.0 + 12.5, 16
+// of 256 dims with 64 rotary (3584, 55) 12.9 + 13.5 against 13.7 + 14.4; 64 of 128
+// (4096, 48), read one element a lane, 19.9 + 21.1 against 19.1 + 19.5, 96 (6144,
+// 32) 28.2 + 29.8 against 26.1 + 26.5.
 inline int qstats_rows(int64_t units) {
+  if (units <= kQsManyUnits) return kQsMaxRows;
   const int64_t rows = ceil_div(760 * 256, units);
-  return static_cast<int>(rows < kQsMinRows ? kQsMinRows : (rows > kQsMaxRows ? kQsMaxRows : rows));
+  return static_cast<int>(rows < kQsMinRows ? kQsMinRows : rows);
 }
 
 // V consecutive elements widened to float32, read with one load of
@@ -146,20 +152,24 @@ __global__ __launch_bounds__(kQsThreads) void qstats_accumulate_kernel(QStatsArg
     red[wave][3 * e + 2][lane] = s_abs[e];
   }
   __syncthreads();
-  // Entry k of lane l: statistic k%3 of unit unit0(l) + k/3, contiguous in the state.
+  if (wave != 0 || !live) return;
   const int64_t units = static_cast<int64_t>(a.heads) * (a.freq + a.pass);
-  for (int i = threadIdx.x; i < 64 * 3 * V; i += kQsThreads) {
-    const int l = i / (3 * V), k = i - l * (3 * V);
-    const int grp = static_cast<int>(blockIdx.x) * 64 + l;
-    if (grp >= groups) continue;
-    const int hh = grp / (fg + pg), cc = grp - hh * (fg + pg);
-    // Frequencies are units h*(F+P) + f, pass dims h*(F+P) + F + p.
-    const int64_t unit0 = static_cast<int64_t>(hh) * (a.freq + a.pass) + (cc < fg ? cc * V : a.freq + (cc - fg) * V);
-    double sum = 0.0;
+  // Unit index of element e: frequencies h*(F+P) + f, pass dims h*(F+P) + F + p.
+  const int64_t unit0 = static_cast<int64_t>(h) * (a.freq + a.pass) + (pair ? c * V : a.freq + (c - fg) * V);
+  double* st = a.state + (static_cast<int64_t>(blockIdx.y) * units + unit0) * 3;
+  double r[3 * V];  // element e, statistic k%3 at unit0 + e: [e][3] is contiguous
 #pragma unroll
-    for (int w = 0; w < kQsWaves; ++w) sum += red[w][k][l];
-    double* st = a.state + (static_cast<int64_t>(blockIdx.y) * units + unit0) * 3 + k;
-    *st = a.store ? sum : *st + sum;
+  for (int k = 0; k < 3 * V; ++k) {
+    r[k] = 0.0;
+#pragma unroll
+    for (int w = 0; w < kQsWaves; ++w) r[k] += red[w][k][lane];
+  }
+  if (a.store) {
+#pragma unroll
+    for (int k = 0; k < 3 * V; ++k) st[k] = r[k];
+  } else {  // every load of the old sums in flight at once
+#pragma unroll
+    for (int k = 0; k < 3 * V; ++k) st[k] += r[k];
   }
 }
 
