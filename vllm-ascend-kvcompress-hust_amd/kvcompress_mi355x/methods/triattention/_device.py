@@ -33,10 +33,12 @@ def stream_handle(device: torch.device) -> int:
     """The current stream's HIP handle, without building a Stream object for
     each of a step's launches.  A device that is no HIP device has none: host
     tensors handed to a launch end here, not in a kernel."""
-    if device.type != "cuda":
-        raise ValueError(f"the MI355X kernels need a HIP device, got {device}")
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    if index is None:  # host tensors' devices have no index
+        if device.type != "cuda":
+            raise ValueError(f"the MI355X kernels need a HIP device, got {device}")
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr(tensor: torch.Tensor | None) -> int | None:
