@@ -268,6 +268,22 @@ def _layer_scores(kernels, device, cache, blocks, stats, cos, sin, tokens):
     return out.cpu(), extra
 
 
+def _assert_float32_scores(got, extra, cache, blocks, stats, cos, sin, tokens, head_dim, rotary) -> None:
+    """Errors of at most 16 x 2^-24 of the terms' magnitudes."""
+    kv, freq, style = stats.q_mean_real.shape[0], rotary // 2, stats.rope_style
+    keys = cache[blocks].reshape(-1, kv, head_dim)[:tokens].double().permute(1, 2, 0).unsqueeze(1)  # [kv, 1, D, tokens]
+    re, im = (keys[:, :, 0:rotary:2], keys[:, :, 1:rotary:2]) if style == "interleaved" else (keys[:, :, :freq], keys[:, :, freq:rotary])
+    a, qr, qi, e = (t.double().unsqueeze(-1) for t in (torch.sqrt(stats.freq_scale_sq), stats.q_mean_real, stats.q_mean_imag, extra))
+    c, s = cos.double().view(-1, 1), sin.double().view(-1, 1)
+    terms = [a * qr * c * re, -a * qi * s * re, a * qi * c * im, a * qr * s * im, a * e * torch.sqrt(re * re + im * im)]
+    if head_dim > rotary:
+        terms.append(stats.q_pass_mean.double().unsqueeze(-1) * keys[:, :, rotary:])
+    want = sum(t.sum(2) for t in terms)
+    size = sum(t.abs().sum(2) for t in terms)
+    err = (got.double() - want).abs() / size
+    assert float(err.max()) <= 16 * 2.0**-24, float(err.max() * 2**24)
+
+
 @pytest.mark.parametrize("case", PART_SHAPES, ids=[f"kv{c[0]}q{c[1]}d{c[2]}r{c[3]}{c[4][0]}{str(c[5]).split('.')[-1]}t{c[6]}" for c in PART_SHAPES])
 def test_score_paged_part_steps_keep_float32(hip_device, case) -> None:
     """Within float32's rounding of a float64 evaluation of the same inputs.
@@ -286,17 +302,38 @@ def test_score_paged_part_steps_keep_float32(hip_device, case) -> None:
     phase = torch.rand(freq, generator=g) * 6.0
     cos, sin = 0.7 * torch.cos(phase), 0.7 * torch.sin(phase)
     got, extra = _layer_scores(kernels, hip_device, cache, blocks, stats, cos, sin, tokens)
-    keys = cache[blocks].reshape(-1, kv, head_dim)[:tokens].double().permute(1, 2, 0).unsqueeze(1)  # [kv, 1, D, tokens]
-    re, im = (keys[:, :, 0:rotary:2], keys[:, :, 1:rotary:2]) if style == "interleaved" else (keys[:, :, :freq], keys[:, :, freq:rotary])
-    a, qr, qi, e = (t.double().unsqueeze(-1) for t in (torch.sqrt(stats.freq_scale_sq), stats.q_mean_real, stats.q_mean_imag, extra))
-    c, s = cos.double().view(-1, 1), sin.double().view(-1, 1)
-    terms = [a * qr * c * re, -a * qi * s * re, a * qi * c * im, a * qr * s * im, a * e * torch.sqrt(re * re + im * im)]
-    if head_dim > rotary:
-        terms.append(stats.q_pass_mean.double().unsqueeze(-1) * keys[:, :, rotary:])
-    want = sum(t.sum(2) for t in terms)
-    size = sum(t.abs().sum(2) for t in terms)
-    err = (got.double() - want).abs() / size
-    assert float(err.max()) <= 16 * 2.0**-24, float(err.max() * 2**24)
+    _assert_float32_scores(got, extra, cache, blocks, stats, cos, sin, tokens, head_dim, rotary)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["weights", "keys"])
+def test_score_paged_part_steps_wide_ranges(hip_device, dtype, kind) -> None:
+    """Three words where fp16's range is narrow: weights of one column spread
+    over seven decades with keys that make every term count alike, and keys of
+    1e-4 whose magnitudes make up the score.  The bound is float32's, as above."""
+    kernels, _, _ = _kvc()
+    kv, qpk, dim, tokens = 2, 4, 96, 300
+    freq = dim // 2
+    g = torch.Generator().manual_seed(31)
+    stats = _random_stats(g, kv, qpk, freq, 0, dim)
+    n_blocks = -(-tokens // 128)
+    keys = torch.randn(n_blocks + 1, 128, kv, dim, generator=g)
+    if kind == "weights":
+        spread = torch.logspace(0, -7, freq)
+        stats = ref.LayerStats(stats.q_mean_real, stats.q_mean_imag, stats.q_abs_mean, stats.freq_scale_sq * spread.square(),
+                               stats.omega, stats.rope_style, stats.rotary_dim, None)
+        keys = (keys * 1e-3 / spread.repeat(2)).clamp(-6e4, 6e4)
+    else:
+        small = 1e-3
+        stats = ref.LayerStats(stats.q_mean_real * small, stats.q_mean_imag * small, stats.q_abs_mean.abs() + 1.0,
+                               stats.freq_scale_sq, stats.omega, stats.rope_style, stats.rotary_dim, None)
+        keys = keys * 1e-4
+    cache = keys.to(dtype)
+    blocks = torch.randperm(n_blocks + 1, generator=g)[:n_blocks]
+    phase = torch.rand(freq, generator=g) * 6.0
+    cos, sin = 0.7 * torch.cos(phase), 0.7 * torch.sin(phase)
+    got, extra = _layer_scores(kernels, hip_device, cache, blocks, stats, cos, sin, tokens)
+    _assert_float32_scores(got, extra, cache, blocks, stats, cos, sin, tokens, dim, dim)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -53,8 +53,9 @@ struct MfmaElem<true> {
   static constexpr float kMagScale = 0.25f;  // |k| of fp16 keys reaches 2^16.5
   // Of three words the first keeps eight significant bits, as bf16 does: its
   // products then leave the matrix core's sum the bits that full fp16 products
-  // would use up.  The lower two words of |k| are held times 2^8 (at most
-  // 2^15), clear of fp16's subnormals; their products are scaled back.
+  // would use up.  Each further word is held times 2^8 (at most 2^15), so that
+  // fp16's subnormals cut a weight at 2^-54 of its column's largest and |k| at
+  // 2^-40; the products are scaled back.
   static constexpr float kLowScale = 1.0f / 256.0f;
   static constexpr uint32_t kLeadMask = 0xfff8u;
   __device__ __forceinline__ static f32x4 mfma(vec a, vec b, f32x4 c) {
@@ -85,9 +86,8 @@ __device__ __forceinline__ float bf16_value(uint32_t bits) { return __uint_as_fl
 
 // |k| of the eight frequencies of magnitude K step q held by this lane, as
 // TERMS 16-bit A operands, each the rounding of what the ones before it leave
-// (two: |k| * kMagScale to ~2^-16; three: to float32, the lower two divided by
-// kLowScale).  Two
-// frequencies per output word: half style pairs word w of linear steps q
+// (two: |k| * kMagScale to ~2^-16; three: to float32, each divided by kLowScale
+// more than the one before).  Two frequencies per output word: half style pairs word w of linear steps q
 // (real parts) and q + NF (imaginary parts); interleaved takes words 2w, 2w+1
 // of step 2q (w < 2) or 2q + 1, each word one (real, imaginary) pair.
 template <bool F16, bool IL, int NK, int NF, int TERMS>
@@ -127,7 +127,7 @@ __device__ __forceinline__ void magnitude_words(const u32x4 (&ka)[NK], int q, ty
       words[k][w] = word;
       m0 -= E::lo(word);
       m1 -= E::hi(word);
-      if (TERMS == 3 && k == 0) {
+      if (TERMS == 3 && k < 2) {
         m0 *= 1.0f / E::kLowScale;
         m1 *= 1.0f / E::kLowScale;
       }

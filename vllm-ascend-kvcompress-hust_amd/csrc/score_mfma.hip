@@ -125,7 +125,8 @@ __device__ __forceinline__ float folded_weight(const FoldArgs& a, const float* p
   return a.scale[o] * a.extra[o];
 }
 
-// The 16-bit words of the eight weights w, word k to dst + k * stride.
+// The 16-bit words of the eight weights w, word k to dst + k * stride (of three
+// fp16 words each divided by kLowScale more than the one before).
 template <bool F16>
 __device__ __forceinline__ void store_words(float (&w)[8], int terms, uint16_t* dst, int64_t stride) {
   for (int k = 0; k < terms; ++k) {
@@ -141,6 +142,7 @@ __device__ __forceinline__ void store_words(float (&w)[8], int terms, uint16_t* 
           bits = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
           if (terms == 3 && k == 0) bits &= MfmaElem<true>::kLeadMask;
           v -= static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(bits)));
+          if (terms == 3) v *= 1.0f / MfmaElem<true>::kLowScale;
         } else {
           bits = bf16_bits(v) & 0xffffu;
           v -= bf16_value(bits);
@@ -422,12 +424,13 @@ __attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) vo
     if constexpr (PART) {
       // Three words a weight and three of |k|: the products that reach 2^-24.
       // Each step's leading products are a sum of their own and the sums meet
-      // pairwise, so that they round at their own size.
+      // pairwise, so that they round at their own size.  fp16: acc0 holds
+      // products one kLowScale up, acc1 two.
       constexpr int kChains = NK + NF;
       f32x4 lead[kChains];
 #pragma unroll
       for (int c = 0; c < kChains; ++c) lead[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      f32x4 low = {0.0f, 0.0f, 0.0f, 0.0f};  // products with the lower words of |k|
+      f32x4 low = {0.0f, 0.0f, 0.0f, 0.0f};  // bf16: products with the lower words of |k|
 #pragma unroll
       for (int j = 0; j < NK; ++j) {
         const vec_t kv = __builtin_bit_cast(vec_t, ka[j]);
@@ -442,16 +445,17 @@ __attribute__((amdgpu_waves_per_eu(MfmaTiling<NK, NF, PART>::kWavesPerSimd))) vo
         lead[NK + q] = E::mfma(k3[0], m[q][0], lead[NK + q]);
         acc0 = E::mfma(k3[0], m[q][1], acc0);
         acc1 = E::mfma(k3[0], m[q][2], acc1);
-        low = E::mfma(k3[1], m[q][0], low);
-        low = E::mfma(k3[1], m[q][1], low);
-        low = E::mfma(k3[2], m[q][0], low);
+        f32x4& once = F16 ? acc0 : low;
+        f32x4& twice = F16 ? acc1 : low;
+        once = E::mfma(k3[1], m[q][0], once);
+        twice = E::mfma(k3[1], m[q][1], twice);
+        twice = E::mfma(k3[2], m[q][0], twice);
       }
 #pragma unroll
       for (int width = 1; width < kChains; width *= 2)
 #pragma unroll
         for (int c = 0; c + width < kChains; c += 2 * width) lead[c] += lead[c + width];
-      acc1 += F16 ? low * E::kLowScale : low;
-      acc1 += acc0;
+      acc1 = F16 ? (acc1 * E::kLowScale + acc0) * E::kLowScale : acc1 + low + acc0;
       acc0 = lead[0];
     } else {
 #pragma unroll
