@@ -42,6 +42,9 @@ struct MfmaElem<false> {
   __device__ __forceinline__ static float lo(uint32_t w) { return bf16_lo(w); }
   __device__ __forceinline__ static float hi(uint32_t w) { return bf16_hi(w); }
   __device__ __forceinline__ static uint32_t pack(float a, float b) { return pack_bf16(a, b); }
+  // Sum of both halves' squares.  The dot instruction rounds a little less well
+  // than a product and a multiply-add (root mean square error 0.112 against 0.103
+  // x 2^-24), far below the 2^-16 that two bf16 words of the root keep.
   __device__ __forceinline__ static float square_sum(uint32_t w) {
     const bf16x2 v = __builtin_bit_cast(bf16x2, w);
     return __builtin_amdgcn_fdot2_f32_bf16(v, v, 0.0f, false);
@@ -64,9 +67,12 @@ struct MfmaElem<true> {
   __device__ __forceinline__ static float lo(uint32_t w) { return fp16_lo(w); }
   __device__ __forceinline__ static float hi(uint32_t w) { return fp16_hi(w); }
   __device__ __forceinline__ static uint32_t pack(float a, float b) { return pack_f16(a, b); }
+  // Two fp16 words keep 2^-22 of the root, where the dot instruction's rounding
+  // (0.31 against 0.29 x 2^-24) showed: scores of 20000 tokens of 128 dims were
+  // 8.246e-8 from float64 with it, 8.214e-8 without.
   __device__ __forceinline__ static float square_sum(uint32_t w) {
-    const f16x2 v = __builtin_bit_cast(f16x2, w);
-    return __builtin_amdgcn_fdot2(v, v, 0.0f, false);
+    const float re = lo(w), im = hi(w);
+    return fmaf(im, im, re * re);
   }
 };
 
@@ -109,7 +115,7 @@ __device__ __forceinline__ void magnitude_words(const u32x4 (&ka)[NK], int q, ty
     }
     float m0, m1;
     if constexpr (TERMS == 2) {
-      // Both squares and their sum in one instruction on (real, imaginary) words.
+      // Sums of squares of (real, imaginary) words.
       const uint32_t p0 = IL ? ka[2 * q + (w >> 1)][(2 * w) & 3] : __builtin_amdgcn_perm(im_w, re_w, 0x05040100);
       const uint32_t p1 = IL ? ka[2 * q + (w >> 1)][(2 * w + 1) & 3] : __builtin_amdgcn_perm(im_w, re_w, 0x07060302);
       m0 = __builtin_amdgcn_sqrtf(E::square_sum(p0)) * E::kMagScale;
