@@ -462,6 +462,32 @@ def test_max_scorer_rejects_oversized_fold_before_launch() -> None:
     assert "exceed one dispatch" in lib.kvc_last_error().decode()
 
 
+@pytest.mark.parametrize("kv, qpk, pairs", [(8, 5, (65535, 65)), (8, 5, (65535, 4097))])
+def test_batch_scorer_rejects_oversized_fold_before_launch(kv, qpk, pairs) -> None:
+    """kvc_score_batch beyond the (sequence, layer) pairs that one dispatch of
+    the joint phases-and-fold launch holds (1024 work-items a pair) forms the
+    phases apart, and a weight fold that one dispatch does not hold either is
+    rejected before that."""
+    import torch
+
+    from kvcompress_mi355x import _native
+
+    if torch.cuda.is_available():
+        pytest.skip("placeholder pointers: run where no device could be reached by a launch")
+    lib = _native.load()
+    n_seq, n_layers = pairs
+    dim, max_len = 128, 256
+    ws = lib.kvc_score_workspace_bytes(n_layers, kv, dim, dim, qpk, n_seq, max_len)
+    assert ws > 0
+    fake = 4096
+    rc = lib.kvc_score_batch(
+        None, 0, n_layers, fake, 100, 128 * kv * dim, kv, dim, dim, qpk, 0, n_seq, max_len, fake, fake, fake, fake, fake, fake,
+        fake, fake, None, fake, fake, 16, fake, fake, fake, fake, 0, 1, 256, fake, ws, fake, fake,
+    )
+    assert rc == _native.EINVAL
+    assert "exceed one dispatch" in lib.kvc_last_error().decode()
+
+
 def test_raw_layout_names_the_scorer_without_gpu() -> None:
     """Matrix-core shapes (bf16 or fp16, half or interleaved RoPE, head_dim and
     F multiples of 32, qpk <= 8) get head-major raw scores; the rest token-major."""

@@ -936,7 +936,12 @@ int kvc::score_paged(bool vector_only, const PhaseArgs* phases, kvc_stream_t str
                            workspace, workspace_bytes_given, need, &s, &fa, &sa))
     return rc;
   const bool matrix = mfma_scorer_supported(s, dtype, rope_style);
-  if (phases && (s.max_tiles == 0 || !matrix)) {
+  // One launch forms the phases and folds the weights, where one dispatch holds it.
+  const bool joint = phases && matrix && s.max_tiles > 0 && mfma_phase_fold_items(s) <= kMaxDispatchItems;
+  if (phases && !joint) {
+    if (matrix && s.max_tiles > 0 && mfma_fold_items(s, dtype) > kMaxDispatchItems)
+      return fail(KVC_EINVAL, "kvc_score_batch: the weight fold's %lld work-items exceed one dispatch",
+                  static_cast<long long>(mfma_fold_items(s, dtype)));
     if (int rc = kvc_mean_phases(stream, n_seq, n_layers, s.freq, phases->round_starts, phases->offsets,
                                  phases->n_offsets, phases->omega, phases->phase_cos, phases->phase_sin))
       return rc;
@@ -944,7 +949,7 @@ int kvc::score_paged(bool vector_only, const PhaseArgs* phases, kvc_stream_t str
   if (s.max_tiles == 0) return 0;
   hipStream_t st = as_stream(stream);
 
-  if (matrix) return launch_mfma_scorer(st, s, dtype, phases, fa, sa, workspace);
+  if (matrix) return launch_mfma_scorer(st, s, dtype, joint ? phases : nullptr, fa, sa, workspace);
 
   const int64_t fold_threads = static_cast<int64_t>(n_seq) * n_layers * kv_heads * s.units;
   fold_weights_kernel<<<static_cast<unsigned>(ceil_div(fold_threads, 64)), 64, 0, st>>>(fa);

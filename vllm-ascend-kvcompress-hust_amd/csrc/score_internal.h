@@ -288,5 +288,7 @@ int launch_mfma_fold(hipStream_t stream, const ScoreShape& s, int dtype, const F
 constexpr int64_t kMaxDispatchItems = 0xffffffffLL;
 // Work-items of launch_mfma_fold's dispatch for this shape and dtype.
 int64_t mfma_fold_items(const ScoreShape& s, int dtype);
+// The same where the launch forms the phases too.
+int64_t mfma_phase_fold_items(const ScoreShape& s);
 
 }  // namespace kvc

@@ -666,6 +666,16 @@ int64_t mfma_fold_items(const ScoreShape& s, int dtype) {
   return static_cast<int64_t>(fold_blocks(s, dtype)) * kFoldThreads * s.n_layers * s.n_seq;
 }
 
+// Workgroups a (sequence, layer) is folded by where they form its phases too.
+static int64_t phase_fold_splits(const ScoreShape& s) {
+  const int64_t splits = ceil_div(512, static_cast<int64_t>(s.n_layers) * s.n_seq);
+  return splits < s.kv_heads ? splits : s.kv_heads;
+}
+
+int64_t mfma_phase_fold_items(const ScoreShape& s) {
+  return static_cast<int64_t>(s.n_layers) * s.n_seq * phase_fold_splits(s) * kFoldPhaseThreads;
+}
+
 int launch_mfma_fold(hipStream_t stream, const ScoreShape& s, int dtype, const FoldArgs& fa, void* weights) {
   const MfmaGeometry geo = geometry(s);
   const int64_t items = mfma_fold_items(s, dtype);
@@ -690,9 +700,8 @@ int launch_mfma_scorer(hipStream_t stream, const ScoreShape& s, int dtype, const
   if (phases) {
     uint16_t* out = static_cast<uint16_t*>(weights);
     float* scale = reinterpret_cast<float*>(static_cast<char*>(weights) + mfma_fragment_only_bytes(s));
-    const int64_t splits = ceil_div(512, static_cast<int64_t>(s.n_layers) * s.n_seq);
     const dim3 grid(static_cast<unsigned>(s.n_layers), static_cast<unsigned>(s.n_seq),
-                    static_cast<unsigned>(splits < s.kv_heads ? splits : s.kv_heads));
+                    static_cast<unsigned>(phase_fold_splits(s)));
     (dtype == KVC_DTYPE_FP16 ? fold_phases_kernel<true> : fold_phases_kernel<false>)<<<grid, kFoldPhaseThreads, 0, stream>>>(
         fa, *phases, phase_lanes(phases->n_offsets), geo.nk, geo.nf, geo.terms, out, scale);
     if (int rc = launch_status("kvc_score_paged(phases and fold)")) return rc;
