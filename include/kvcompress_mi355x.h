@@ -199,10 +199,14 @@ int kvc_score_batch(kvc_stream_t stream, int dtype, int n_layers, const uint64_t
  * cannot allocate device memory (code under HIP graph capture, serving loops
  * that forbid allocation).  It allocates and frees nothing.  Arguments as
  * kvc_score_paged without the workspace, plus kvc_head_stats's mean/var
- * outputs; the results equal those two calls'.  Returns KVC_EINVAL when the
- * batch needs more scratch than 64 MiB (kvc_score_workspace_bytes of the same
- * shape; e.g. 6 scoring layers x 16 sequences of 16384 tokens x 40 query heads
- * need 7 MiB) and when `stream` does not belong to the current device.  Every
+ * outputs; the results equal those two calls' if the batch's
+ * kvc_score_workspace_bytes are at most 64 MiB (6 scoring layers x 16 sequences
+ * of 16384 tokens x 40 query heads need 7 MiB).  Head sizes whose weights the
+ * matrix cores take in three words (96 or 80 dims, partly rotated ones) need
+ * about half of that with the vector scorer, which serves batches that only
+ * then fit, with float32 rounding of its own.  Returns KVC_EINVAL when the batch
+ * needs more scratch than 64 MiB either way and when `stream` does not belong to
+ * the current device.  Every
  * call on a device shares that device's array: calls that overlap in time on
  * one device (concurrent streams, several threads) race and must be
  * serialised by the caller. */

@@ -97,6 +97,41 @@ def test_noalloc_scorer_matches_workspace_scorer_twice(hip_device, config):
 
 
 @pytest.mark.gpu
+def test_noalloc_scorer_of_a_batch_that_only_the_vector_scorer_fits(hip_device):
+    """480 sequences x 4 layers x 8 KV heads x 4 query heads of 96 dims: the
+    matrix cores' three words a weight need 67 MiB of scratch, the vector
+    scorer's floats 33, so the static array serves the batch with that scorer.
+    Both are within 16 x 2^-24 of the terms' magnitudes (some 100 terms, at most
+    20 times a head's largest score) of the exact score: 4e-5 of the largest."""
+    spec = workloads.config_spec(
+        2, n_layers=4, score_layer_stride=1, seq_lens=(200,) * 480, budget=100, recent=32, head_dim=96, rotary_dim=96,
+        num_attention_heads=32, num_kv_heads=8, max_model_len=65536)
+    cache = workloads.build_synthetic_cache(spec, hip_device, seed=6)
+    pipeline, batch = workloads.build_pipeline(cache)
+    t, lib = pipeline.tables, _native.load()
+    assert lib.kvc_score_workspace_bytes(t.n_layers, 8, 96, 96, t.qpk, batch.n_seq, 200) > 64 << 20
+    pipeline.score(batch)
+    total = batch.total_tokens
+    raw2 = torch.full_like(pipeline.raw, float("nan"))
+    mean2 = torch.full((t.n_layers, batch.n_seq, pipeline.n_heads), float("nan"), device=pipeline.device)
+    var2 = torch.full_like(mean2, float("nan"))
+    assert _noalloc(pipeline, batch, raw2, mean2, var2) == 0, lib.kvc_last_error().decode()
+    got = (raw2.transpose(1, 2) if pipeline.head_major else raw2)[:, :total]
+    want = pipeline.raw_scores()[:, :total]
+    limit = 4e-5 * want.abs().amax(1, keepdim=True)
+    assert bool(((got - want).abs() <= limit).all())
+    assert not torch.equal(got, want)  # another kernel's rounding: the vector scorer ran
+    want_mean, want_var = pipeline.head_statistics(batch)
+    scale = limit.transpose(0, 1).reshape(t.n_layers, 1, -1)
+    assert bool(((mean2 - want_mean).abs() <= scale).all())
+    torch.testing.assert_close(var2, want_var, rtol=1e-3, atol=1e-4)
+    # A batch that fits next: the matrix cores' weights and layout again.
+    small = Batch.build(hip_device, [200, 150], [200, 150], cache.source_tables[:2], None if cache.destination_tables is None
+                        else cache.destination_tables[:2], budget=spec.budget)
+    _check_call(pipeline, small)
+
+
+@pytest.mark.gpu
 def test_noalloc_scorer_under_graph_capture(hip_device):
     """The entry point captured into a HIP graph on a side stream (after one
     eager call on the device, which takes the scratch array's address):

@@ -3,7 +3,8 @@
 // file-scope device array instead of a caller workspace, for callers that
 // cannot allocate device memory (HIP graph capture, serving loops that forbid
 // allocation).  The kernels are the ones kvc_score_paged and kvc_head_stats
-// launch; only where the scratch lives differs.
+// launch; only where the scratch lives differs, and batches whose three-word
+// weights do not fit it take the vector scorer.
 //
 // The array is a device symbol: its name in host code is a host-side stand-in,
 // not a device address.  The device address is taken once per device with
