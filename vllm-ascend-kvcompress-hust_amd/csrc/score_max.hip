@@ -503,23 +503,18 @@ __attribute__((amdgpu_waves_per_eu(MaxTiling<NK, LEAN>::kWavesPerSimd))) void sc
               f32x4 res[T];
               if constexpr (LEAN) {
                 const u32x4* wl = lds_frag + (min(it + 1, n_items - 1) * NR) * 128 + lane;
-                f32x4 acc[T][2];
 #pragma unroll
-                for (int u = 0; u < T; ++u) acc[u][0] = acc[u][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int u = 0; u < T; ++u) res[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int st = 0; st < NR; ++st) {
 #pragma unroll
                   for (int h = 0; h < 2; ++h) {
 #pragma unroll
-                    for (int u = 0; u < T; ++u) {
-                      const int chain = T == 1 ? h : 0;
-                      acc[u][chain] = E::mfma(wbuf[0][2 * st + h], __builtin_bit_cast(vec_t, kk[u][st]), acc[u][chain]);
-                    }
+                    for (int u = 0; u < T; ++u)
+                      res[u] = E::mfma(wbuf[0][2 * st + h], __builtin_bit_cast(vec_t, kk[u][st]), res[u]);
                     wbuf[0][2 * st + h] = __builtin_bit_cast(vec_t, wl[st * 128 + h * 64]);
                   }
                 }
-#pragma unroll
-                for (int u = 0; u < T; ++u) res[u] = T == 1 ? acc[u][0] + acc[u][1] : acc[u][0];
               } else {
                 load_w(it + 1, wbuf[(it + 1) & 1]);
                 chunk_products(wbuf[it & 1], res);
