@@ -576,7 +576,7 @@ def test_aggregate_finalize_non_finite_matches_oracle(hip_device, layer_mode) ->
 
 
 @pytest.mark.parametrize("layer_mode", ["mean", "max"])
-@pytest.mark.parametrize("layers,heads", [(1, 4), (3, 16), (2, 20), (5, 32), (4, 64)])
+@pytest.mark.parametrize("layers,heads", [(1, 20), (3, 36), (2, 20), (5, 32), (4, 64)])
 def test_aggregate_whole_rows_match_single_floats(hip_device, layers, heads, layer_mode) -> None:
     """Token-major rows of whole 16-byte words against the same scores shifted
     by one float (read one by one): idle lanes, odd layer counts, several turns

@@ -393,16 +393,21 @@ def test_batch_descriptors_of_one_copy(hip_device, n_seq) -> None:
 
 
 @pytest.mark.parametrize("shape", [(8, 2, 128, 128, torch.bfloat16), (12, 4, 96, 96, torch.float16), (8, 1, 192, 192, torch.bfloat16),
-                                   (16, 2, 256, 256, torch.bfloat16)])
+                                   (16, 2, 256, 256, torch.bfloat16), (8, 8, 64, 64, torch.bfloat16, 60),
+                                   (15, 5, 96, 96, torch.float16, 60), (4, 4, 64, 64, torch.float16, 60),
+                                   (4, 2, 64, 64, torch.bfloat16, 180)])
 def test_batch_scoring_equals_its_three_calls(hip_device, shape) -> None:
     """kvc_score_batch against kvc_mean_phases, kvc_score_paged and
     kvc_head_stats on the same batch, bit for bit (matrix-core shapes of two and
-    three words, the vector scorer, heads split over workgroups and not)."""
+    three words, the vector scorer; the KV heads one a workgroup with 9 (sequence,
+    layer) pairs; with 180 in three workgroups' shares of 3 + 3 + 2, 2 + 2 + 1 and
+    2 + 2 + 0; with 540 in one)."""
     from kvcompress_mi355x import _native, workloads
     from kvcompress_mi355x.methods.triattention import _device as dev
 
-    heads, kv, dim, rotary, dtype = shape
-    spec = workloads.config_spec(2, n_layers=3, score_layer_stride=1, seq_lens=(1500, 700, 2049), budget=512, recent=64, head_dim=dim,
+    heads, kv, dim, rotary, dtype = shape[:5]
+    lens = tuple(600 + 7 * i for i in range(shape[5])) if len(shape) > 5 else (1500, 700, 2049)
+    spec = workloads.config_spec(2, n_layers=3, score_layer_stride=1, seq_lens=lens, budget=512, recent=64, head_dim=dim,
                                  rotary_dim=rotary, num_attention_heads=heads, num_kv_heads=kv, max_model_len=65536)
     cache = workloads.build_synthetic_cache(spec, hip_device, seed=7)
     if dtype != cache.k_caches[0].dtype:
