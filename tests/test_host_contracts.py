@@ -642,3 +642,12 @@ def test_split_scratch_covers_the_batches_the_rule_sends_there():
                 accepted = [n for n in range(1, max_seqs + 1) if selection.prefers_split([max_len] * n, **windows)]
                 assert cap == max(accepted, default=0), (policy, segments, max_len, max_seqs)
                 assert cap * (segments if policy == "v3" else 1) <= selection.SPLIT_MAX_JOBS
+
+
+@pytest.mark.parametrize("entry", ["kvc_qstats_start", "kvc_qstats_accumulate"])
+def test_qstats_errors_name_their_entry(entry) -> None:
+    from kvcompress_mi355x import _native
+
+    lib = _native.load()
+    assert getattr(lib, entry)(None, 0, 4096, 8, 64, 1, 64, 64, None, 0) == _native.EINVAL
+    assert lib.kvc_last_error().decode().startswith(f"{entry}: state of ")

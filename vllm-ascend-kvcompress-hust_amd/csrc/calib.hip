@@ -229,20 +229,20 @@ extern "C" size_t kvc_qstats_state_bytes(int heads, int head_dim, int rotary_dim
 namespace kvc {
 namespace {
 
-int launch_accumulate(kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens, int64_t token_stride, int heads,
-                      int head_dim, int rotary_dim, void* state, size_t state_bytes, bool store) {
+int launch_accumulate(const char* who, kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens,
+                      int64_t token_stride, int heads, int head_dim, int rotary_dim, void* state, size_t state_bytes, bool store) {
   if (dtype != KVC_DTYPE_BF16 && dtype != KVC_DTYPE_FP16 && dtype != KVC_DTYPE_FP32)
-    return fail(KVC_EINVAL, "kvc_qstats_accumulate: unknown dtype %d", dtype);
-  if (heads <= 0 || head_dim <= 0 || n_tokens < 0) return fail(KVC_EINVAL, "kvc_qstats_accumulate: bad sizes");
+    return fail(KVC_EINVAL, "%s: unknown dtype %d", who, dtype);
+  if (heads <= 0 || head_dim <= 0 || n_tokens < 0) return fail(KVC_EINVAL, "%s: bad sizes", who);
   if (!shape_ok(heads, head_dim, rotary_dim))
-    return fail(KVC_EINVAL, "kvc_qstats_accumulate: rotary_dim must be positive, even and <= head_dim");
+    return fail(KVC_EINVAL, "%s: rotary_dim must be positive, even and <= head_dim", who);
   if (token_stride < static_cast<int64_t>(heads) * head_dim)
-    return fail(KVC_EINVAL, "kvc_qstats_accumulate: token_stride smaller than a token's row");
+    return fail(KVC_EINVAL, "%s: token_stride smaller than a token's row", who);
   const size_t need = kvc_qstats_state_bytes(heads, head_dim, rotary_dim);
   if (!state || state_bytes < need)
-    return fail(KVC_EINVAL, "kvc_qstats_accumulate: state of %zu bytes needed", need);
+    return fail(KVC_EINVAL, "%s: state of %zu bytes needed", who, need);
   if (n_tokens == 0 && !store) return 0;
-  if (!q && n_tokens > 0) return fail(KVC_EINVAL, "kvc_qstats_accumulate: null input");
+  if (!q && n_tokens > 0) return fail(KVC_EINVAL, "%s: null input", who);
   QStatsArgs a;
   a.q = q;
   a.n_tokens = n_tokens;
@@ -269,7 +269,7 @@ int launch_accumulate(kvc_stream_t stream, int dtype, const void* q, int64_t n_t
   const int v = wide ? 4 : 1;
   const int64_t groups = static_cast<int64_t>(heads) * (a.freq / v + a.pass / v);
   const int64_t blocks = ceil_div(groups, 64);
-  if (groups > 0x7fffffff - 64) return fail(KVC_EINVAL, "kvc_qstats_accumulate: too many heads");
+  if (groups > 0x7fffffff - 64) return fail(KVC_EINVAL, "%s: too many heads", who);
   const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(splits));
   hipStream_t st = as_stream(stream);
   switch (dtype * 2 + (wide ? 1 : 0)) {
@@ -280,7 +280,7 @@ int launch_accumulate(kvc_stream_t stream, int dtype, const void* q, int64_t n_t
     case KVC_DTYPE_FP32 * 2 + 1: qstats_accumulate_kernel<float, 4><<<grid, kQsThreads, 0, st>>>(a); break;
     default: qstats_accumulate_kernel<float, 1><<<grid, kQsThreads, 0, st>>>(a); break;
   }
-  return launch_status("kvc_qstats_accumulate");
+  return launch_status(who);
 }
 
 }  // namespace
@@ -289,14 +289,14 @@ int launch_accumulate(kvc_stream_t stream, int dtype, const void* q, int64_t n_t
 extern "C" int kvc_qstats_accumulate(kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens,
                                      int64_t token_stride, int heads, int head_dim, int rotary_dim, void* state,
                                      size_t state_bytes) {
-  return launch_accumulate(stream, dtype, q, n_tokens, token_stride, heads, head_dim, rotary_dim, state, state_bytes,
-                           false);
+  return launch_accumulate("kvc_qstats_accumulate", stream, dtype, q, n_tokens, token_stride, heads, head_dim, rotary_dim,
+                           state, state_bytes, false);
 }
 
 extern "C" int kvc_qstats_start(kvc_stream_t stream, int dtype, const void* q, int64_t n_tokens, int64_t token_stride,
                                 int heads, int head_dim, int rotary_dim, void* state, size_t state_bytes) {
-  return launch_accumulate(stream, dtype, q, n_tokens, token_stride, heads, head_dim, rotary_dim, state, state_bytes,
-                           true);
+  return launch_accumulate("kvc_qstats_start", stream, dtype, q, n_tokens, token_stride, heads, head_dim, rotary_dim,
+                           state, state_bytes, true);
 }
 
 extern "C" int kvc_qstats_finish(kvc_stream_t stream, int heads, int head_dim, int rotary_dim, const void* state,
