@@ -651,3 +651,21 @@ def test_qstats_errors_name_their_entry(entry) -> None:
     lib = _native.load()
     assert getattr(lib, entry)(None, 0, 4096, 8, 64, 1, 64, 64, None, 0) == _native.EINVAL
     assert lib.kvc_last_error().decode().startswith(f"{entry}: state of ")
+
+
+def test_block_tables_are_recorded_on_the_stream_that_reads_them(monkeypatch):
+    """Rows on the reader's device are recorded on it (they may have been
+    allocated on another stream); lists and rows elsewhere are not."""
+    from kvcompress_mi355x.methods.triattention import _device as dev
+
+    seen = []
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, s: seen.append((t.tolist(), s)))
+    reader = SimpleNamespace(device_index=-1)  # host tensors' device number
+    rows = [torch.tensor([3, 1], dtype=torch.int32), torch.tensor([7])]
+    flat, lengths = dev.ragged_ids(rows, torch.device("cpu"), reader)
+    assert flat.tolist() == [3, 1, 7] and lengths == [2, 1] and flat.dtype == torch.int64
+    assert seen == [([3, 1], reader), ([7], reader)]
+    seen.clear()
+    dev.ragged_ids(rows, torch.device("cpu"), SimpleNamespace(device_index=0))
+    dev.ragged_ids([[1, 2], (3,)], torch.device("cpu"))
+    assert seen == []

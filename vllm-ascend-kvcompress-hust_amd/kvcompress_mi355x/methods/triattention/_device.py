@@ -94,12 +94,20 @@ def pointer_table(tensors: list[torch.Tensor], device: torch.device) -> torch.Te
     return torch.tensor(signed, dtype=torch.int64, device=device)
 
 
-def ragged_ids(rows: list[torch.Tensor | list[int] | tuple[int, ...]], device: torch.device) -> tuple[torch.Tensor, list[int]]:
-    """Concatenate int64 rows; return (flat ids, host lengths)."""
+def ragged_ids(
+    rows: list[torch.Tensor | list[int] | tuple[int, ...]], device: torch.device, reader: torch.cuda.Stream | None = None
+) -> tuple[torch.Tensor, list[int]]:
+    """Concatenate int64 rows; return (flat ids, host lengths).  ``reader``: the
+    device's current stream, which reads the rows that are there already; they
+    are recorded on it, so that a row allocated on another stream may be dropped
+    at once."""
     lengths: list[int] = []
     parts: list[torch.Tensor] = []
+    index = -2 if reader is None else reader.device_index
     for row in rows:
         t = row if isinstance(row, torch.Tensor) else torch.tensor(list(row), dtype=torch.int64)
+        if t.get_device() == index:
+            t.record_stream(reader)
         t = t.to(device=device, dtype=torch.int64).reshape(-1)
         parts.append(t)
         lengths.append(int(t.numel()))

@@ -215,7 +215,9 @@ class TriAttentionMethod(KVCompressionMethod):
         return self.compress_batch((request,))[0]
 
     def compress_batch(self, requests: Sequence[CompressionRequest]) -> list[CompressionResult]:
-        """Compress many scheduler-authorised requests in one batched step."""
+        """Compress many scheduler-authorised requests in one batched step,
+        enqueued on the current stream: it reads the requests' device tables and
+        writes their pages in that stream's order."""
         if self.pipeline is None or self.offsets is None or not self.layer_caches:
             raise RuntimeError("TriAttention method is not bound to KV cache")
         if not requests:
@@ -232,11 +234,8 @@ class TriAttentionMethod(KVCompressionMethod):
             block_size=self.cache_block_size,
             budget=self.config.kv_budget,
         )
-        try:
-            self._select(batch)
-            self.pipeline.compact(batch)
-        finally:
-            batch.wait()  # the requests' block tables are the caller's again
+        self._select(batch)
+        self.pipeline.compact(batch)
         return [self._result() for _ in requests]
 
     def _select(self, batch: Batch) -> torch.Tensor:
@@ -249,10 +248,7 @@ class TriAttentionMethod(KVCompressionMethod):
         if self.pipeline is None:
             raise RuntimeError("TriAttention method is not bound to KV cache")
         batch = Batch.queue(self.pipeline.device, [int(physical_num_tokens)], [int(round_start)], [source_block_ids])
-        try:
-            return self._select(batch)[0].clone()
-        finally:
-            batch.wait()
+        return self._select(batch)[0].clone()
 
 
 def tensor_parallel_group() -> Any:

@@ -102,7 +102,7 @@ class Batch:
     ``build`` returns when they are written and the block tables it was given
     are read, so the batch may be used, and the tables changed, on any stream.
     ``queue`` only puts the copies on the current stream: for callers that use
-    the batch on that stream and call ``wait`` before they hand back the tables."""
+    the batch on that stream, whose own results are complete there."""
 
     n_seq: int
     seq_lens_host: list[int]
@@ -116,7 +116,6 @@ class Batch:
     dst_offsets: torch.Tensor | None
     dst_ids: torch.Tensor | None
     rewrite_buffers: dict = field(default_factory=dict)
-    written: torch.cuda.Event | None = field(default=None, repr=False, compare=False)
 
     @property
     def total_tokens(self) -> int:
@@ -141,13 +140,9 @@ class Batch:
         batch = cls.queue(
             device, seq_lens, round_starts, source_tables, destination_tables, block_size=block_size, budget=budget
         )
-        batch.wait()
+        if batch.seq_lens.is_cuda:
+            torch.cuda.current_stream(device).synchronize()
         return batch
-
-    def wait(self) -> None:
-        """Until the device has run the copies that ``queue`` put on its stream."""
-        if self.written is not None:
-            self.written.synchronize()
 
     @classmethod
     def queue(
@@ -164,7 +159,8 @@ class Batch:
         n = len(seq_lens)
         if n == 0 or len(round_starts) != n or len(source_tables) != n:
             raise ValueError("a batch needs matching lengths, round starts and source tables")
-        src_ids, src_lens = dev.ragged_ids(list(source_tables), device)
+        reader = torch.cuda.current_stream(device) if device.type == "cuda" else None
+        src_ids, src_lens = dev.ragged_ids(list(source_tables), device, reader)
         for length, blocks in zip(seq_lens, src_lens):
             if length < 0 or blocks * block_size < length:
                 raise ValueError("source block table does not cover the sequence")
@@ -173,17 +169,13 @@ class Batch:
         if destination_tables is not None:
             if len(destination_tables) != n:
                 raise ValueError("one destination table per sequence")
-            dst_ids, dst_lens = dev.ragged_ids(list(destination_tables), device)
+            dst_ids, dst_lens = dev.ragged_ids(list(destination_tables), device, reader)
             columns.append(dev.prefix_offsets(dst_lens))
             if budget is not None:
                 need = (budget + block_size - 1) // block_size
                 if any(d < need for d in dst_lens):
                     raise ValueError("destination table too short for the budget")
         (token_offsets, round_starts_dev, src_off, *rest), seq_lens_dev = dev.pack_words(columns, seq_lens, device)
-        written = None
-        if seq_lens_dev.is_cuda:
-            written = torch.cuda.Event()
-            written.record(torch.cuda.current_stream(device))
         return cls(
             n_seq=n,
             seq_lens_host=[int(x) for x in seq_lens],
@@ -196,7 +188,6 @@ class Batch:
             src_ids=src_ids,
             dst_offsets=rest[0] if rest else None,
             dst_ids=dst_ids,
-            written=written,
         )
 
 
