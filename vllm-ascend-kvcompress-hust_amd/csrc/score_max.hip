@@ -254,9 +254,11 @@ struct MaxGeometry {
 // the next head's as their products issue, so that two tiles fit three waves
 // per SIMD.  Scoring and aggregating 8 x 16384 tokens x 6 layers, 16 offsets, 5
 // query heads: 495 us with one tile and the heads under run-time branches, 488
-// with the heads' number known, 482 with two tiles (half the LDS reads; about
-// 420 of it is this kernel: the matrix cores take 118 us, the vector ALUs about
-// as much, the LDS reads 100, the mixed reads and writes of HBM 330).
+// with the heads' number known, 482 with two tiles (half the LDS reads).  Of
+// those this kernel's launches trace at 493 (median of 20, the least 422); by
+// themselves the matrix cores would take 118 us, the vector ALUs about as much,
+// the LDS reads 100 and the mixed reads and writes of HBM 330: they overlap
+// only in part.
 template <int NK, bool LEAN>
 struct MaxTiling {
   static constexpr int T = NK >= 8 ? 1 : 2;
