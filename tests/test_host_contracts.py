@@ -669,3 +669,14 @@ def test_block_tables_are_recorded_on_the_stream_that_reads_them(monkeypatch):
     dev.ragged_ids(rows, torch.device("cpu"), SimpleNamespace(device_index=0))
     dev.ragged_ids([[1, 2], (3,)], torch.device("cpu"))
     assert seen == []
+
+
+@pytest.mark.parametrize("device", ["cpu", torch.device("cpu")])
+def test_batch_takes_a_device_or_its_name(device) -> None:
+    from kvcompress_mi355x.methods.triattention.pipeline import Batch
+
+    batch = Batch.build(device, [300, 5], [300, 1 << 40], [[4, 2, 9], torch.tensor([1])], [[7, 8], [6]], budget=100)
+    assert batch.seq_lens.tolist() == [300, 5] and batch.seq_lens.dtype == torch.int32
+    assert batch.token_offsets.tolist() == [0, 300, 305] and batch.round_starts.tolist() == [300, 1 << 40]
+    assert batch.src_offsets.tolist() == [0, 3, 4] and batch.src_ids.tolist() == [4, 2, 9, 1]
+    assert batch.dst_offsets.tolist() == [0, 2, 3] and batch.dst_ids.tolist() == [7, 8, 6]

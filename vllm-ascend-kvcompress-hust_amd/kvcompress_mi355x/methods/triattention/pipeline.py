@@ -156,6 +156,7 @@ class Batch:
         block_size: int = 128,
         budget: int | None = None,
     ) -> Batch:
+        device = torch.device(device)  # a name is taken too
         n = len(seq_lens)
         if n == 0 or len(round_starts) != n or len(source_tables) != n:
             raise ValueError("a batch needs matching lengths, round starts and source tables")
