@@ -19,10 +19,11 @@ POLICY_CODES = {"global": _native.POLICY_GLOBAL, "v3": _native.POLICY_V3}
 # kvc_select_keep runs one workgroup per (sequence, segment), 11 us for 16K
 # scores and about 0.35 us per further 1K of the longest segment;
 # kvc_select_keep_split (three launches, chunks spread over the chip) takes
-# 18-23 us for a few segments of up to 256K scores and up to 37 for 32 of them:
-# 1 x 49152 scores 18.5 us against 25.4, 4 x 131072 19.7 against 54, 16 x 32768
-# 19.8 against 20.0, 1 x 16384 17 against 11.  At 32K the two are level; the
-# line is above it, where the chunks win with 32 jobs too (65536: 27 against 32).
+# 18-23 us for a few segments of up to 256K scores and up to 36 for 32 of them:
+# 1 x 49152 scores 18.3 us against 26.7, 4 x 131072 19.6 against 56, 16 x 32768
+# 19.8 against 21.1, 1 x 16384 17 against 11.  At 32K the two are level (32 jobs:
+# 22.8 against 21.3); the line is above it, where the chunks win with 32 jobs too
+# (65536: 27 against 34).
 SPLIT_MIN_SEGMENT = 49152
 SPLIT_MAX_JOBS = 32
 
